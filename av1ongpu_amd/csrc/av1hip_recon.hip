@@ -1300,6 +1300,286 @@ __device__ __forceinline__ EarlyRes early_residual(RArgs a, BlkRef b) {
   return e;
 }
 
+/* ---- small intra blocks ------------------------------------------------
+ * The blocks the queue's critical path is made of (4x4 .. 8x8, 4x16, 16x4:
+ * at most 64 samples and 41 edge entries, three quarters and more of a
+ * frame's queued blocks), one sample and one edge entry per lane, without
+ * LDS. What bounds them is the latency of one wave from its neighbours'
+ * words to its own, so everything that does not depend on the edges'
+ * values - which word each lane polls, which entries and weights its sample
+ * is made of, where it is stored - is computed into registers before the
+ * wait; after it a sample takes one or two rounds of ds_bpermute between
+ * the entries' lanes and a few multiply-adds, and the packed words are
+ * formed by a DPP from the neighbouring lane. Against the LDS passes of
+ * predict_intra for every size: queue of a 1080p key frame 2097 -> 1034 us
+ * (768 levels), of a 426x240 one 497 -> 225 us, of a 1080p inter frame
+ * 119 -> 66 us. Larger blocks keep those passes: they hold several samples
+ * per lane, and one of them stands for several levels of small ones. */
+constexpr int kSmallSamples = 64, kSmallEdge = 20; /* w * h, w + h */
+
+__device__ __forceinline__ bool small_block(const QBlk& q, BlkRef b, const EarlyRes& er) {
+  return q.kind == kIntra && (q.flags & (kPackedEdges | kFilterIntra | kPalette)) == kPackedEdges &&
+         q.mode <= AV1H_PRED_PAETH && q.w * q.h <= kSmallSamples && q.w + q.h <= kSmallEdge &&
+         (er.on || b.tx_count == 0);
+}
+
+/* the value of lane `at` / 4 */
+__device__ __forceinline__ int from_lane(int at, int v) { return __builtin_amdgcn_ds_bpermute(at, v); }
+template <int kCtrl, int kRows = 0xf>
+__device__ __forceinline__ int dpp(int v) {
+  return __builtin_amdgcn_update_dpp(0, v, kCtrl, kRows, 0xf, false);
+}
+/* the sum over the wave, in every lane's scalar: four row steps, two
+ * broadcasts between the rows */
+__device__ __forceinline__ int wave_total(int v) {
+  v += dpp<0x111>(v);
+  v += dpp<0x112>(v);
+  v += dpp<0x114>(v);
+  v += dpp<0x118>(v);
+  v += dpp<0x142, 0xa>(v);
+  v += dpp<0x143, 0xc>(v);
+  return __builtin_amdgcn_readlane(v, 63);
+}
+
+#define AV1H_KEEP(...) asm volatile("" : __VA_ARGS__)
+
+__device__ __forceinline__ void queue_small(RArgs a, BlkRef b, const QBlk& q, const EarlyRes& er, const int* tab,
+                                            uint32_t* error, uint64_t* ready, bool trace) {
+  LayRef L = a.lay;
+  const int lane = threadIdx.x;
+  const int w = q.w, h = q.h, n = w + h, lw = ilog2(w), lh = ilog2(h);
+  const int x = lane & (w - 1), y = lane >> lw; /* this lane's sample */
+  const bool sample = lane < w * h;
+  const int sh = L.cell_shift[q.plane], mid = 1 << (q.bd - 1), maxv = q.maxv;
+  const bool ha = (q.flags & kHaveAbove) != 0, hl = (q.flags & kHaveLeft) != 0;
+  /* this lane's edge entry: lane n the corner, n + 1 + k above[k], n - 1 - k
+   * left[k]; where it comes from as gather_packed has it */
+  const int d = lane - n;
+  const bool entry = lane <= 2 * n;
+  const bool use_a = d >= 0 ? ha : (!hl && ha);
+  const bool use_l = d <= 0 ? (hl && !(d == 0 && ha)) : (!ha && hl);
+  int val = mid + (d > 0 ? -1 : (d < 0 ? 1 : 0)), half = 0;
+  bool pend = false;
+  AV1H_GLOBAL uint64_t* word = (AV1H_GLOBAL uint64_t*)a.edges;
+  {
+    const int alast = min(q.max_x, q.x + ((q.flags & kHaveAR) ? 2 * w : w) - 1);
+    const int llast = min(q.max_y, q.y + ((q.flags & kHaveBL) ? 2 * h : h) - 1);
+    const int ae = min(b.dep_x1, alast) - q.x, le = min(b.dep_y1, llast) - q.y;
+    AV1H_GLOBAL uint64_t* rowp = word + L.edge_row_off[q.plane] + (int64_t)((q.y >> sh) - 1) * L.edge_row_words[q.plane];
+    AV1H_GLOBAL uint64_t* colp = word + L.edge_col_off[q.plane] + (int64_t)((q.x >> sh) - 1) * L.edge_col_words[q.plane];
+    const uint32_t ma = (uint32_t)b.edge_mask_a, ml = (uint32_t)b.edge_mask_l;
+    const AV1H_GLOBAL uint16_t* from = q.dst;
+    bool load = false;
+    if (entry) {
+      if (d == 0 && ha && hl) {
+        if (q.flags & kCornerFrame) {
+          load = true;
+          from = q.dst - q.stride - 1;
+        } else {
+          pend = true;
+          half = 16;
+          word = (q.flags & kCornerRow) ? rowp + (q.x >> 1) - 1 : colp + (q.y >> 1) - 1;
+        }
+      } else if (use_a) {
+        const int i = d > 0 ? min(d - 1, ae) : 0;
+        if ((ma >> (i >> sh)) & 1) {
+          pend = true;
+          half = 16 * (i & 1);
+          word = rowp + ((q.x + i) >> 1);
+        } else {
+          load = true;
+          from = q.dst + i - q.stride;
+        }
+      } else if (use_l) {
+        const int i = d < 0 ? min(-d - 1, le) : 0;
+        if ((ml >> (i >> sh)) & 1) {
+          pend = true;
+          half = 16 * (i & 1);
+          word = colp + ((q.y + i) >> 1);
+        } else {
+          load = true;
+          from = q.dst + (int64_t)i * q.stride - 1;
+        }
+      }
+    }
+    if (load) val = *from; /* blocks outside the queue: final before it */
+  }
+  /* what the sample is made of */
+  const int mode = q.mode;
+  const bool dir = mode >= 1 && mode <= 8, smooth = mode >= AV1H_PRED_SMOOTH && mode <= AV1H_PRED_SMOOTH_H;
+  const bool filt = dir && (((q.dir_a >> kDirStrA) | (q.dir_a >> kDirStrL)) & 7) != 0;
+  const bool ups = dir && (q.dir_a & (kDirUpA | kDirUpL)) != 0;
+  int i0 = 0, i1 = 0, i2 = 0, i3 = 0;  /* entries (lane * 4)             */
+  int c0 = 0, c1 = 0, c2 = 0, c3 = 0;  /* weights                        */
+  int j0 = 0, j1 = 0, j2 = 0, j3 = 0;  /* edge filter: tap entries       */
+  int k0 = 16, k1 = 0, k2 = 0;         /* its kernel: centre, +-1, +-2   */
+  if (dir) {
+    const int pa = q.dir_a & 511, dx = q.dir_b & 0xffff, dy = (int)((uint32_t)q.dir_b >> 16);
+    const int ua = (q.dir_a & kDirUpA) ? 1 : 0, ul = (q.dir_a & kDirUpL) ? 1 : 0;
+    int left = 0, base, fr, up = 0;
+    if (pa < 90) {
+      const int idx = (y + 1) * dx;
+      base = (idx >> (6 - ua)) + (x << ua);
+      fr = ((idx << ua) >> 1) & 31;
+      up = ua;
+      if (base >= (n - 1) << ua) {
+        base = n - 1;
+        fr = up = 0;
+      }
+    } else if (pa > 90 && pa < 180) {
+      int idx = (x << 6) - (y + 1) * dx;
+      base = idx >> (6 - ua);
+      up = ua;
+      if (base < -(1 << ua)) {
+        left = 1;
+        idx = (y << 6) - (x + 1) * dy;
+        base = idx >> (6 - ul);
+        up = ul;
+      }
+      fr = ((idx * (1 << up)) >> 1) & 31;
+    } else if (pa > 180) {
+      const int idx = (x + 1) * dy;
+      left = 1;
+      base = (idx >> (6 - ul)) + (y << ul);
+      fr = ((idx << ul) >> 1) & 31;
+      up = ul;
+    } else {
+      left = pa == 180;
+      base = left ? y : x;
+      fr = 0;
+    }
+    /* entry k of the side as a lane address */
+    auto at = [&](int k) { return 4 * (left ? n - 1 - k : n + 1 + k); };
+    /* an upsampled entry 2i - 1 interpolates entries i - 2 .. i + 1 of the
+     * edge, 2i is its entry i; of the pair base, base + 1 the odd one is
+     * interpolated */
+    const int odd = base & 1, m = (left ? h + (pa > 180 ? w : 0) : w + (pa < 90 ? h : 0)) - 1;
+    if (up) {
+      const int t = ((base + odd) >> 1) - 1 - odd;
+      i0 = at(clampi(t, -1, m));
+      i1 = at(clampi(t + 1, -1, m));
+      i2 = at(clampi(t + 2, -1, m));
+      i3 = at(clampi(t + 3, -1, m));
+    } else {
+      i1 = at(clampi(base, -1, n - 1));
+      i2 = at(clampi(base + 1, -1, n - 1));
+    }
+    c0 = 32 - fr;
+    c1 = fr;
+    c2 = up && odd;
+    c3 = up && !odd;
+    if (filt) {
+      const int stra = (q.dir_a >> kDirStrA) & 7, strl = (q.dir_a >> kDirStrL) & 7;
+      const bool el = d < 0;
+      const int str = el ? strl : stra, k = el ? -d - 1 : d - 1;
+      const int last = (el ? min(h, q.max_y - q.y + 1) + (pa > 180 ? w : 0) : min(w, q.max_x - q.x + 1) + (pa < 90 ? h : 0)) - 1;
+      auto te = [&](int i) { return 4 * (el ? n - 1 - clampi(i, -1, last) : n + 1 + clampi(i, -1, last)); };
+      if (str && k >= 0 && k <= last) {
+        const int* kk = TAB(AV1T_OFF_EDGE_KERNEL) + 5 * (str - 1);
+        k0 = kk[2];
+        k1 = kk[1];
+        k2 = kk[0];
+        j0 = te(k - 2);
+        j1 = te(k - 1);
+        j2 = te(k + 1);
+        j3 = te(k + 2);
+      }
+    }
+  } else if (smooth) {
+    const int* sw = TAB(AV1T_OFF_SM_WEIGHTS);
+    const int wy = mode == AV1H_PRED_SMOOTH_H ? 0 : sw[h - 4 + y], wx = mode == AV1H_PRED_SMOOTH_V ? 0 : sw[w - 4 + x];
+    i1 = 4 * (n + 1 + x);
+    i2 = 4 * (n - 1 - y);
+    c0 = wy;
+    c1 = mode == AV1H_PRED_SMOOTH_H ? 0 : 256 - wy;
+    c2 = wx;
+    c3 = mode == AV1H_PRED_SMOOTH_V ? 0 : 256 - wx;
+  } else if (mode == AV1H_PRED_PAETH) {
+    i1 = 4 * (n + 1 + x);
+    i2 = 4 * (n - 1 - y);
+  } else {
+    /* DC: the entries it sums */
+    c0 = ((ha && d > 0 && d <= w) || (hl && d < 0 && -d <= h)) ? 1 : 0;
+  }
+  /* DC: (sum + cnt / 2) / cnt as a high product with ceil(2^32 / cnt): exact
+   * for sums below 2^32 / cnt^2 (cnt 4 .. 20, at most 20 samples of 12 bits) */
+  const int cnt = (ha ? w : 0) + (hl ? h : 0);
+  const uint32_t recip = cnt == 12 ? 0x15555556u : cnt == 20 ? 0x0ccccccdu : cnt ? 1u << (32 - ilog2(cnt)) : 0;
+  /* where the sample and the packed words go: the last row's words by its
+   * even columns, the last column's by the even rows, never the same lane */
+  const int res = er.on ? (int)er.v[0] : 0;
+  AV1H_GLOBAL uint16_t* dst = q.dst + (int64_t)y * q.stride + x;
+  const bool row = sample && (q.flags & kEdgeRow) && y == h - 1 && !(x & 1);
+  const bool col = sample && (q.flags & kEdgeCol) && x == w - 1 && !(y & 1);
+  AV1H_GLOBAL uint64_t* pub = row ? q.row_pub + (x >> 1) : q.col_pub + (y >> 1);
+  AV1H_KEEP("+v"(val), "+v"(half), "+v"(word), "+v"(dst), "+v"(pub), "+v"(i0), "+v"(i1), "+v"(i2), "+v"(i3), "+v"(c0),
+            "+v"(c1), "+v"(c2), "+v"(c3), "+v"(j0), "+v"(j1), "+v"(j2), "+v"(j3), "+v"(k0), "+v"(k1), "+v"(k2));
+  /* the wait: every lane polls its entry's word until it carries this
+   * frame's epoch (poll_word) */
+  for (int iter = 0;; ++iter) {
+    if (pend) {
+      const uint64_t v = __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if ((uint32_t)(v >> 32) == q.epoch) {
+        val = (int)(((uint32_t)v >> half) & 0xffffu);
+        pend = false;
+      }
+    }
+    if (!__any(pend)) break;
+    if (iter >= a.spin_limit) {
+      if (lane == 0) atomicOr(error, 1u);
+      break;
+    }
+    __builtin_amdgcn_s_sleep(1);
+  }
+  if (trace) *ready = (uint64_t)wall_clock64();
+  int v;
+  if (dir) {
+    int e = val;
+    if (filt)
+      e = (k0 * val + k1 * (from_lane(j1, val) + from_lane(j2, val)) + k2 * (from_lane(j0, val) + from_lane(j3, val)) + 8) >> 4;
+    int t1 = from_lane(i1, e), t2 = from_lane(i2, e);
+    if (ups) {
+      const int t0 = from_lane(i0, e), t3 = from_lane(i3, e);
+      const int mv = clampi((9 * (t1 + t2) - t0 - t3 + 8) >> 4, 0, maxv);
+      if (c2) t1 = mv;
+      if (c3) t2 = mv;
+    }
+    v = (t1 * c0 + t2 * c1 + 16) >> 5;
+  } else if (smooth) {
+    const int bl = __builtin_amdgcn_readlane(val, w), ar = __builtin_amdgcn_readlane(val, n + w);
+    v = c0 * from_lane(i1, val) + c1 * bl + c2 * from_lane(i2, val) + c3 * ar;
+    v = mode == AV1H_PRED_SMOOTH ? (v + 256) >> 9 : (v + 128) >> 8;
+  } else if (mode == AV1H_PRED_PAETH) {
+    const int tl = __builtin_amdgcn_readlane(val, n), t = from_lane(i1, val), l = from_lane(i2, val);
+    const int pl = abs(t - tl), pt = abs(l - tl), ptl = abs(t + l - 2 * tl);
+    v = (pl <= pt && pl <= ptl) ? l : (pt <= ptl ? t : tl);
+  } else {
+    const int sum = wave_total(c0 ? val : 0);
+    v = cnt ? (int)__umulhi((uint32_t)(sum + (cnt >> 1)), recip) : mid;
+  }
+  v = clampi(clampi(v, 0, maxv) + res, 0, maxv);
+  /* packed words: this sample and the next one of its row / column */
+  const int right = dpp<0xb1>(v); /* lane ^ 1 */
+  if (q.flags & (kEdgeRow | kEdgeCol)) {
+    int next = right;
+    if (q.flags & kEdgeCol) {
+      const int below = w == 4 ? dpp<0x104>(v) : (w == 8 ? dpp<0x108>(v) : from_lane(4 * (lane + w), v));
+      if (col) next = below;
+    }
+    if (row || col)
+      __hip_atomic_store(pub, ((uint64_t)q.epoch << 32) | ((uint32_t)next << 16) | (uint32_t)v, __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+  }
+  if (sample && !(x & 1)) {
+    const uint32_t two = ((uint32_t)right << 16) | (uint32_t)v;
+    AV1H_GLOBAL uint32_t* to = (AV1H_GLOBAL uint32_t*)dst;
+    if (q.flags & kSkipMark)
+      *to = two;
+    else
+      __hip_atomic_store(to, two, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+}
+
 __device__ void reconstruct_queued(RArgs a, BlkRef b, const QBlk& q, int* work, uint16_t* pred, const EarlyRes& er,
                                    const int* tab, uint32_t* error) {
   bool fused = false;
@@ -1564,18 +1844,23 @@ __global__ __launch_bounds__(64) void k_queue(BatchDev B) {
   __shared__ int s_work[kWork];
   __shared__ uint16_t s_pred[64 * 64];
   __shared__ int s_tab[kTabHi - kTabLo];
+  const int nqueue = kernel_prefix(B, kKernels)[0];
+  /* more workgroups than entries: the rest leave without the device-scope
+   * atomic each would make on the one counter (with the small blocks' path,
+   * a 160x96 inter frame's queue of 27 blocks 28.8 -> 8.9 us) */
+  const int takers = min((int)gridDim.x, nqueue);
+  if ((int)blockIdx.x >= takers) return;
   for (int i = threadIdx.x; i < kTabHi - kTabLo; i += 64) s_tab[i] = av1t_spec_table[kTabLo + i];
   __syncthreads();
-  const int nqueue = kernel_prefix(B, kKernels)[0];
   for (;;) {
     int idx = 0;
     if (threadIdx.x == 0) idx = (int)atomicAdd(B.queue_counter, 1u);
     idx = __builtin_amdgcn_readfirstlane(__shfl(idx, 0));
     if (idx >= nqueue) {
-      /* every workgroup takes exactly one entry past the end; the last of
+      /* every taking workgroup takes exactly one entry past the end; the last of
        * those is the counter's last use in this launch, so it resets the
        * counter for the next one */
-      if (threadIdx.x == 0 && idx == nqueue + (int)gridDim.x - 1)
+      if (threadIdx.x == 0 && idx == nqueue + takers - 1)
         __hip_atomic_store(B.queue_counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       return;
     }
@@ -1592,15 +1877,20 @@ __global__ __launch_bounds__(64) void k_queue(BatchDev B) {
     BlkRef b = cmem(a.plan.blocks)[__builtin_amdgcn_readfirstlane(blk)];
     const EarlyRes er = early_residual(a, b);
     const QBlk q = queued_block(a, b);
-    if (b.flags & kPackedEdges)
-      gather_edges(a, b, s_work, B.error);
-    else
-      wait_cells(a, b, B.error);
-    const uint64_t t1 = B.trace ? (uint64_t)wall_clock64() : 0;
-    reconstruct_queued(a, b, q, s_work, s_pred, er, s_tab, B.error);
-    /* the packed edges first: the blocks waiting on this one read only them */
-    if (q.flags & (kEdgeRow | kEdgeCol)) write_edges(q, s_pred);
-    store_block(q, s_pred);
+    uint64_t t1 = 0;
+    if (small_block(q, b, er)) {
+      queue_small(a, b, q, er, s_tab, B.error, &t1, B.trace != nullptr);
+    } else {
+      if (b.flags & kPackedEdges)
+        gather_edges(a, b, s_work, B.error);
+      else
+        wait_cells(a, b, B.error);
+      t1 = B.trace ? (uint64_t)wall_clock64() : 0;
+      reconstruct_queued(a, b, q, s_work, s_pred, er, s_tab, B.error);
+      /* the packed edges first: the blocks waiting on this one read only them */
+      if (q.flags & (kEdgeRow | kEdgeCol)) write_edges(q, s_pred);
+      store_block(q, s_pred);
+    }
     if (!(q.flags & kSkipMark)) {
       /* every sample store of the block has completed before its cells flip */
       __builtin_amdgcn_s_waitcnt(0);
