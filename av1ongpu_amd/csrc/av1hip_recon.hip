@@ -1283,13 +1283,17 @@ __device__ void wait_cells(RArgs a, BlkRef b, uint32_t* error) {
  * add), into `pred`; the caller stores it. */
 
 
-__device__ __forceinline__ EarlyRes early_residual(RArgs a, BlkRef b) {
-  EarlyRes e;
-  e.on = false;
-  if (b.tx_count != 1 || b.w * b.h > 256) return e;
+/* one transform covers the block */
+__device__ __forceinline__ bool one_transform(RArgs a, BlkRef b) {
+  if (b.tx_count != 1) return false;
   const AV1H_CMEM DevTx& tx = cmem(a.plan.tx)[b.tx_first];
-  if (tx.x != b.x || tx.y != b.y || tx.w != b.w || tx.h != b.h) return e;
-  e.on = true;
+  return tx.x == b.x && tx.y == b.y && tx.w == b.w && tx.h == b.h;
+}
+
+__device__ __forceinline__ EarlyRes early_residual(RArgs a, BlkRef b, bool one) {
+  EarlyRes e;
+  e.on = one && b.w * b.h <= 256;
+  if (!e.on) return e;
   const int p = b.plane, stride = a.lay.stride[p], lw = ilog2(b.w);
   const int16_t* r = a.res + a.lay.plane_off[p] + (int64_t)b.y * stride + b.x;
 #pragma unroll
@@ -1317,10 +1321,10 @@ __device__ __forceinline__ EarlyRes early_residual(RArgs a, BlkRef b) {
  * per lane, and one of them stands for several levels of small ones. */
 constexpr int kSmallSamples = 64, kSmallEdge = 20; /* w * h, w + h */
 
-__device__ __forceinline__ bool small_block(const QBlk& q, BlkRef b, const EarlyRes& er) {
+__device__ __forceinline__ bool small_block(const QBlk& q, BlkRef b, bool one) {
   return q.kind == kIntra && (q.flags & (kPackedEdges | kFilterIntra | kPalette)) == kPackedEdges &&
          q.mode <= AV1H_PRED_PAETH && q.w * q.h <= kSmallSamples && q.w + q.h <= kSmallEdge &&
-         (er.on || b.tx_count == 0);
+         (one || b.tx_count == 0);
 }
 
 /* the value of lane `at` / 4 */
@@ -1343,13 +1347,16 @@ __device__ __forceinline__ int wave_total(int v) {
 
 #define AV1H_KEEP(...) asm volatile("" : __VA_ARGS__)
 
-__device__ __forceinline__ void queue_small(RArgs a, BlkRef b, const QBlk& q, const EarlyRes& er, const int* tab,
+__device__ __forceinline__ void queue_small(RArgs a, BlkRef b, const QBlk& q, bool has_res, const int* tab,
                                             uint32_t* error, uint64_t* ready, bool trace) {
   LayRef L = a.lay;
   const int lane = threadIdx.x;
   const int w = q.w, h = q.h, n = w + h, lw = ilog2(w), lh = ilog2(h);
   const int x = lane & (w - 1), y = lane >> lw; /* this lane's sample */
   const bool sample = lane < w * h;
+  int res = 0;
+  if (has_res && sample)
+    res = ((const AV1H_GLOBAL int16_t*)a.res)[(q.dst - (AV1H_GLOBAL uint16_t*)a.frame) + (int64_t)y * q.stride + x];
   const int sh = L.cell_shift[q.plane], mid = 1 << (q.bd - 1), maxv = q.maxv;
   const bool ha = (q.flags & kHaveAbove) != 0, hl = (q.flags & kHaveLeft) != 0;
   /* this lane's edge entry: lane n the corner, n + 1 + k above[k], n - 1 - k
@@ -1507,12 +1514,11 @@ __device__ __forceinline__ void queue_small(RArgs a, BlkRef b, const QBlk& q, co
   const uint32_t recip = cnt == 12 ? 0x15555556u : cnt == 20 ? 0x0ccccccdu : cnt ? 1u << (32 - ilog2(cnt)) : 0;
   /* where the sample and the packed words go: the last row's words by its
    * even columns, the last column's by the even rows, never the same lane */
-  const int res = er.on ? (int)er.v[0] : 0;
   AV1H_GLOBAL uint16_t* dst = q.dst + (int64_t)y * q.stride + x;
   const bool row = sample && (q.flags & kEdgeRow) && y == h - 1 && !(x & 1);
   const bool col = sample && (q.flags & kEdgeCol) && x == w - 1 && !(y & 1);
   AV1H_GLOBAL uint64_t* pub = row ? q.row_pub + (x >> 1) : q.col_pub + (y >> 1);
-  AV1H_KEEP("+v"(val), "+v"(half), "+v"(word), "+v"(dst), "+v"(pub), "+v"(i0), "+v"(i1), "+v"(i2), "+v"(i3), "+v"(c0),
+  AV1H_KEEP("+v"(val), "+v"(res), "+v"(half), "+v"(word), "+v"(dst), "+v"(pub), "+v"(i0), "+v"(i1), "+v"(i2), "+v"(i3), "+v"(c0),
             "+v"(c1), "+v"(c2), "+v"(c3), "+v"(j0), "+v"(j1), "+v"(j2), "+v"(j3), "+v"(k0), "+v"(k1), "+v"(k2));
   /* the wait: every lane polls its entry's word until it carries this
    * frame's epoch (poll_word) */
@@ -1577,6 +1583,321 @@ __device__ __forceinline__ void queue_small(RArgs a, BlkRef b, const QBlk& q, co
       *to = two;
     else
       __hip_atomic_store(to, two, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+}
+
+/* ---- large intra blocks --------------------------------------------------
+ * The packed-edge blocks beyond 64 samples (8x16 .. 64x64) with one
+ * transform or none. A chain of them is bound by the time from a block's
+ * edges to its own last row and column, not by its samples: those are
+ * predicted first, one packed word per lane, and published before the rest
+ * of the block, whose pairs of samples then go straight from registers to
+ * the frame. The polled words (two entries each, at most three per lane) are
+ * all in flight together; edges and filtered edges lie in LDS. No size here
+ * upsamples its edges (that takes w + h <= 16). A 16x16 block's work after
+ * its wait, to the end of its stores, 3.2 -> 1.7 us, a 32x32 block's 12 ->
+ * 3.8 us; queue of a 1080p key frame 1034 -> 801 us, of a 426x240 one 225 ->
+ * 191 us, of a 2160p inter frame 164 -> 129 us. */
+__device__ __forceinline__ bool big_block(const QBlk& q, BlkRef b, bool one) {
+  return q.kind == kIntra && (q.flags & (kPackedEdges | kFilterIntra | kPalette)) == kPackedEdges &&
+         q.mode <= AV1H_PRED_PAETH && q.w * q.h > kSmallSamples && !(q.dir_a & (kDirUpA | kDirUpL)) &&
+         (one || b.tx_count == 0);
+}
+
+enum BigKind { kBigDc, kBigV, kBigH, kBigZ1, kBigZ2, kBigZ3, kBigSmooth, kBigSmoothV, kBigSmoothH, kBigPaeth };
+
+/* sample (x, y) of a block of kind K: ea / el the edges, m0 .. m2 what the
+ * kind needs of them or of the block (DC's value, the far corners) */
+template <int K>
+__device__ __forceinline__ int big_sample(int x, int y, int w, int h, int dx, int dy, const int* ea, const int* el,
+                                          const int* sw, int m0, int m1) {
+  if (K == kBigDc) return m0;
+  if (K == kBigV) return ea[x];
+  if (K == kBigH) return el[y];
+  if (K == kBigZ1) {
+    /* entries past the last repeat it, and a blend of equals is the value */
+    const int idx = (y + 1) * dx, base = (idx >> 6) + x, fr = (idx >> 1) & 31, last = w + h - 1;
+    return rnd2(ea[min(base, last)] * (32 - fr) + ea[min(base + 1, last)] * fr, 5);
+  }
+  if (K == kBigZ2) {
+    const int ia = (x << 6) - (y + 1) * dx, il = (y << 6) - (x + 1) * dy;
+    const bool up = (ia >> 6) >= -1;
+    const int idx = up ? ia : il, fr = (idx >> 1) & 31;
+    const int* e = (up ? ea : el) + (idx >> 6);
+    return rnd2(e[0] * (32 - fr) + e[1] * fr, 5);
+  }
+  if (K == kBigZ3) {
+    const int idx = (x + 1) * dy, fr = (idx >> 1) & 31;
+    const int* e = el + (idx >> 6) + y;
+    return rnd2(e[0] * (32 - fr) + e[1] * fr, 5);
+  }
+  if (K == kBigSmooth) {
+    const int wy = sw[h - 4 + y], wx = sw[w - 4 + x];
+    return rnd2(wy * ea[x] + (256 - wy) * m0 + wx * el[y] + (256 - wx) * m1, 9);
+  }
+  if (K == kBigSmoothV) {
+    const int wy = sw[h - 4 + y];
+    return rnd2(wy * ea[x] + (256 - wy) * m0, 8);
+  }
+  if (K == kBigSmoothH) {
+    const int wx = sw[w - 4 + x];
+    return rnd2(wx * el[y] + (256 - wx) * m1, 8);
+  }
+  const int t = ea[x], l = el[y]; /* Paeth: m0 the corner */
+  const int pl = abs(t - m0), pt = abs(l - m0), ptl = abs(t + l - 2 * m0);
+  return (pl <= pt && pl <= ptl) ? l : (pt <= ptl ? t : m0);
+}
+
+/* What a lane keeps of the block across the wait: its packed word's samples
+ * and their residuals, the first residual pairs of its share of the block. */
+struct BigLane {
+  AV1H_GLOBAL uint64_t* pub;
+  int x0, y0, x1, y1, r0, r1;
+  bool on;
+};
+constexpr int kBigStep = 4; /* pairs per lane and step */
+
+template <int K>
+__device__ __forceinline__ void big_emit(const QBlk& q, const BigLane& g, uint32_t (&r)[kBigStep], bool has_res,
+                                         const AV1H_GLOBAL uint32_t* res, int dx, int dy, const int* ea, const int* el,
+                                         const int* sw, int m0, int m1) {
+  const int w = q.w, h = q.h, maxv = q.maxv, lane = threadIdx.x, lw = ilog2(w);
+  auto at = [&](int x, int y, int rv) {
+    const int v = big_sample<K>(x, y, w, h, dx, dy, ea, el, sw, m0, m1);
+    return clampi(clampi(v, 0, maxv) + rv, 0, maxv);
+  };
+  if (g.on) {
+    const uint32_t two = (uint32_t)at(g.x0, g.y0, g.r0) | ((uint32_t)at(g.x1, g.y1, g.r1) << 16);
+    __hip_atomic_store(g.pub, ((uint64_t)q.epoch << 32) | two, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  /* every pair of the block, the next step's residuals loaded ahead */
+  const int pairs = (w * h) >> 1, half = q.stride >> 1;
+  AV1H_GLOBAL uint32_t* dst = (AV1H_GLOBAL uint32_t*)q.dst;
+  for (int p0 = 0; p0 < pairs; p0 += 64 * kBigStep) {
+    uint32_t rn[kBigStep];
+#pragma unroll
+    for (int k = 0; k < kBigStep; ++k) {
+      const int s = 2 * (p0 + 64 * (kBigStep + k) + lane);
+      rn[k] = has_res && s < 2 * pairs ? res[(int64_t)(s >> lw) * half + ((s & (w - 1)) >> 1)] : 0u;
+    }
+#pragma unroll
+    for (int k = 0; k < kBigStep; ++k) {
+      const int s = 2 * (p0 + 64 * k + lane);
+      if (s >= 2 * pairs) break;
+      const int x = s & (w - 1), y = s >> lw;
+      const uint32_t two = (uint32_t)at(x, y, (int)(int16_t)r[k]) | ((uint32_t)at(x + 1, y, (int)r[k] >> 16) << 16);
+      AV1H_GLOBAL uint32_t* to = dst + (int64_t)y * half + (x >> 1);
+      if (q.flags & kSkipMark)
+        *to = two;
+      else
+        __hip_atomic_store(to, two, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+#pragma unroll
+    for (int k = 0; k < kBigStep; ++k) r[k] = rn[k];
+  }
+}
+
+__device__ __forceinline__ void queue_big(RArgs a, BlkRef b, const QBlk& q, bool has_res, int* work, const int* tab,
+                                          uint32_t* error, uint64_t* ready, bool trace) {
+  LayRef L = a.lay;
+  const int lane = threadIdx.x;
+  const int w = q.w, h = q.h, n = w + h, lw = ilog2(w);
+  const int sh = L.cell_shift[q.plane], mid = 1 << (q.bd - 1), maxv = q.maxv;
+  const bool ha = (q.flags & kHaveAbove) != 0, hl = (q.flags & kHaveLeft) != 0;
+  int* above = work + kEdgeOff;
+  int* left = above + kEdge + 2 * kEdgeOff;
+  /* residuals: the lane's border samples, its first pairs of the block */
+  const AV1H_GLOBAL int16_t* res = (const AV1H_GLOBAL int16_t*)a.res + (q.dst - (AV1H_GLOBAL uint16_t*)a.frame);
+  const AV1H_GLOBAL uint32_t* res2 = (const AV1H_GLOBAL uint32_t*)res;
+  const int half = q.stride >> 1;
+  BigLane g;
+  {
+    const bool row = lane < (w >> 1);
+    const int j = row ? lane : lane - (w >> 1);
+    g.x0 = row ? 2 * j : w - 1;
+    g.x1 = row ? 2 * j + 1 : w - 1;
+    g.y0 = row ? h - 1 : 2 * j;
+    g.y1 = row ? h - 1 : 2 * j + 1;
+    g.pub = row ? q.row_pub + j : q.col_pub + j;
+    g.on = row ? (q.flags & kEdgeRow) != 0 : (q.flags & kEdgeCol) != 0 && j < (h >> 1);
+    g.r0 = has_res && g.on ? res[(int64_t)g.y0 * q.stride + g.x0] : 0;
+    g.r1 = has_res && g.on ? res[(int64_t)g.y1 * q.stride + g.x1] : 0;
+  }
+  uint32_t r[kBigStep];
+#pragma unroll
+  for (int k = 0; k < kBigStep; ++k) {
+    const int s = 2 * (64 * k + lane);
+    r[k] = has_res && s < w * h ? res2[(int64_t)(s >> lw) * half + ((s & (w - 1)) >> 1)] : 0u;
+  }
+  /* the words of the edges, two entries each: above 0 .. n - 1, left
+   * 0 .. n - 1, the corner; sources as gather_packed has them */
+  constexpr int kSlots = 3;
+  const int words = n + 1;
+  AV1H_GLOBAL uint64_t* word[kSlots];
+  int v0[kSlots], v1[kSlots], s0[kSlots], s1[kSlots];
+  bool pend[kSlots];
+  {
+    const int alast = min(q.max_x, q.x + ((q.flags & kHaveAR) ? 2 * w : w) - 1);
+    const int llast = min(q.max_y, q.y + ((q.flags & kHaveBL) ? 2 * h : h) - 1);
+    const int ae = min(b.dep_x1, alast) - q.x, le = min(b.dep_y1, llast) - q.y;
+    AV1H_GLOBAL uint64_t* base = (AV1H_GLOBAL uint64_t*)a.edges;
+    AV1H_GLOBAL uint64_t* rowp = base + L.edge_row_off[q.plane] + (int64_t)((q.y >> sh) - 1) * L.edge_row_words[q.plane];
+    AV1H_GLOBAL uint64_t* colp = base + L.edge_col_off[q.plane] + (int64_t)((q.x >> sh) - 1) * L.edge_col_words[q.plane];
+    const uint32_t ma = (uint32_t)b.edge_mask_a, ml = (uint32_t)b.edge_mask_l;
+#pragma unroll
+    for (int u = 0; u < kSlots; ++u) {
+      const int e = lane + 64 * u, nw = n >> 1;
+      const int d = e < nw ? 1 : (e < 2 * nw ? -1 : 0), j = d < 0 ? e - nw : e;
+      word[u] = base;
+      pend[u] = false;
+      s0[u] = s1[u] = 0;
+      v0[u] = v1[u] = mid + (d > 0 ? -1 : (d < 0 ? 1 : 0));
+      if (e >= words) continue;
+      const bool use_a = d >= 0 ? ha : (!hl && ha), use_l = d <= 0 ? (hl && !(d == 0 && ha)) : (!ha && hl);
+      if (d == 0 && ha && hl) {
+        if (q.flags & kCornerFrame) {
+          v0[u] = q.dst[-q.stride - 1];
+        } else {
+          pend[u] = true;
+          s0[u] = s1[u] = 16;
+          word[u] = (q.flags & kCornerRow) ? rowp + (q.x >> 1) - 1 : colp + (q.y >> 1) - 1;
+        }
+      } else if (use_a) {
+        const int i0 = d > 0 ? min(2 * j, ae) : 0, i1 = d > 0 ? min(2 * j + 1, ae) : 0;
+        if ((ma >> (i0 >> sh)) & 1) {
+          pend[u] = true;
+          s0[u] = 16 * (i0 & 1);
+          s1[u] = 16 * (i1 & 1);
+          word[u] = rowp + ((q.x + i0) >> 1);
+        } else {
+          v0[u] = q.dst[i0 - q.stride];
+          v1[u] = q.dst[i1 - q.stride];
+        }
+      } else if (use_l) {
+        const int i0 = d < 0 ? min(2 * j, le) : 0, i1 = d < 0 ? min(2 * j + 1, le) : 0;
+        if ((ml >> (i0 >> sh)) & 1) {
+          pend[u] = true;
+          s0[u] = 16 * (i0 & 1);
+          s1[u] = 16 * (i1 & 1);
+          word[u] = colp + ((q.y + i0) >> 1);
+        } else {
+          v0[u] = q.dst[(int64_t)i0 * q.stride - 1];
+          v1[u] = q.dst[(int64_t)i1 * q.stride - 1];
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < kSlots; ++u) AV1H_KEEP("+v"(word[u]), "+v"(v0[u]), "+v"(v1[u]), "+v"(s0[u]), "+v"(s1[u]));
+  AV1H_KEEP("+v"(g.pub), "+v"(g.r0), "+v"(g.r1), "+v"(g.x0), "+v"(g.x1), "+v"(g.y0), "+v"(g.y1));
+  for (int iter = 0;; ++iter) {
+    uint64_t v[kSlots];
+#pragma unroll
+    for (int u = 0; u < kSlots; ++u)
+      v[u] = pend[u] ? __hip_atomic_load(word[u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+    bool any = false;
+#pragma unroll
+    for (int u = 0; u < kSlots; ++u) {
+      if (pend[u] && (uint32_t)(v[u] >> 32) == q.epoch) {
+        v0[u] = (int)(((uint32_t)v[u] >> s0[u]) & 0xffffu);
+        v1[u] = (int)(((uint32_t)v[u] >> s1[u]) & 0xffffu);
+        pend[u] = false;
+      }
+      any = any || pend[u];
+    }
+    if (!__any(any)) break;
+    if (iter >= a.spin_limit) {
+      if (lane == 0) atomicOr(error, 1u);
+      break;
+    }
+    __builtin_amdgcn_s_sleep(1);
+  }
+  if (trace) *ready = (uint64_t)wall_clock64();
+#pragma unroll
+  for (int u = 0; u < kSlots; ++u) {
+    const int e = lane + 64 * u, nw = n >> 1;
+    if (e >= words) continue;
+    if (e < 2 * nw) {
+      int* to = e < nw ? above + 2 * e : left + 2 * (e - nw);
+      to[0] = v0[u];
+      to[1] = v1[u];
+    } else {
+      above[-1] = left[-1] = v0[u];
+    }
+  }
+  wsync();
+  const int mode = q.mode, pa = q.dir_a & 511, dx = q.dir_b & 0xffff, dy = (int)((uint32_t)q.dir_b >> 16);
+  const int* ea = above;
+  const int* el = left;
+  const int* sw = TAB(AV1T_OFF_SM_WEIGHTS);
+  if (mode >= 1 && mode <= 8) {
+    const int stra = (q.dir_a >> kDirStrA) & 7, strl = (q.dir_a >> kDirStrL) & 7;
+    if ((q.dir_a & kDirCorner) || stra || strl) {
+      /* the entries the zone reads (av1gpu_kernels.h:1157-1173): above of
+       * w + h, left of w + h, or the w + h around the corner */
+      int corner = above[-1];
+      if (q.dir_a & kDirCorner) corner = rnd2(left[0] * 5 + above[-1] * 6 + above[0] * 5, 4);
+      int* fa = work + kPrep1 + kEdgeOff;
+      int* fl = fa + kEdge + 2 * kEdgeOff;
+      const int na = pa < 90 ? n : (pa > 180 ? 0 : w);
+      for (int e = lane; e <= n; e += 64) {
+        const bool is_l = e > na;
+        const int k = is_l ? e - na - 1 : e - 1; /* -1: the corner */
+        const int* src = is_l ? left : above;
+        const int str = is_l ? strl : stra;
+        const int last = is_l ? min(h, q.max_y - q.y + 1) + (pa > 180 ? w : 0) - 1 : min(w, q.max_x - q.x + 1) + (pa < 90 ? h : 0) - 1;
+        int v = k < 0 ? corner : src[k];
+        if (str && k >= 0 && k <= last) {
+          const int* kk = TAB(AV1T_OFF_EDGE_KERNEL) + 5 * (str - 1);
+          int acc = 8;
+#pragma unroll
+          for (int t = 0; t < 5; ++t) {
+            const int m = clampi(k + t - 2, -1, last);
+            acc += kk[t] * (m < 0 ? corner : src[m]);
+          }
+          v = acc >> 4;
+        }
+        if (k < 0)
+          fa[-1] = fl[-1] = v;
+        else
+          (is_l ? fl : fa)[k] = v;
+      }
+      wsync();
+      ea = fa;
+      el = fl;
+    }
+    if (pa == 90)
+      big_emit<kBigV>(q, g, r, has_res, res2, dx, dy, ea, el, sw, 0, 0);
+    else if (pa == 180)
+      big_emit<kBigH>(q, g, r, has_res, res2, dx, dy, ea, el, sw, 0, 0);
+    else if (pa < 90)
+      big_emit<kBigZ1>(q, g, r, has_res, res2, dx, dy, ea, el, sw, 0, 0);
+    else if (pa < 180)
+      big_emit<kBigZ2>(q, g, r, has_res, res2, dx, dy, ea, el, sw, 0, 0);
+    else
+      big_emit<kBigZ3>(q, g, r, has_res, res2, dx, dy, ea, el, sw, 0, 0);
+  } else if (mode == AV1H_PRED_SMOOTH) {
+    big_emit<kBigSmooth>(q, g, r, has_res, res2, dx, dy, ea, el, sw, left[h - 1], above[w - 1]);
+  } else if (mode == AV1H_PRED_SMOOTH_V) {
+    big_emit<kBigSmoothV>(q, g, r, has_res, res2, dx, dy, ea, el, sw, left[h - 1], 0);
+  } else if (mode == AV1H_PRED_SMOOTH_H) {
+    big_emit<kBigSmoothH>(q, g, r, has_res, res2, dx, dy, ea, el, sw, 0, above[w - 1]);
+  } else if (mode == AV1H_PRED_PAETH) {
+    big_emit<kBigPaeth>(q, g, r, has_res, res2, dx, dy, ea, el, sw, above[-1], 0);
+  } else {
+    /* DC (av1gpu_kernels.h:1430-1447): w + h <= 128 samples, two per lane */
+    int s = 0;
+    if (ha && lane < w) s += above[lane];
+    if (hl && lane < h) s += left[lane];
+    s = wave_total(s);
+    int dc = mid;
+    if (ha && hl)
+      dc = (s + (n >> 1)) / n;
+    else if (hl)
+      dc = (s + (h >> 1)) >> ilog2(h);
+    else if (ha)
+      dc = (s + (w >> 1)) >> lw;
+    big_emit<kBigDc>(q, g, r, has_res, res2, dx, dy, ea, el, sw, clampi(dc, 0, maxv), 0);
   }
 }
 
@@ -1875,12 +2196,15 @@ __global__ __launch_bounds__(64) void k_queue(BatchDev B) {
     }
     RArgs a = recon_args(B, __builtin_amdgcn_readfirstlane(job));
     BlkRef b = cmem(a.plan.blocks)[__builtin_amdgcn_readfirstlane(blk)];
-    const EarlyRes er = early_residual(a, b);
+    const bool one = one_transform(a, b);
     const QBlk q = queued_block(a, b);
     uint64_t t1 = 0;
-    if (small_block(q, b, er)) {
-      queue_small(a, b, q, er, s_tab, B.error, &t1, B.trace != nullptr);
+    if (small_block(q, b, one)) {
+      queue_small(a, b, q, one, s_tab, B.error, &t1, B.trace != nullptr);
+    } else if (big_block(q, b, one)) {
+      queue_big(a, b, q, one, s_work, s_tab, B.error, &t1, B.trace != nullptr);
     } else {
+      const EarlyRes er = early_residual(a, b, one);
       if (b.flags & kPackedEdges)
         gather_edges(a, b, s_work, B.error);
       else

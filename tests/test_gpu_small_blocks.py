@@ -19,6 +19,9 @@ pytestmark = pytest.mark.gpu
     ("c2_mini", dict(frames=1, max_tx=8, width=173, height=99, coded_width=0)),
     ("c2_mini", dict(frames=1, max_tx=16, width=66, height=58, coded_width=0, bit_depth=8)),
     ("c2_mini", dict(frames=1, bit_depth=12, width=120, height=200, coded_width=90)),
+    # large blocks: 32x32 to 64x64 and 2:1, one stripe of them and many; edges of both kinds
+    ("c2_mini", dict(frames=1, coef_zero=0.98, width=640, height=72, coded_width=0)),
+    ("c2_mini", dict(frames=3, width=392, height=328, coded_width=0, intra_frac=0.4, bit_depth=8)),
     # the smallest picture of one block column
     ("c1_mini", dict(frames=1, width=16, height=16, bit_depth=10)),
     # half the blocks intra among inter ones: edges mixed from words and frame
