@@ -178,7 +178,7 @@ struct Ctx {
   uint64_t* edges = nullptr; /* packed edge words, cleared with the cells */
   int64_t edges_cap = 0;
   uint32_t epoch = 0;
-  uint32_t* counters = nullptr; /* [0] queue counter, [1] error word */
+  uint32_t* counters = nullptr; /* [1] error word, from kTicketStep on the queue's ticket counters */
   int32_t* cdef_dir = nullptr;   /* CDEF direction map                */
   bool trace_on = false;         /* queue timestamps (diagnostics)    */
   int spin_limit = kSpinLimitDefault; /* polls of a dependency wait before a time-out */
@@ -2254,7 +2254,7 @@ int batch_launch(Ctx* lead, std::vector<JobSpec>& js, double t0) {
   B.prefix = reinterpret_cast<const int32_t*>(tab + o_prefix);
   B.njobs = n;
   B.queue = n > 1 ? reinterpret_cast<const uint32_t*>(tab + o_queue) : nullptr;
-  B.queue_counter = lead->counters;
+  B.queue_counter = lead->counters + kTicketStep;
   B.error = lead->counters + 1;
   B.trace = nullptr;
   grain_jump_matrices(B.jump82, B.jump44);
@@ -2634,7 +2634,7 @@ int av1h_create(int device_index, av1h_ctx** out) {
   default_tuning_impl(&c->tune);
   std::memset(&c->stats, 0, sizeof(c->stats));
   if (hipSetDevice(device_index) != hipSuccess || hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess ||
-      hipMalloc(&c->counters, 64) != hipSuccess || hipMemset(c->counters, 0, 64) != hipSuccess ||
+      hipMalloc(&c->counters, kCounterBytes) != hipSuccess || hipMemset(c->counters, 0, kCounterBytes) != hipSuccess ||
       hipMalloc(&c->hash_dev, kMaxBatch * 8) != hipSuccess ||
       hipMalloc(&c->grain_tmpl, 3 * 82 * 73 * 2) != hipSuccess) {
     delete h;

@@ -356,6 +356,11 @@ __device__ __forceinline__ int find_job(const AV1H_CMEM int32_t* pre, int n, int
  * frame hands out the frame's own queue list. */
 constexpr int kQueueJobShift = 24;
 constexpr int kMaxBatch = 128;
+/* The queue's ticket counters, kTicketStep words apart (own cache lines and
+ * memory channels); entry idx is ticket idx / counters of counter
+ * idx % counters (k_queue). */
+constexpr int kTickets = 8, kTicketStep = 512;
+constexpr size_t kCounterBytes = (size_t)(kTickets + 1) * kTicketStep * 4;
 
 /* CDEF: groups of 256 / (block samples) blocks a workgroup takes per step
  * (a thread's samples of up to kCdefMaxBatch blocks computed together) */

@@ -2173,18 +2173,33 @@ __global__ __launch_bounds__(64) void k_queue(BatchDev B) {
   if ((int)blockIdx.x >= takers) return;
   for (int i = threadIdx.x; i < kTabHi - kTabLo; i += 64) s_tab[i] = av1t_spec_table[kTabLo + i];
   __syncthreads();
+  /* Tickets: atomics on one address are served one after another (11.4 ns
+   * each: 17 us for the first tickets of 1536 waves, with their descriptor
+   * loads stuck behind them), so a large queue is dealt to kTickets counters,
+   * entry idx to counter idx % kTickets. Every entry still gets a wave: an
+   * XCD's workgroups start in order of their number, the first kTickets of
+   * them on any XCD cover every counter, and a counter's waves take its
+   * entries in order, so the smallest unfinished entry is held by a wave or
+   * next on a counter with a wave that holds none. Queue of a 1080p inter
+   * frame (2518 entries) 67 -> 42 us, of a batch of eight (12,400) 169 -> 61. */
+  const int deal = takers >= 16 * kTickets ? kTickets : 1;
+  const int own = ((int)blockIdx.x >> 3) & (deal - 1);
+  const int own_n = (nqueue - own + deal - 1) / deal; /* entries and takers of this counter */
+  const int own_takers = deal == 1 ? takers : takers / (8 * deal) * 8 + clampi(takers % (8 * deal) - 8 * own, 0, 8);
+  uint32_t* counter = B.queue_counter + own * kTicketStep;
   for (;;) {
-    int idx = 0;
-    if (threadIdx.x == 0) idx = (int)atomicAdd(B.queue_counter, 1u);
-    idx = __builtin_amdgcn_readfirstlane(__shfl(idx, 0));
-    if (idx >= nqueue) {
-      /* every taking workgroup takes exactly one entry past the end; the last of
+    int ticket = 0;
+    if (threadIdx.x == 0) ticket = (int)atomicAdd(counter, 1u);
+    ticket = __builtin_amdgcn_readfirstlane(ticket);
+    if (ticket >= own_n) {
+      /* every taking workgroup takes exactly one ticket past the end; the last of
        * those is the counter's last use in this launch, so it resets the
        * counter for the next one */
-      if (threadIdx.x == 0 && idx == nqueue + takers - 1)
-        __hip_atomic_store(B.queue_counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (threadIdx.x == 0 && ticket == own_n + own_takers - 1)
+        __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       return;
     }
+    const int idx = ticket * deal + own;
     const uint64_t t0 = B.trace ? (uint64_t)wall_clock64() : 0;
     int job = 0, blk;
     if (B.queue) {
