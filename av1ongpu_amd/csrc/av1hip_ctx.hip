@@ -208,7 +208,7 @@ struct Ctx {
   /* grain templates depend only on the grain parameters: they are built on a
    * second stream while the frame reconstructs */
   hipStream_t side = nullptr;
-  hipEvent_t ev_side_go = nullptr, ev_side_done = nullptr, ev_itx_done = nullptr;
+  hipEvent_t ev_side_go = nullptr, ev_side_done = nullptr;
   bool timing = false;
   hipEvent_t sev[2 * AV1H_STAGES] = {};
   /* the frame table of a batch this context leads: jobs, prefix table,
@@ -241,7 +241,7 @@ struct Ctx {
   bool graphs = true;
   bool graph_sets = true; /* graphs keyed by the set of kernels with work too */
   Tuning tune;                   /* launch shapes of the batches it leads */
-  std::vector<std::pair<uint64_t, hipGraphExec_t>> graph_exec; /* (kernel set << 8 | frames, graph) */
+  std::vector<std::pair<uint64_t, hipGraphExec_t>> graph_exec; /* (buffer set, size classes, kernel set, frames; graph) */
   bool stage_hit[AV1H_STAGES] = {};
   double stage_ms[AV1H_STAGES] = {};
   int64_t stage_n[AV1H_STAGES] = {};
@@ -2288,22 +2288,40 @@ int batch_launch(Ctx* lead, std::vector<JobSpec>& js, double t0) {
   if (use_graph && !lead->graph_sets) live = ~0ull >> (63 - kKernels); /* every kernel, the queue */
   static_assert(kKernels < 64, "kernel set mask");
   auto has = [&](int k) { return ((live >> k) & 1) != 0; };
+  /* kernels whose work rides in another's launch: CDEF's chroma blocks in
+   * the luma launch, the intra transforms in the inter ones' */
+  auto rider = [](int k) {
+    return k == kKCdefLuma ? (int)kKCdefChroma : k == kKItxInter ? (int)kKItxIntra : k == kKItxInterL ? (int)kKItxIntraL : -1;
+  };
+  auto rides = [](int k) { return k == kKCdefChroma || k == kKItxIntra || k == kKItxIntraL; };
+  auto work_of = [&](int k) { return total_of(k) + (rider(k) >= 0 ? total_of(rider(k)) : 0); };
+  /* A captured launch has one grid for every batch of its key; workgroups
+   * beyond a small frame's work only dispatch and leave, 1-3 us a launch. So
+   * the key also holds the size class of the batch's largest kernel, and of
+   * its queue: grids of at most 256 or 1024 workgroups where that covers all
+   * (any grid is correct, the kernels walk their work). With one graph per
+   * frame count (mode 2) every grid is full. */
+  int grid_class = 2, queue_class = 1;
+  if (use_graph && lead->graph_sets) {
+    int most = 0;
+    for (int k = 0; k < kKernels; ++k)
+      if (!rides(k)) most = std::max(most, work_of(k));
+    grid_class = most <= 256 ? 0 : most <= 1024 ? 1 : 2;
+    queue_class = nq <= 256 ? 0 : 1;
+  }
+  const int grid_cap = grid_class == 0 ? 256 : grid_class == 1 ? 1024 : kAnyTotal;
   auto run = [&](int k, hipStream_t st) -> hipError_t {
-    /* CDEF's luma launch also filters the chroma blocks */
-    if (k == kKCdefChroma) return hipSuccess;
-    const bool work = k == kKCdefLuma ? has(kKCdefLuma) || has(kKCdefChroma) : has(k);
-    const int total = use_graph ? (work ? kAnyTotal : 0)
-                                : total_of(k) + (k == kKCdefLuma ? total_of(kKCdefChroma) : 0);
+    if (rides(k)) return hipSuccess;
+    const bool work = has(k) || (rider(k) >= 0 && has(rider(k)));
+    const int total = use_graph ? (work ? kAnyTotal : 0) : work_of(k);
     if (total <= 0) return hipSuccess;
     ++launches;
-    const int cap = lead->cus * lead->tune.v[k];
+    const int cap = std::min(lead->cus * lead->tune.v[k], grid_cap);
     switch (k) {
       case kKMc:
       case kKSpecial:
       case kKItxInter:
-      case kKItxIntra:
-      case kKItxInterL:
-      case kKItxIntraL: return launch_recon_kernel(B, k, total, cap, st);
+      case kKItxInterL: return launch_recon_kernel(B, k, total, cap, st);
       case kKGrainTemplate:
       case kKGrainApply: return launch_grain_kernel(B, k, total, cap, st);
       default: return launch_filter_kernel(B, k, total, cap, lead->tune.v[kTuneCdefBatch], st);
@@ -2324,10 +2342,8 @@ int batch_launch(Ctx* lead, std::vector<JobSpec>& js, double t0) {
     }
     return hipSuccess;
   };
-  /* The second stream takes what does not depend on the prediction: the
-   * transforms of intra blocks (the queue waits for them) and the grain
-   * templates (the grain blend waits for them). */
-  const bool side_itx = has(kKItxIntra) || has(kKItxIntraL);
+  /* The second stream takes the grain templates, which depend on no picture
+   * (the grain blend waits for them). */
   const bool side_grain = has(kKGrainTemplate);
   auto sequence = [&]() -> hipError_t {
     hipError_t e = hipSuccess;
@@ -2337,25 +2353,19 @@ int batch_launch(Ctx* lead, std::vector<JobSpec>& js, double t0) {
     if (e != hipSuccess) return e; \
   } while (0)
     if (n == 1) SEQ(launch_fetch_table(lead->batch_pin[b], tab, n, s));
-    if (side_itx || side_grain) {
+    if (side_grain) {
       SEQ(hipEventRecord(lead->ev_side_go, s));
       SEQ(hipStreamWaitEvent(lead->side, lead->ev_side_go, 0));
-    }
-    if (side_itx) {
-      SEQ(run(kKItxIntraL, lead->side));
-      SEQ(run(kKItxIntra, lead->side));
-      SEQ(hipEventRecord(lead->ev_itx_done, lead->side));
-    }
-    if (side_grain) {
       SEQ(run(kKGrainTemplate, lead->side));
       SEQ(hipEventRecord(lead->ev_side_done, lead->side));
     }
     if (!use_graph) SEQ(hipEventRecord(lead->bev[b][0], s));
-    SEQ(stage(AV1H_STAGE_INTER, {kKMc, kKSpecial, kKItxInterL, kKItxInter}));
-    if (side_itx) SEQ(hipStreamWaitEvent(s, lead->ev_itx_done, 0));
+    SEQ(stage(AV1H_STAGE_INTER, {kKMc, kKSpecial, kKItxInterL, kKItxIntraL, kKItxInter, kKItxIntra}));
     if (has(kKernels)) {
       if (lead->timing) (void)hipEventRecord(lead->sev[2 * AV1H_STAGE_QUEUE], s);
-      SEQ(launch_queue(B, use_graph ? -1 : (int)nq, lead->cus * lead->tune.v[kTuneQueue], s, &launches));
+      SEQ(launch_queue(B, use_graph ? -1 : (int)nq,
+                       queue_class ? lead->cus * lead->tune.v[kTuneQueue] : std::min(256, lead->cus * lead->tune.v[kTuneQueue]),
+                       s, &launches));
       if (lead->timing) {
         (void)hipEventRecord(lead->sev[2 * AV1H_STAGE_QUEUE + 1], s);
         lead->stage_hit[AV1H_STAGE_QUEUE] = true;
@@ -2384,7 +2394,9 @@ int batch_launch(Ctx* lead, std::vector<JobSpec>& js, double t0) {
   for (bool& h : lead->stage_hit) h = false;
   if (use_graph) {
     hipGraphExec_t exec = nullptr;
-    const uint64_t key = (uint64_t)b << 62 | live << 8 | (uint64_t)n; /* n <= 128 */
+    static_assert(8 + kKernels + 1 <= 48, "graph key");
+    const uint64_t key = (uint64_t)b << 62 | (uint64_t)queue_class << 50 | (uint64_t)grid_class << 48 | live << 8 |
+                         (uint64_t)n; /* n <= 128 */
     for (auto& g : lead->graph_exec)
       if (g.first == key) exec = g.second;
     if (!exec) {
@@ -2647,8 +2659,7 @@ int av1h_create(int device_index, av1h_ctx** out) {
     }
   if (hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking) != hipSuccess ||
       hipEventCreateWithFlags(&c->ev_side_go, hipEventDisableTiming) != hipSuccess ||
-      hipEventCreateWithFlags(&c->ev_side_done, hipEventDisableTiming) != hipSuccess ||
-      hipEventCreateWithFlags(&c->ev_itx_done, hipEventDisableTiming) != hipSuccess) {
+      hipEventCreateWithFlags(&c->ev_side_done, hipEventDisableTiming) != hipSuccess) {
     delete h;
     return AV1H_ERR_DEVICE;
   }
@@ -2699,7 +2710,6 @@ void av1h_destroy(av1h_ctx* h) {
   if (c->side) (void)hipStreamSynchronize(c->side);
   if (c->ev_side_go) (void)hipEventDestroy(c->ev_side_go);
   if (c->ev_side_done) (void)hipEventDestroy(c->ev_side_done);
-  if (c->ev_itx_done) (void)hipEventDestroy(c->ev_itx_done);
   if (c->side) (void)hipStreamDestroy(c->side);
   if (c->stream) (void)hipStreamDestroy(c->stream);
   delete h;

@@ -316,17 +316,25 @@ __device__ __forceinline__ void itx_body(RArgs a, const int32_t* offs, int b, in
   }
 }
 
+/* Both sets of every frame, the inter blocks' first: the intra blocks'
+ * residuals are independent of the prediction, and one launch of both is as
+ * long as one of either on all but the largest frames (a wave's transform is
+ * latency: 1080p inter frame, 32- and 64-point classes, 24 + 27 us in two
+ * launches). */
 template <int C0, int C1>
-__global__ __launch_bounds__(64) void k_itx(BatchDev B, int set) {
+__global__ __launch_bounds__(64) void k_itx(BatchDev B) {
   constexpr int kG = 4 << (C1 - 1);
   __shared__ int s_tmp[64 * (kG + 1)];
-  const int kid = C0 == 0 ? (set ? kKItxIntra : kKItxInter) : (set ? kKItxIntraL : kKItxInterL);
-  const AV1H_CMEM int32_t* pre = kernel_prefix(B, kid);
-  const int total = pre[B.njobs];
+  const AV1H_CMEM int32_t* pre0 = kernel_prefix(B, C0 == 0 ? kKItxInter : kKItxInterL);
+  const AV1H_CMEM int32_t* pre1 = kernel_prefix(B, C0 == 0 ? kKItxIntra : kKItxIntraL);
+  const int inter = pre0[B.njobs], total = inter + pre1[B.njobs];
   for (int v = blockIdx.x; v < total; v += gridDim.x) {
-    const int j = find_job(pre, B.njobs, v);
+    const int set = v >= inter;
+    const AV1H_CMEM int32_t* pre = set ? pre1 : pre0;
+    const int u = set ? v - inter : v;
+    const int j = find_job(pre, B.njobs, u);
     RArgs a = recon_args(B, j);
-    itx_body<C0, C1>(a, a.plan.itx_offs + set * (kTxClasses + 1), v - pre[j], s_tmp);
+    itx_body<C0, C1>(a, a.plan.itx_offs + set * (kTxClasses + 1), u - pre[j], s_tmp);
     __syncthreads();
   }
 }
@@ -2265,10 +2273,9 @@ hipError_t launch_recon_kernel(const BatchDev& b, int k, int total, int cap, hip
   switch (k) {
     case kKMc: hipLaunchKernelGGL(k_mc, grid, dim3(256), 0, s, b); break;
     case kKSpecial: hipLaunchKernelGGL(k_inter_special, grid, dim3(64), 0, s, b); break;
-    case kKItxInter: hipLaunchKernelGGL((k_itx<0, 3>), grid, dim3(64), 0, s, b, 0); break;
-    case kKItxIntra: hipLaunchKernelGGL((k_itx<0, 3>), grid, dim3(64), 0, s, b, 1); break;
-    case kKItxInterL: hipLaunchKernelGGL((k_itx<3, 5>), grid, dim3(64), 0, s, b, 0); break;
-    case kKItxIntraL: hipLaunchKernelGGL((k_itx<3, 5>), grid, dim3(64), 0, s, b, 1); break;
+    /* both sets of transforms in one launch: `total` counts both */
+    case kKItxInter: hipLaunchKernelGGL((k_itx<0, 3>), grid, dim3(64), 0, s, b); break;
+    case kKItxInterL: hipLaunchKernelGGL((k_itx<3, 5>), grid, dim3(64), 0, s, b); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
