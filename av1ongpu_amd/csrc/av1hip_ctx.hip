@@ -1629,6 +1629,7 @@ int flatten(const av1h_frame_desc& f, Plan* plan, Host* H, std::string* err) {
   std::memcpy(P.itx_off, itx_off, sizeof(itx_off));
   P.n_special = (int32_t)H->special_list.size();
   P.mc_tasks = mc_tasks;
+  P.cell_waits = !H->queue_list.empty() && plan->q_counts[1] < plan->q_counts[0];
   P.n_cdef_luma = n_cdef_luma;
   P.n_cdef_dir = (int32_t)H->cdef_dir_list.size();
   P.n_lr_tiles = (int32_t)(H->lr_tiles.size() / 2);

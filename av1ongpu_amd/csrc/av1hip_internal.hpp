@@ -228,6 +228,9 @@ struct FramePlanDev {
   const McItemDev* mc_items;
   const McTaskDev* mc_task;
   int32_t mc_tasks;
+  /* whether a queued block waits on dependency cells (else nobody reads the
+   * cells inter blocks mark) */
+  int32_t cell_waits;
   /* transform blocks: set 0 those of inter blocks, set 1 those of intra
    * blocks; inside a set by class (larger side 4 8 16 32 64), inside a class
    * by size; set s class c is itx_list[itx_off[s][c] .. itx_off[s][c + 1]).

@@ -1959,184 +1959,250 @@ __device__ void reconstruct_queued(RArgs a, BlkRef b, const QBlk& q, int* work, 
 /* Motion compensation, one 256 thread workgroup per task (at most 512
  * samples of consecutive items in coding order, an item being a block or a
  * row strip of a large one):
- *   A  the task's item descriptors (positions, reference windows, LDS
- *      offsets, all computed by the host) are copied into LDS;
+ *   A  a thread per item and one per item's reference turn the host's
+ *      descriptors into what the passes read per lane (addresses, positions,
+ *      places in LDS), with the item of every 16 samples and the reference of
+ *      every 64 intermediates;
  *   B  the horizontal 8 tap pass over every reference row the item's
- *      vertical taps need, the taps read from the reference and clamped to
- *      its visible area the way each tap is (av1gpu_kernels.h:1704-1711),
- *      rounded by InterRound0, into an LDS intermediate (16 bit: at most
- *      200 * 4095 >> 5); neighbouring threads read neighbouring columns, so
- *      the 8 reads of a thread come from the same cache lines;
- *   C  per output sample: the vertical pass, InterRound1, the compound blend
- *      (av1gpu_kernels.h:2207-2293), the store. */
+ *      vertical taps need, four columns per lane, the taps read from the
+ *      reference and clamped to its visible area the way each tap is
+ *      (av1gpu_kernels.h:1704-1711), rounded by InterRound0, into an LDS
+ *      intermediate (16 bit: at most 200 * 4095 >> 5);
+ *   C  per four output samples of a row: the vertical pass, InterRound1, the
+ *      compound blend (av1gpu_kernels.h:2207-2293), one 8 byte store.
+ * Bound by instructions and their latency, not bytes (a 1080p frame's 15 MB
+ * of references and 7 MB of prediction are 5 us at the copy rate), so a lane
+ * takes four neighbouring samples: their item is looked up once, an unscaled
+ * row's eleven samples come in two loads and a scaled sample's eight in one,
+ * and taps are multiplied two at a time (v_dot2_i32_i16: samples and taps are
+ * 16 bit, sums below 2^31); 64 registers keep 8 workgroups on a compute unit.
+ * A launch against one thread per sample: 720p frame 22.5 -> 12.3 us, 1080p
+ * (scaled, compound) 45 -> 30, 2160p 169 -> 104, eight streams 122 -> 58. */
 constexpr int kMcPairs = 2 * kMcItems;
+constexpr int kMcChunkS = 16, kMcChunkM = 64; /* lookup: samples, intermediates */
 
-__device__ __forceinline__ int find_prefix(const int* pre, int n, int v, int lo = 0) {
-  /* the last k < n with pre[k] <= v, known to be >= lo */
-  int hi = n - 1;
-  while (lo < hi) {
-    const int m = (lo + hi + 1) >> 1;
-    if (pre[m] <= v)
-      lo = m;
-    else
-      hi = m - 1;
-  }
-  return lo;
-}
-
-__device__ __forceinline__ McPos mc_pos_of(const McItemDev& it, const McRefDev& r, int sub_x, int sub_y) {
-  McPos P;
-  P.scaled = r.scaled;
-  P.bx = it.x;
-  P.by = it.y;
-  P.sub_x = sub_x;
-  P.sub_y = sub_y;
-  P.ix = r.ix;
-  P.iy = r.iy;
-  P.fx = r.fx;
-  P.fy = r.fy;
-  P.sx0 = r.sx0;
-  P.sy0 = r.sy0;
-  P.stx = r.stx;
-  P.sty = r.sty;
-  return P;
-}
-
+/* one reference of an item, for the horizontal pass: its plane, the column
+ * position of the first sample (stx 0: unscaled, in samples, else in 1/1024
+ * with the step stx), its window's first row, its visible size, its filter row
+ * (unscaled: with the phase) */
+struct __align__(16) McPair {
+  const AV1H_GLOBAL uint16_t* base;
+  int stride, mid, lw, x0, stx, y0, rw, rh, taps, pad;
+};
+/* an item, for the vertical pass; of each reference, its intermediates and the
+ * row position of its first row in them (1/1024) with the step */
+struct __align__(16) McItem {
+  AV1H_GLOBAL uint16_t* out;
+  int stride, px0, lw, compound, w0, w1, taps, plane, ax, ay;
+  struct {
+    int mid, pos, step, pad;
+  } r[2];
+};
 struct McLds {
-  int16_t mid[kMcMid];
-  McItemDev it[kMcItems];
-  int moff[kMcPairs + 1], px[kMcItems + 1];
+  __align__(16) int16_t mid[kMcMid];
+  McPair pair[kMcPairs];
+  McItem item[kMcItems];
+  int moff[kMcPairs + 1];
+  uint8_t item_of[kMcSamples / kMcChunkS], pair_of[kMcMid / kMcChunkM];
 };
 
-/* the 8 taps of a subpel filter row: 8 int16 in one 16-byte LDS read */
-__device__ __forceinline__ void mc_taps(const int16_t* f, int* t) {
-  const int4 v = *reinterpret_cast<const int4*>(f);
-  t[0] = (int)(int16_t)v.x;
-  t[1] = v.x >> 16;
-  t[2] = (int)(int16_t)v.y;
-  t[3] = v.y >> 16;
-  t[4] = (int)(int16_t)v.z;
-  t[5] = v.z >> 16;
-  t[6] = (int)(int16_t)v.w;
-  t[7] = v.w >> 16;
+typedef short mc_s2 __attribute__((ext_vector_type(2)));
+/* n words of sample pairs from any sample's address, one wide load */
+template <int N>
+struct __attribute__((packed, aligned(2))) McWords {
+  uint32_t v[N];
+};
+template <int N>
+__device__ __forceinline__ void load_words(const AV1H_GLOBAL uint16_t* p, uint32_t* s) {
+  const AV1H_GLOBAL McWords<N>* q = (const AV1H_GLOBAL McWords<N>*)p;
+#pragma unroll
+  for (int t = 0; t < N; ++t) s[t] = q->v[t];
 }
+__device__ __forceinline__ int dot2(uint32_t s, int taps, int acc) {
+  return __builtin_amdgcn_sdot2(__builtin_bit_cast(mc_s2, s), __builtin_bit_cast(mc_s2, taps), acc, false);
+}
+/* 8 samples in four words by the 8 taps of a filter row */
+__device__ __forceinline__ int dot8(uint32_t s0, uint32_t s1, uint32_t s2, uint32_t s3, int4 f, int acc) {
+  return dot2(s3, f.w, dot2(s2, f.z, dot2(s1, f.y, dot2(s0, f.x, acc))));
+}
+__device__ __forceinline__ uint32_t pack2(int lo, int hi) { return (uint32_t)(lo & 0xffff) | ((uint32_t)hi << 16); }
 
 __device__ void mc_body(RArgs a, int tn, const int16_t* s_filt, McLds& L_) {
-  int16_t* s_mid = L_.mid;
-  McItemDev* s_it = L_.it;
-  int* s_moff = L_.moff;
-  int* s_px = L_.px;
   const int tid = threadIdx.x;
   const AV1H_CMEM McTaskDev& task = cmem(a.plan.mc_task)[tn];
-  const int nit = task.count, npairs = 2 * nit;
-  {
-    /* all of a thread's loads issued before its LDS writes */
-    const int32_t* src = reinterpret_cast<const int32_t*>(a.plan.mc_items + task.first);
-    int32_t* dst = reinterpret_cast<int32_t*>(s_it);
-    const int n = nit * (int)(sizeof(McItemDev) / 4);
-    constexpr int kPer = (kMcItems * (int)(sizeof(McItemDev) / 4) + 255) / 256;
-    int32_t val[kPer];
+  const int nit = task.count, npairs = 2 * nit, mtotal = task.mtotal, samples = task.samples;
+  const PlaneVals<int> strides = plane_vals(a.lay.stride);
+  const PlaneVals<int64_t> poffs = plane_vals(a.lay.plane_off);
+  if (tid < npairs) {
+    const McItemDev& it = a.plan.mc_items[task.first + (tid >> 1)];
+    const McRefDev& q = it.r[tid & 1];
+    McPair m;
+    m.base = (const AV1H_GLOBAL uint16_t*)a.pool + (size_t)q.slot * a.slot_size + poffs[it.plane];
+    m.stride = strides[it.plane];
+    m.mid = q.mid_off;
+    m.lw = ilog2(it.w);
+    m.x0 = q.scaled ? q.sx0 : it.x + q.ix;
+    m.stx = q.scaled ? q.stx : 0;
+    m.y0 = q.wy0;
+    m.rw = it.ref_w;
+    m.rh = it.ref_h;
+    m.taps = it.hk + (q.scaled ? 0 : q.fx * 8);
+    m.pad = 0;
+    L_.pair[tid] = m;
+    L_.moff[tid] = m.mid;
+    const int end = (tid & 1) < it.nref ? m.mid + q.wh * it.w : m.mid;
+    for (int c = (m.mid + kMcChunkM - 1) / kMcChunkM; c * kMcChunkM < end; ++c) L_.pair_of[c] = (uint8_t)tid;
+  } else if (tid >= 128 && tid < 128 + nit) {
+    const int i = tid - 128;
+    const McItemDev& it = a.plan.mc_items[task.first + i];
+    McItem m;
+    m.plane = it.plane;
+    m.stride = strides[it.plane];
+    m.ax = it.x;
+    m.ay = it.y + it.y0;
+    m.out = (AV1H_GLOBAL uint16_t*)a.frame + poffs[it.plane] + (int64_t)m.ay * m.stride + m.ax;
+    m.px0 = it.px0;
+    m.lw = ilog2(it.w);
+    m.compound = it.compound;
+    m.w0 = it.w0;
+    m.w1 = it.w1;
+    m.taps = it.vk;
 #pragma unroll
-    for (int u = 0; u < kPer; ++u) val[u] = tid + 256 * u < n ? src[tid + 256 * u] : 0;
-#pragma unroll
-    for (int u = 0; u < kPer; ++u)
-      if (tid + 256 * u < n) dst[tid + 256 * u] = val[u];
+    for (int r = 0; r < 2; ++r) {
+      const McRefDev& q = it.r[r];
+      m.r[r].mid = q.mid_off;
+      m.r[r].pos = q.scaled ? q.sy0 + q.sty * it.y0 - ((q.wy0 + 3) << 10) : q.fy << 6;
+      m.r[r].step = q.scaled ? q.sty : 1024;
+      m.r[r].pad = 0;
+    }
+    L_.item[i] = m;
+    /* blocks hold multiples of 16 samples: a chunk lies in one item */
+    for (int c = m.px0 / kMcChunkS; c * kMcChunkS < m.px0 + (it.rows << m.lw); ++c) L_.item_of[c] = (uint8_t)i;
   }
-  __syncthreads();
-  if (tid < npairs) s_moff[tid] = s_it[tid >> 1].r[tid & 1].mid_off;
-  if (tid < nit) s_px[tid] = s_it[tid].px0;
-  if (tid == 0) {
-    s_moff[npairs] = task.mtotal;
-    s_px[nit] = task.samples;
-  }
+  if (tid == 0) L_.moff[npairs] = mtotal;
   __syncthreads();
   const int bd = a.lay.bit_depth;
   const int round0 = bd >= 12 ? 5 : 3;
-  const PlaneVals<int> strides = plane_vals(a.lay.stride);
-  const PlaneVals<int64_t> poffs = plane_vals(a.lay.plane_off);
+  const int add0 = 1 << (round0 - 1);
   /* horizontal pass over every reference row an item needs, taps read from
-   * the reference (clamped to it) */
-  int kprev = 0;
-  for (int e = tid; e < task.mtotal; e += 256) {
-    const int k = kprev = find_prefix(s_moff, npairs, e, kprev);
-    const McItemDev& it = s_it[k >> 1];
-    const McRefDev& q = it.r[k & 1];
-    const int o = e - q.mid_off;
-    const int lw = ilog2(it.w);
-    const int rr = o >> lw, x = o & (it.w - 1);
-    const int p = it.plane;
-    const int sub_x = p > 0 ? a.lay.ss_x : 0;
-    const McPos P = mc_pos_of(it, q, sub_x, 0);
-    int cx, fx;
-    P.col(x, &cx, &fx);
-    const int y = clampi(q.wy0 + rr, 0, it.ref_h - 1);
-    const uint16_t* row = a.pool + (size_t)q.slot * a.slot_size + poffs[p] + (size_t)y * strides[p];
-    int hk[8];
-    mc_taps(s_filt + it.hk + fx * 8, hk);
-    int sum = 0;
-    if (cx >= 3 && cx + 4 < it.ref_w) {
+   * the reference (clamped to it); block widths are multiples of 4, so the
+   * four intermediates lie in one row */
+  for (int e = tid * 4; e < mtotal; e += 1024) {
+    int k = L_.pair_of[e / kMcChunkM];
+    while (L_.moff[k + 1] <= e) ++k;
+    const McPair q = L_.pair[k];
+    const int o = e - q.mid, rr = o >> q.lw, x = o & ((1 << q.lw) - 1);
+    const int y = clampi(q.y0 + rr, 0, q.rh - 1);
+    const AV1H_GLOBAL uint16_t* row = q.base + (int64_t)y * q.stride;
+    int v[4];
+    if (!q.stx) {
+      const int cx = q.x0 + x;
+      const int4 f = *reinterpret_cast<const int4*>(s_filt + q.taps);
+      uint32_t s[6];
+      if (cx >= 3 && cx + 7 < q.rw) {
+        /* cx - 3 .. cx + 7 (and one of the row's padding at its end) */
+        load_words<4>(row + cx - 3, s);
+        load_words<2>(row + cx + 5, s + 4);
+      } else {
 #pragma unroll
-      for (int t = 0; t < 8; ++t) sum += (int)row[cx - 3 + t] * hk[t];
+        for (int t = 0; t < 6; ++t)
+          s[t] = pack2(row[clampi(cx - 3 + 2 * t, 0, q.rw - 1)], row[clampi(cx - 2 + 2 * t, 0, q.rw - 1)]);
+      }
+      uint32_t m[5]; /* the pairs in between */
+#pragma unroll
+      for (int t = 0; t < 5; ++t) m[t] = __builtin_amdgcn_alignbit(s[t + 1], s[t], 16);
+      v[0] = dot8(s[0], s[1], s[2], s[3], f, add0);
+      v[1] = dot8(m[0], m[1], m[2], m[3], f, add0);
+      v[2] = dot8(s[1], s[2], s[3], s[4], f, add0);
+      v[3] = dot8(m[1], m[2], m[3], m[4], f, add0);
     } else {
+      uint32_t s[4][4];
+      const int pos = q.x0 + q.stx * x;
+      if ((pos >> 10) >= 3 && ((pos + 3 * q.stx) >> 10) + 4 < q.rw) {
 #pragma unroll
-      for (int t = 0; t < 8; ++t) sum += (int)row[clampi(cx - 3 + t, 0, it.ref_w - 1)] * hk[t];
+        for (int i = 0; i < 4; ++i) load_words<4>(row + ((pos + i * q.stx) >> 10) - 3, s[i]);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int cx = (pos + i * q.stx) >> 10;
+#pragma unroll
+          for (int t = 0; t < 4; ++t)
+            s[i][t] = pack2(row[clampi(cx - 3 + 2 * t, 0, q.rw - 1)], row[clampi(cx - 2 + 2 * t, 0, q.rw - 1)]);
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int ph = ((pos + i * q.stx) & 1023) >> 6;
+        v[i] = dot8(s[i][0], s[i][1], s[i][2], s[i][3], *reinterpret_cast<const int4*>(s_filt + q.taps + ph * 8), add0);
+      }
     }
-    s_mid[e] = (int16_t)((sum + (1 << (round0 - 1))) >> round0);
+    uint2 out;
+    out.x = pack2(v[0] >> round0, v[1] >> round0);
+    out.y = pack2(v[2] >> round0, v[3] >> round0);
+    *reinterpret_cast<uint2*>(L_.mid + e) = out;
   }
   __syncthreads();
-  /* vertical pass and blend, one thread per output sample */
-  const PlaneVals<int> cshift = plane_vals(a.lay.cell_shift), cwidth = plane_vals(a.lay.cells_w),
-                       cheight = plane_vals(a.lay.cells_h);
-  const PlaneVals<int64_t> coffs = plane_vals(a.lay.cell_off);
-  int iprev = 0;
-  for (int si = tid; si < task.samples; si += 256) {
-    const int item = iprev = find_prefix(s_px, nit, si, iprev);
-    const McItemDev& it = s_it[item];
-    const int s = si - it.px0;
-    const int lw = ilog2(it.w), x = s & (it.w - 1), y = it.y0 + (s >> lw);
-    const int compound = it.compound != 0;
+  /* vertical pass and blend, four output samples of a row per lane */
+  for (int si = tid * 4; si < samples; si += 1024) {
+    const McItem& it = L_.item[L_.item_of[si / kMcChunkS]];
+    const int s = si - it.px0, lw = it.lw, w = 1 << lw;
+    const int x = s & (w - 1), ry = s >> lw;
+    const int compound = it.compound;
     int round1 = compound ? 7 : 11;
     if (bd >= 12 && !compound) round1 -= 2;
-    const int sub_y = it.plane > 0 ? a.lay.ss_y : 0;
-    int v[2] = {0, 0};
+    int v[2][4] = {};
 #pragma unroll
     for (int r = 0; r < 2; ++r) {
       if (r == 1 && !compound) break;
-      const McRefDev& q = it.r[r];
-      const McPos P = mc_pos_of(it, q, 0, sub_y);
-      int cy, fy;
-      P.row(y, &cy, &fy);
-      const int16_t* m = s_mid + q.mid_off + (cy - 3 - q.wy0) * it.w + x;
-      int vk[8];
-      mc_taps(s_filt + it.vk + fy * 8, vk);
-      int acc = 0;
+      const int pos = it.r[r].pos + it.r[r].step * ry;
+      const int16_t* m = L_.mid + it.r[r].mid + ((pos >> 10) << lw) + x;
+      const int4 f = *reinterpret_cast<const int4*>(s_filt + it.taps + ((pos & 1023) >> 6) * 8);
+      const int ft[4] = {f.x, f.y, f.z, f.w};
+      int acc[4];
 #pragma unroll
-      for (int t = 0; t < 8; ++t) acc += (int)m[t * it.w] * vk[t];
-      v[r] = (acc + (1 << (round1 - 1))) >> round1;
+      for (int i = 0; i < 4; ++i) acc[i] = 1 << (round1 - 1);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        /* two rows' columns side by side: low halves, high halves */
+        const uint2 u = *reinterpret_cast<const uint2*>(m + ((2 * t) << lw));
+        const uint2 d = *reinterpret_cast<const uint2*>(m + ((2 * t + 1) << lw));
+        acc[0] = dot2(__builtin_amdgcn_perm(d.x, u.x, 0x05040100u), ft[t], acc[0]);
+        acc[1] = dot2(__builtin_amdgcn_perm(d.x, u.x, 0x07060302u), ft[t], acc[1]);
+        acc[2] = dot2(__builtin_amdgcn_perm(d.y, u.y, 0x05040100u), ft[t], acc[2]);
+        acc[3] = dot2(__builtin_amdgcn_perm(d.y, u.y, 0x07060302u), ft[t], acc[3]);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[r][i] = acc[i] >> round1;
     }
-    int out = v[0];
-    if (compound) {
-      const int post = 2 * 7 - (round0 + 7);
-      if (it.compound == AV1H_COMPOUND_AVERAGE)
-        out = (v[0] + v[1] + (1 << post)) >> (1 + post);
-      else
-        out = (it.w0 * v[0] + it.w1 * v[1] + (1 << (3 + post))) >> (4 + post);
+    const int post = 2 * 7 - (round0 + 7), w0 = it.w0, w1 = it.w1;
+    int out[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      int o = v[0][i];
+      if (compound) {
+        if (compound == AV1H_COMPOUND_AVERAGE)
+          o = (v[0][i] + v[1][i] + (1 << post)) >> (1 + post);
+        else
+          o = (w0 * v[0][i] + w1 * v[1][i] + (1 << (3 + post))) >> (4 + post);
+      }
+      out[i] = clampi(o, 0, a.maxv);
     }
-    const int p = it.plane;
-    const int ax = it.x + x, ay = it.y + y;
-    a.frame[poffs[p] + (int64_t)ay * strides[p] + ax] = (uint16_t)clampi(out, 0, a.maxv);
-    /* the block's dependency cells, each by the thread of its first sample
-     * in the block: final once the inter transforms after this launch have
+    *(AV1H_GLOBAL uint64_t*)(it.out + (int64_t)ry * it.stride + x) =
+        (uint64_t)pack2(out[2], out[3]) << 32 | pack2(out[0], out[1]);
+    /* the block's dependency cells (2 or 4 samples a side; blocks lie on
+     * multiples of 4): final once the inter transforms after this launch have
      * run, which the queue launch follows */
-    const int sh = cshift[p], cm = (1 << sh) - 1;
-    if (((ax & cm) == 0 || x == 0) && ((ay & cm) == 0 || y == 0)) {
-      const int cx = ax >> sh, cy = ay >> sh;
-      if (cx < cwidth[p] && cy < cheight[p]) a.cells[coffs[p] + (int64_t)cy * cwidth[p] + cx] = a.epoch;
+    const int p = it.plane, sh = plane_vals(a.lay.cell_shift)[p], ax = it.ax + x, ay = it.ay + ry;
+    if (a.plan.cell_waits && (ay & ((1 << sh) - 1)) == 0) {
+      const int cw = plane_vals(a.lay.cells_w)[p], cy = ay >> sh;
+      uint32_t* cells = a.cells + plane_vals(a.lay.cell_off)[p] + (int64_t)cy * cw;
+      for (int cx = ax >> sh; cx << sh < ax + 4; ++cx)
+        if (cx < cw && cy < plane_vals(a.lay.cells_h)[p]) cells[cx] = a.epoch;
     }
   }
 }
 
-__global__ __launch_bounds__(256) void k_mc(BatchDev B) {
+__global__ __launch_bounds__(256, 8) void k_mc(BatchDev B) {
   __shared__ __align__(16) int16_t s_filt[768];
   __shared__ McLds s_lds;
   for (int i = threadIdx.x; i < 768; i += 256) s_filt[i] = (int16_t)av1t_spec_table[AV1T_OFF_SUBPEL + i];
@@ -2165,7 +2231,7 @@ __global__ __launch_bounds__(64) void k_inter_special(BatchDev B) {
     uint16_t* dst = a.frame + a.lay.plane_off[p] + (size_t)b.y * stride + b.x;
     for (int s = threadIdx.x; s < b.w * b.h; s += 64)
       dst[(size_t)(s >> lw) * stride + (s & (b.w - 1))] = (uint16_t)inter_sample(a, b, s & (b.w - 1), s >> lw);
-    mark_cells(a, b, false);
+    if (a.plan.cell_waits) mark_cells(a, b, false);
   }
 }
 
