@@ -1004,6 +1004,13 @@ int flatten(const av1h_frame_desc& f, Plan* plan, Host* H, std::string* err) {
           d.dep_corner = 0;
         }
         if (!b.intrabc) d.dep_rx1 = d.dep_rx0 - 1;
+        /* the inter half of inter/intra reads references only: computed ahead
+         * of the queue (overlapped motion compensation blends after the
+         * intra half, so a block with both keeps the one path) */
+        if (b.interintra && !b.intrabc && d.obmc_count == 0) {
+          d.flags |= kInterDone;
+          H->special_list.push_back(i);
+        }
         H->queue_list.push_back(i);
       } else if (special) {
         H->special_list.push_back(i);
@@ -2012,7 +2019,7 @@ int kernel_groups(const FrameJob& fj, int k, int cdef_batch) {
   const Layout& L = fj.r.lay;
   switch (k) {
     case kKMc: return p.mc_tasks;
-    case kKSpecial: return p.n_special;
+    case kKSpecial: return p.n_special * kSpecialStrips;
     case kKItxInter: return itx_groups(p, 0, 0, 3);
     case kKItxIntra: return itx_groups(p, 1, 0, 3);
     case kKItxInterL: return itx_groups(p, 0, 3, kTxClasses);

@@ -61,7 +61,10 @@ enum {
    * kEdgeRow / kEdgeCol - the block publishes its last row / column as
    * packed words; kSkipMark - no block waits on its cells */
   kPackedEdges = 1 << 15, kCornerRow = 1 << 16, kEdgeRow = 1 << 17, kEdgeCol = 1 << 18, kSkipMark = 1 << 19,
-  kCornerFrame = 1 << 20
+  kCornerFrame = 1 << 20,
+  /* inter/intra: the inter prediction is in the frame before the queue starts
+   * (k_inter_special), the queue blends the intra part in */
+  kInterDone = 1 << 21
 };
 
 struct DevBlock {
@@ -364,6 +367,9 @@ constexpr int kMaxBatch = 128;
  * idx % counters (k_queue). */
 constexpr int kTickets = 8, kTicketStep = 512;
 constexpr size_t kCounterBytes = (size_t)(kTickets + 1) * kTicketStep * 4;
+
+/* k_inter_special: workgroups (of one wave) that share a block's samples */
+constexpr int kSpecialStrips = 4;
 
 /* CDEF: groups of 256 / (block samples) blocks a workgroup takes per step
  * (a thread's samples of up to kCdefMaxBatch blocks computed together) */

@@ -37,6 +37,9 @@ namespace {
 
 constexpr int kWork = 2048;            /* int32 intra work area (edges, CFL)    */
 
+/* global (not generic) pointers: their accesses need no wait for LDS */
+#define AV1H_GLOBAL __attribute__((address_space(1)))
+
 __device__ __forceinline__ int clampi(int v, int lo, int hi) { return v < lo ? lo : (v > hi ? hi : v); }
 __device__ __forceinline__ int rnd2(int v, int n) { return n <= 0 ? v : (v + (1 << (n - 1))) >> n; }
 __device__ __forceinline__ int rnd2s(int v, int n) {
@@ -412,18 +415,52 @@ __device__ const uint16_t* ref_plane(RArgs a, int slot, int plane) {
 /* direct way; samples of the frame being decoded are read at device scope.  */
 /* ------------------------------------------------------------------------ */
 
-__device__ __forceinline__ int fetch_px(const uint16_t* p, bool cur, int stride, int x, int y, int x1, int y1) {
-  x = clampi(x, 0, x1);
-  y = clampi(y, 0, y1);
-  const uint16_t* q = p + (size_t)y * stride + x;
-  return cur ? ld_dev(q) : (int)*q;
+typedef short mc_s2 __attribute__((ext_vector_type(2)));
+/* n words of sample pairs from any sample's address, one wide load */
+template <int N>
+struct __attribute__((packed, aligned(2))) McWords {
+  uint32_t v[N];
+};
+template <int N>
+__device__ __forceinline__ void load_words(const AV1H_GLOBAL uint16_t* p, uint32_t* s) {
+  const AV1H_GLOBAL McWords<N>* q = (const AV1H_GLOBAL McWords<N>*)p;
+#pragma unroll
+  for (int t = 0; t < N; ++t) s[t] = q->v[t];
+}
+__device__ __forceinline__ int dot2(uint32_t s, int taps, int acc) {
+  return __builtin_amdgcn_sdot2(__builtin_bit_cast(mc_s2, s), __builtin_bit_cast(mc_s2, taps), acc, false);
+}
+/* 8 samples in four words by the 8 taps of a filter row */
+__device__ __forceinline__ int dot8(uint32_t s0, uint32_t s1, uint32_t s2, uint32_t s3, int4 f, int acc) {
+  return dot2(s3, f.w, dot2(s2, f.z, dot2(s1, f.y, dot2(s0, f.x, acc))));
+}
+__device__ __forceinline__ uint32_t pack2(int lo, int hi) { return (uint32_t)(lo & 0xffff) | ((uint32_t)hi << 16); }
+
+/* the 8 samples x - 3 .. x + 4 of row y, clamped to the reference's visible
+ * area, as four words. kCur: the frame being decoded, whose samples other
+ * waves of this launch write (device scope loads); a finished reference is
+ * read in one wide load where no clamp moves a sample. */
+template <bool kCur>
+__device__ __forceinline__ void ref_row8(const uint16_t* p, int stride, int x, int y, int x1, int y1, uint32_t* s) {
+  const AV1H_GLOBAL uint16_t* row = (const AV1H_GLOBAL uint16_t*)p + (int64_t)clampi(y, 0, y1) * stride;
+  if (!kCur && x >= 3 && x + 4 <= x1) {
+    load_words<4>(row + x - 3, s);
+    return;
+  }
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    const AV1H_GLOBAL uint16_t* lo = row + clampi(x - 3 + 2 * t, 0, x1);
+    const AV1H_GLOBAL uint16_t* hi = row + clampi(x - 2 + 2 * t, 0, x1);
+    s[t] = kCur ? pack2(ld_dev((const uint16_t*)lo), ld_dev((const uint16_t*)hi)) : pack2(*lo, *hi);
+  }
 }
 
 /* one sample of one reference through the two stage filter, unscaled or
- * scaled (av1gpu_kernels.h:1756-1857) */
-__device__ int mc_tap(const uint16_t* ref, bool cur, int stride, int ref_w, int ref_h, int sub_x, int sub_y,
-                      int scx, int scy, int bx, int by, int ew, int eh, int mvx, int mvy, int filt, int filt_v,
-                      int x, int y, int compound, int bd) {
+ * scaled (av1gpu_kernels.h:1756-1857), its eight rows' loads all in flight */
+template <bool kCur>
+__device__ __forceinline__ int mc_tap(const uint16_t* ref, int stride, int ref_w, int ref_h, int sub_x, int sub_y,
+                                      int scx, int scy, int bx, int by, int ew, int eh, int mvx, int mvy, int filt,
+                                      int filt_v, int x, int y, int compound, int bd) {
   const int round0 = bd >= 12 ? 5 : 3;
   int round1 = compound ? 7 : 11;
   if (bd >= 12 && !compound) round1 -= 2;
@@ -433,21 +470,23 @@ __device__ int mc_tap(const uint16_t* ref, bool cur, int stride, int ref_w, int 
   P.row(y, &cy, &fy);
   const int* hk = SPEC(AV1T_OFF_SUBPEL) + (filt_row(filt, ew) * 16 + fx) * 8;
   const int* vk = SPEC(AV1T_OFF_SUBPEL) + (filt_row(filt_v, eh) * 16 + fy) * 8;
+  uint32_t s[8][4];
+#pragma unroll
+  for (int r = 0; r < 8; ++r) ref_row8<kCur>(ref, stride, cx, cy - 3 + r, ref_w - 1, ref_h - 1, s[r]);
+  const int4 f = make_int4(pack2(hk[0], hk[1]), pack2(hk[2], hk[3]), pack2(hk[4], hk[5]), pack2(hk[6], hk[7]));
   int acc = 0;
-  for (int r = 0; r < 8; ++r) {
-    int s = 0;
-    for (int t = 0; t < 8; ++t) s += fetch_px(ref, cur, stride, cx - 3 + t, cy - 3 + r, ref_w - 1, ref_h - 1) * hk[t];
-    acc += ((s + (1 << (round0 - 1))) >> round0) * vk[r];
-  }
+#pragma unroll
+  for (int r = 0; r < 8; ++r) acc += __mul24(dot8(s[r][0], s[r][1], s[r][2], s[r][3], f, 1 << (round0 - 1)) >> round0, vk[r]);
   return (acc + (1 << (round1 - 1))) >> round1;
 }
 
 __device__ __forceinline__ int warp_offs(int v) { return clampi(((v + 512) >> 10) + 64, 0, 192); }
 
 /* one sample of a warped reference (av1gpu_kernels.h:1919-1958) */
-__device__ int warp_tap(int sub_x, int sub_y, int ref_w, int ref_h, const AV1H_CMEM int* wp, const AV1H_CMEM int* abcd,
-                        const uint16_t* ref, bool cur, int stride, int bx, int by, int x, int y, int bd,
-                        int compound) {
+template <bool kCur>
+__device__ __forceinline__ int warp_tap(int sub_x, int sub_y, int ref_w, int ref_h, const AV1H_CMEM int* wp,
+                                        const AV1H_CMEM int* abcd, const uint16_t* ref, int stride, int bx, int by,
+                                        int x, int y, int bd, int compound) {
   const int* wf = SPEC(AV1T_OFF_WARP);
   const int i1 = (y & 7) - 4, i2 = (x & 7) - 4;
   const int64_t srcx = (int64_t)((bx + (x >> 3) * 8 + 4) << sub_x);
@@ -461,14 +500,15 @@ __device__ int warp_tap(int sub_x, int sub_y, int ref_w, int ref_h, const AV1H_C
   int round1 = compound ? 7 : 11;
   if (bd >= 12 && !compound) round1 -= 2;
   const int oy = warp_offs(sy4 + abcd[2] * i2 + abcd[3] * i1);
+  uint32_t s[8][4];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) ref_row8<kCur>(ref, stride, ix4 + i2, iy4 + i1 - 3 + k, ref_w - 1, ref_h - 1, s[k]);
   int acc = 0;
+#pragma unroll
   for (int k = 0; k < 8; ++k) {
-    const int row = i1 - 3 + k;
-    const int ox = warp_offs(sx4 + abcd[0] * i2 + abcd[1] * row);
-    int s = 0;
-    for (int t = 0; t < 8; ++t)
-      s += wf[ox * 8 + t] * fetch_px(ref, cur, stride, ix4 + i2 - 3 + t, iy4 + row, ref_w - 1, ref_h - 1);
-    acc += ((s + (1 << (round0 - 1))) >> round0) * wf[oy * 8 + k];
+    const int* w = wf + warp_offs(sx4 + abcd[0] * i2 + abcd[1] * (i1 - 3 + k)) * 8;
+    const int4 f = make_int4(pack2(w[0], w[1]), pack2(w[2], w[3]), pack2(w[4], w[5]), pack2(w[6], w[7]));
+    acc += __mul24(dot8(s[k][0], s[k][1], s[k][2], s[k][3], f, 1 << (round0 - 1)) >> round0, wf[oy * 8 + k]);
   }
   return (acc + (1 << (round1 - 1))) >> round1;
 }
@@ -587,6 +627,7 @@ __device__ int ii_mask(BlkRef b, int sub_x, int sub_y, int xs, int ys) {
 
 /* Sample (xs, ys) of a block using any inter tool (av1gpu_kernels.h:2207-2326).
  * References of slot -1 (intra block copy) are the frame being decoded. */
+template <bool kCur>
 __device__ __forceinline__ int inter_sample(RArgs a, BlkRef b, int xs, int ys) {
   LayRef L = a.lay;
   const int p = b.plane, bd = L.bit_depth;
@@ -596,12 +637,11 @@ __device__ __forceinline__ int inter_sample(RArgs a, BlkRef b, int xs, int ys) {
   int v[2] = {0, 0};
   for (int r = 0; r < (compound ? 2 : 1); ++r) {
     const uint16_t* base = ref_plane(a, b.slot[r], p);
-    const bool cur = b.slot[r] < 0;
     const int cmp = r ? 1 : compound;
     v[r] = (b.flags & (r ? kWarp1 : kWarp0))
-               ? warp_tap(sub_x, sub_y, b.ref_w, b.ref_h, b.warp_params[r], b.warp_abcd[r], base, cur, stride,
+               ? warp_tap<kCur>(sub_x, sub_y, b.ref_w, b.ref_h, b.warp_params[r], b.warp_abcd[r], base, stride,
                           b.x, b.y, xs, ys, bd, cmp)
-               : mc_tap(base, cur, stride, b.ref_w, b.ref_h, sub_x, sub_y, b.scale_x, b.scale_y, b.x, b.y, b.w,
+               : mc_tap<kCur>(base, stride, b.ref_w, b.ref_h, sub_x, sub_y, b.scale_x, b.scale_y, b.x, b.y, b.w,
                         b.h, b.mv[r][0], b.mv[r][1], b.filt, b.filt_v, xs, ys, cmp, bd);
   }
   int out = v[0];
@@ -626,11 +666,10 @@ __device__ __forceinline__ int inter_sample(RArgs a, BlkRef b, int xs, int ys) {
             int lv[2];
             for (int r = 0; r < 2; ++r) {
               const uint16_t* lb = ref_plane(a, b.slot[r], 0);
-              const bool cur = b.slot[r] < 0;
               lv[r] = (b.flags & (r ? kMaskWarp1 : kMaskWarp0))
-                          ? warp_tap(0, 0, L.out_w[0], L.out_h[0], b.warp_params[r], b.warp_abcd[r], lb, cur,
+                          ? warp_tap<kCur>(0, 0, L.out_w[0], L.out_h[0], b.warp_params[r], b.warp_abcd[r], lb,
                                      L.stride[0], b.x << L.ss_x, b.y << L.ss_y, lx, ly, bd, 1)
-                          : mc_tap(lb, cur, L.stride[0], L.out_w[0], L.out_h[0], 0, 0, b.scale_x, b.scale_y,
+                          : mc_tap<kCur>(lb, L.stride[0], L.out_w[0], L.out_h[0], 0, 0, b.scale_x, b.scale_y,
                                    b.x << L.ss_x, b.y << L.ss_y, b.w << sub_x, b.h << sub_y, b.mv[r][0],
                                    b.mv[r][1], b.filt, b.filt_v, lx, ly, 1, bd);
             }
@@ -648,7 +687,7 @@ __device__ __forceinline__ int inter_sample(RArgs a, BlkRef b, int xs, int ys) {
     }
   }
   out = clampi(out, 0, a.maxv);
-  if (b.flags & kInterIntra) {
+  if ((b.flags & (kInterIntra | kInterDone)) == kInterIntra) {
     IiCtx c;
     c.p = a.frame + L.plane_off[p] + (size_t)b.y * stride + b.x;
     c.stride = stride;
@@ -670,12 +709,20 @@ __device__ __forceinline__ int inter_sample(RArgs a, BlkRef b, int xs, int ys) {
     const int cj = xs - o.rx, ci = ys - o.ry;
     const int m = o.pass == 0 ? obmc_mask(o.h, ci) : obmc_mask(o.w, cj);
     const uint16_t* base = ref_plane(a, o.slot, p);
-    int pred = mc_tap(base, o.slot < 0, stride, b.ref_w, b.ref_h, sub_x, sub_y, b.scale_x, b.scale_y, b.x + o.rx,
+    int pred = mc_tap<false>(base, stride, b.ref_w, b.ref_h, sub_x, sub_y, b.scale_x, b.scale_y, b.x + o.rx,
                       b.y + o.ry, o.w, o.h, o.mvx, o.mvy, o.filt, o.filt_v, cj, ci, 0, bd);
     pred = clampi(pred, 0, a.maxv);
     out = (m * out + (64 - m) * pred + 32) >> 6;
   }
   return out;
+}
+
+/* inter_sample as a call, for the queue: inlined there it takes the registers
+ * of every block's path */
+template <bool kCur>
+__device__ __noinline__ int queue_inter(const AV1H_CMEM ReconArgs* args, const AV1H_CMEM DevBlock* block, int xs, int ys) {
+  return inter_sample<kCur>(*(const AV1H_CMEM ReconArgs*)sreg((int64_t)args),
+                            *(const AV1H_CMEM DevBlock*)sreg((int64_t)block), xs, ys);
 }
 
 /* ------------------------------------------------------------------------ */
@@ -709,7 +756,6 @@ static_assert(kPrep2 + 2 * (kEdge + 2 * kEdgeOff) <= kWork, "edge preparation ar
  * one after another (the plane's strides and offsets, then the address):
  * about 0.3 us of each block's work after its wait (2.13 -> 1.85 us on the
  * 1080p key frame) that now overlaps the wait. */
-#define AV1H_GLOBAL __attribute__((address_space(1)))
 struct QBlk {
   int x, y, w, h, plane, kind, flags, mode, dir_a, dir_b;
   int stride, max_x, max_y, maxv, bd;
@@ -1909,15 +1955,93 @@ __device__ __forceinline__ void queue_big(RArgs a, BlkRef b, const QBlk& q, bool
   }
 }
 
+/* ---- inter/intra blocks whose inter half is done -----------------------
+ * Before the wait the inter samples go to `pred` and the blend masks to bytes
+ * in the work area; after it the edges are read once (the per sample path
+ * read each DC sample's w + h neighbours again), then every sample is a blend
+ * of values in LDS (av1gpu_kernels.h:2120-2205). */
+constexpr int kIiMask = 512; /* the masks' place in the work area, in words */
+static_assert(kIiMask + 64 * 64 / 4 <= kWork, "inter/intra masks");
+
+__device__ __forceinline__ void ii_ahead(RArgs a, BlkRef b, const QBlk& q, int* work, uint16_t* pred) {
+  const int n = q.w * q.h, lw = ilog2(q.w);
+  const int sub_x = q.plane > 0 ? a.lay.ss_x : 0, sub_y = q.plane > 0 ? a.lay.ss_y : 0;
+  uint8_t* mask = reinterpret_cast<uint8_t*>(work + kIiMask);
+  for (int s0 = threadIdx.x; s0 < n; s0 += 64 * 4) {
+    uint16_t v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int s = s0 + 64 * u;
+      v[u] = s < n ? q.dst[(int64_t)(s >> lw) * q.stride + (s & (q.w - 1))] : 0;
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int s = s0 + 64 * u;
+      if (s >= n) break;
+      pred[s] = v[u];
+      mask[s] = (uint8_t)ii_mask(b, sub_x, sub_y, s & (q.w - 1), s >> lw);
+    }
+  }
+}
+
+__device__ __forceinline__ void ii_blend(BlkRef b, const QBlk& q, int* work, uint16_t* pred) {
+  const int lane = threadIdx.x, w = q.w, h = q.h, lw = ilog2(w), mode = b.ii_mode;
+  const bool ha = (q.flags & kHaveAbove) != 0, hl = (q.flags & kHaveLeft) != 0;
+  int* above = work;
+  int* left = work + 64;
+  const uint8_t* mask = reinterpret_cast<const uint8_t*>(work + kIiMask);
+  IiCtx c;
+  c.p = (const uint16_t*)q.dst;
+  c.stride = q.stride;
+  c.x = q.x;
+  c.y = q.y;
+  c.w = w;
+  c.h = h;
+  c.max_x = q.max_x;
+  c.max_y = q.max_y;
+  c.have_left = hl;
+  c.have_above = ha;
+  c.bd = q.bd;
+  const int va = lane < w ? c.above(lane) : 0, vl = lane < h ? c.left(lane) : 0;
+  above[lane] = va;
+  left[lane] = vl;
+  wsync();
+  int dc = 1 << (q.bd - 1);
+  if (mode == 0 && (ha || hl)) {
+    const int sum = wave_total((ha ? va : 0) + (hl ? vl : 0));
+    dc = ha && hl ? (sum + ((w + h) >> 1)) / (w + h) : hl ? (sum + (h >> 1)) >> ilog2(h) : (sum + (w >> 1)) >> lw;
+  }
+  const int* sw = SPEC(AV1T_OFF_SM_WEIGHTS);
+  for (int s = lane; s < w * h; s += 64) {
+    const int x = s & (w - 1), y = s >> lw;
+    int v = dc;
+    if (mode == 1) {
+      v = above[x];
+    } else if (mode == 2) {
+      v = left[y];
+    } else if (mode == 3) {
+      const int wy = sw[h - 4 + y], wx = sw[w - 4 + x];
+      v = rnd2(wy * above[x] + (256 - wy) * left[h - 1] + wx * left[y] + (256 - wx) * above[w - 1], 9);
+    }
+    const int m = mask[s];
+    pred[s] = (uint16_t)((m * v + (64 - m) * (int)pred[s] + 32) >> 6);
+  }
+  wsync();
+}
+
 __device__ void reconstruct_queued(RArgs a, BlkRef b, const QBlk& q, int* work, uint16_t* pred, const EarlyRes& er,
                                    const int* tab, uint32_t* error) {
   bool fused = false;
   if (q.kind == kIntra) {
     fused = predict_intra(a, b, q, work, pred, tab, er, error);
+  } else if (q.flags & kInterDone) {
+    ii_blend(b, q, work, pred);
   } else {
     /* inter/intra or intra block copy: reads the frame being decoded */
     const int lw = ilog2(b.w);
-    for (int s = threadIdx.x; s < b.w * b.h; s += 64) pred[s] = (uint16_t)inter_sample(a, b, s & (b.w - 1), s >> lw);
+    for (int s = threadIdx.x; s < b.w * b.h; s += 64)
+      pred[s] = (uint16_t)(q.flags & kIntraBC ? queue_inter<true>(&a, &b, s & (b.w - 1), s >> lw)
+                                              : queue_inter<false>(&a, &b, s & (b.w - 1), s >> lw));
     wsync();
   }
   const int p = q.plane, stride = q.stride;
@@ -2005,27 +2129,6 @@ struct McLds {
   int moff[kMcPairs + 1];
   uint8_t item_of[kMcSamples / kMcChunkS], pair_of[kMcMid / kMcChunkM];
 };
-
-typedef short mc_s2 __attribute__((ext_vector_type(2)));
-/* n words of sample pairs from any sample's address, one wide load */
-template <int N>
-struct __attribute__((packed, aligned(2))) McWords {
-  uint32_t v[N];
-};
-template <int N>
-__device__ __forceinline__ void load_words(const AV1H_GLOBAL uint16_t* p, uint32_t* s) {
-  const AV1H_GLOBAL McWords<N>* q = (const AV1H_GLOBAL McWords<N>*)p;
-#pragma unroll
-  for (int t = 0; t < N; ++t) s[t] = q->v[t];
-}
-__device__ __forceinline__ int dot2(uint32_t s, int taps, int acc) {
-  return __builtin_amdgcn_sdot2(__builtin_bit_cast(mc_s2, s), __builtin_bit_cast(mc_s2, taps), acc, false);
-}
-/* 8 samples in four words by the 8 taps of a filter row */
-__device__ __forceinline__ int dot8(uint32_t s0, uint32_t s1, uint32_t s2, uint32_t s3, int4 f, int acc) {
-  return dot2(s3, f.w, dot2(s2, f.z, dot2(s1, f.y, dot2(s0, f.x, acc))));
-}
-__device__ __forceinline__ uint32_t pack2(int lo, int hi) { return (uint32_t)(lo & 0xffff) | ((uint32_t)hi << 16); }
 
 __device__ void mc_body(RArgs a, int tn, const int16_t* s_filt, McLds& L_) {
   const int tid = threadIdx.x;
@@ -2217,22 +2320,58 @@ __global__ __launch_bounds__(256, 8) void k_mc(BatchDev B) {
   }
 }
 
-/* Inter blocks with warp, masks or OBMC (they read only references): one
- * workgroup per block, the direct per sample computation. */
+/* Inter blocks with warp, masks or OBMC, and the inter half of inter/intra
+ * blocks (all read only references): the direct per sample computation, a
+ * sample's eight rows loaded together. kSpecialStrips waves share a block: with
+ * one, the launch is as long as the largest block; with 16, most of them find
+ * no sample. 853x479 frame of these tools: 249 us with one load after another
+ * and one wave a block, 117 with 16 waves, 63 with four. */
 __global__ __launch_bounds__(64) void k_inter_special(BatchDev B) {
   const AV1H_CMEM int32_t* pre = kernel_prefix(B, kKSpecial);
   const int total = pre[B.njobs];
   for (int v = blockIdx.x; v < total; v += gridDim.x) {
     const int j = find_job(pre, B.njobs, v);
     RArgs a = recon_args(B, j);
-    const int bi = cmem(a.plan.special_list)[v - pre[j]];
+    const int strip = (v - pre[j]) % kSpecialStrips;
+    const int bi = cmem(a.plan.special_list)[(v - pre[j]) / kSpecialStrips];
     BlkRef b = cmem(a.plan.blocks)[bi];
     const int p = b.plane, stride = a.lay.stride[p], lw = ilog2(b.w);
     uint16_t* dst = a.frame + a.lay.plane_off[p] + (size_t)b.y * stride + b.x;
-    for (int s = threadIdx.x; s < b.w * b.h; s += 64)
-      dst[(size_t)(s >> lw) * stride + (s & (b.w - 1))] = (uint16_t)inter_sample(a, b, s & (b.w - 1), s >> lw);
-    if (a.plan.cell_waits) mark_cells(a, b, false);
+    for (int s = strip * 64 + threadIdx.x; s < b.w * b.h; s += 64 * kSpecialStrips)
+      dst[(size_t)(s >> lw) * stride + (s & (b.w - 1))] = (uint16_t)inter_sample<false>(a, b, s & (b.w - 1), s >> lw);
+    if (strip == 0 && a.plan.cell_waits && !(b.flags & kInterIntra)) mark_cells(a, b, false);
   }
+}
+
+/* Every block the two paths above do not take (CFL, palette, filter intra,
+ * several transforms, inter/intra, intra block copy, edges that need the cell
+ * wait), from its wait to its stores; returns when it was ready. A call of its
+ * own: inlined, its registers (above 256) halved the kernel's waves and its
+ * spills lay in the way of every block (queue of a 1080p key frame 762 -> 992
+ * us). */
+#define AV1H_LDS __attribute__((address_space(3)))
+__device__ __noinline__ uint64_t queue_general(const AV1H_CMEM ReconArgs* args, const AV1H_CMEM DevBlock* block,
+                                               AV1H_LDS int* lds_work, AV1H_LDS uint16_t* lds_pred,
+                                               AV1H_LDS const int* lds_tab, uint32_t* error, bool trace) {
+  /* arguments come in vector registers: these are the same in every lane */
+  RArgs a = *(const AV1H_CMEM ReconArgs*)sreg((int64_t)args);
+  BlkRef b = *(const AV1H_CMEM DevBlock*)sreg((int64_t)block);
+  int* work = (int*)lds_work;
+  uint16_t* pred = (uint16_t*)lds_pred;
+  const int* tab = (const int*)lds_tab;
+  const EarlyRes er = early_residual(a, b, one_transform(a, b));
+  const QBlk q = queued_block(a, b);
+  if (q.flags & kInterDone) ii_ahead(a, b, q, work, pred);
+  if (b.flags & kPackedEdges)
+    gather_edges(a, b, work, error);
+  else
+    wait_cells(a, b, error);
+  const uint64_t ready = trace ? (uint64_t)wall_clock64() : 0;
+  reconstruct_queued(a, b, q, work, pred, er, tab, error);
+  /* the packed edges first: the blocks waiting on this one read only them */
+  if (q.flags & (kEdgeRow | kEdgeCol)) write_edges(q, pred);
+  store_block(q, pred);
+  return ready;
 }
 
 __global__ __launch_bounds__(64) void k_queue(BatchDev B) {
@@ -2293,16 +2432,8 @@ __global__ __launch_bounds__(64) void k_queue(BatchDev B) {
     } else if (big_block(q, b, one)) {
       queue_big(a, b, q, one, s_work, s_tab, B.error, &t1, B.trace != nullptr);
     } else {
-      const EarlyRes er = early_residual(a, b, one);
-      if (b.flags & kPackedEdges)
-        gather_edges(a, b, s_work, B.error);
-      else
-        wait_cells(a, b, B.error);
-      t1 = B.trace ? (uint64_t)wall_clock64() : 0;
-      reconstruct_queued(a, b, q, s_work, s_pred, er, s_tab, B.error);
-      /* the packed edges first: the blocks waiting on this one read only them */
-      if (q.flags & (kEdgeRow | kEdgeCol)) write_edges(q, s_pred);
-      store_block(q, s_pred);
+      t1 = queue_general(&a, &b, (AV1H_LDS int*)s_work, (AV1H_LDS uint16_t*)s_pred, (AV1H_LDS const int*)s_tab, B.error,
+                         B.trace != nullptr);
     }
     if (!(q.flags & kSkipMark)) {
       /* every sample store of the block has completed before its cells flip */

@@ -20,6 +20,9 @@ pytestmark = pytest.mark.gpu
     ("c2_mini", dict(width=131, height=77, coded_width=120, mv_sigma=30.0, bit_depth=12, compound_frac=1.0)),
     ("c2_mini", dict(width=328, height=136, coded_width=246, bit_depth=8, compound_frac=0.0, intra_frac=0.0)),
     ("tools_mini", dict(mv_sigma=300.0)),
+    # every inter tool on odd sizes and at both ends of the depths: inter halves ahead of the queue
+    ("tools_mini", dict(width=333, height=157, inter_tools=0.9, bit_depth=8)),
+    ("tools_mini", dict(width=142, height=230, inter_tools=0.9, bit_depth=12, intrabc=0.5)),
 ])
 @pytest.mark.parametrize("seed", [21, 22])
 def test_motion(workload, over, seed):
