@@ -39,6 +39,7 @@ constexpr int kWork = 2048;            /* int32 intra work area (edges, CFL)    
 
 /* global (not generic) pointers: their accesses need no wait for LDS */
 #define AV1H_GLOBAL __attribute__((address_space(1)))
+#define AV1H_LDS __attribute__((address_space(3)))
 
 __device__ __forceinline__ int clampi(int v, int lo, int hi) { return v < lo ? lo : (v > hi ? hi : v); }
 __device__ __forceinline__ int rnd2(int v, int n) { return n <= 0 ? v : (v + (1 << (n - 1))) >> n; }
@@ -69,229 +70,253 @@ __device__ int wave_sum(int v) {
   return v;
 }
 
+/* n words of 16-bit pairs from any such value's address, one wide load */
+template <int N>
+struct __attribute__((packed, aligned(2))) PairWords {
+  uint32_t v[N];
+};
+template <int N>
+__device__ __forceinline__ void load_words(const AV1H_GLOBAL uint16_t* p, uint32_t* s) {
+  const AV1H_GLOBAL PairWords<N>* q = (const AV1H_GLOBAL PairWords<N>*)p;
+#pragma unroll
+  for (int t = 0; t < N; ++t) s[t] = q->v[t];
+}
 /* ------------------------------------------------------------------------ */
-/* inverse transform of one transform block into the LDS prediction          */
+/* inverse transforms                                                        */
 /* ------------------------------------------------------------------------ */
 
-/* row pass (av1gpu_kernels.h:869-904): lane = row */
+/* where a transform's residual goes: added to the frame within the sample
+ * range (inter blocks, whose prediction is there), or stored as it is */
+struct ItxOut {
+  AV1H_GLOBAL uint16_t* dst; /* the transform's first sample */
+  int stride, lo, hi;
+  bool add;
+};
+
+/* One line of a pass (av1gpu_kernels.h:869-904 the rows, 907-930 the
+ * columns): pass 0 the row `l` of N = w coefficients in place in LDS, pass 1
+ * the column `l` of N = h values out to the picture. Both passes run this one
+ * copy of the N point transform: a launch's time on frames up to 1080p is that
+ * of fetching its instructions once per compute unit, so the second pass
+ * finds them in the instruction cache (with a copy per pass and class, 185 and
+ * 77 KB of code in the two launches, now 61 and 24: 1080p inter frame 27 + 15
+ * -> 14 + 11 us, 2160p 29 + 34 -> 16 + 26, eight streams 20 + 43 -> 12 + 30;
+ * the 24-bit form alone gave 27 -> 24). The addresses run along with the
+ * values (the compiler would hold one per value, 396 registers). */
 template <int N>
-__device__ __forceinline__ void row_pass(int* tmp, int lane, int w, int h, int tx_type, int lossless, int row_shift, int bd,
-                         int rect) {
-  const int y = lane;
-  if (y >= h) return;
-  /* a row holds min(N, 32) coefficients (AV1 codes none beyond 32): the
-   * other inputs are constant zeros, which folds the first stages of the
-   * 64-point transform */
-  constexpr int kCs = N < 32 ? N : 32;
-  const int st = w + 1;
-  const int cr = (1 << (max(bd + 6, 16) - 1));
-  if (y >= 32) {
+__device__ __forceinline__ void itx_line(int pass, int* tmp, int l, int w, int h, int tx_type, int lossless,
+                                         int row_shift, int bd, int rect, const ItxOut& out) {
+  if (l >= (pass ? w : h)) return;
+  /* a line holds min(N, 32) coefficients (AV1 codes none beyond 32; rows
+   * from 32 on are zero after the row pass): the other inputs are constant
+   * zeros, which folds the first stages of the 64-point transform */
+  constexpr int kIn = N < 32 ? N : 32;
+  const int st = w + 1, step = pass ? st : 1;
+  AV1H_LDS int* p = (AV1H_LDS int*)tmp + (pass ? l : l * st);
+  if (!pass && l >= 32) {
 #pragma unroll
-    for (int x = 0; x < N; ++x) tmp[y * st + x] = 0;
+    for (int i = 0; i < N; ++i) p[i] = 0;
     return;
   }
   int t[N];
 #pragma unroll
-  for (int x = 0; x < N; ++x) t[x] = x < kCs ? tmp[y * st + x] : 0;
-  if (rect) {
-#pragma unroll
-    for (int x = 0; x < N; ++x) t[x] = itx::r12((int64_t)t[x] * 2896);
+  for (int i = 0; i < N; ++i) {
+    t[i] = i < kIn ? *p : 0;
+    p += step;
+    /* one running address, not one per value */
+    if (i < kIn) asm volatile("" : "+v"(p));
   }
-  if (lossless) {
-    if constexpr (N == 4) itx::iwht(t, 2);
+  p = (AV1H_LDS int*)tmp + (pass ? l : l * st);
+  const int r = pass ? max(bd + 6, 16) : bd + 8;
+  if (!lossless && itx::all_small<kIn>(t, r)) {
+    if (rect && !pass) {
+#pragma unroll
+      for (int i = 0; i < kIn; ++i) t[i] = (__mul24(t[i], 2896) + 2048) >> 12;
+    }
+    itx::tx1d<true>(t, pass ? itx::col_kind(tx_type) : itx::row_kind(tx_type), 0, 0);
   } else {
-    const int r = bd + 8;
-    itx::tx1d<N>(t, itx::row_kind(tx_type), -(1 << (r - 1)), (1 << (r - 1)) - 1);
-  }
+    if (rect && !pass) {
 #pragma unroll
-  for (int x = 0; x < N; ++x) {
-    const int v = lossless ? t[x] : rnd2(t[x], row_shift);
-    tmp[y * st + x] = clampi(v, -cr, cr - 1);
+      for (int i = 0; i < kIn; ++i) t[i] = itx::r12((int64_t)t[i] * 2896);
+    }
+    if (lossless) {
+      if constexpr (N == 4) itx::iwht(t, pass ? 0 : 2);
+    } else {
+      itx::tx1d<false>(t, pass ? itx::col_kind(tx_type) : itx::row_kind(tx_type), -(1 << (r - 1)), (1 << (r - 1)) - 1);
+    }
   }
-}
-
-/* column pass (av1gpu_kernels.h:907-930): lane = column; hands each residual
- * sample to `out(x, y, value)` */
-template <int M, typename Out>
-__device__ __forceinline__ void col_pass(const int* tmp, int lane, int w, int tx_type, int lossless, int bd, Out&& out) {
-  const int x = lane;
-  if (x >= w) return;
-  const int st = w + 1;
-  int t[M];
-  /* rows from 32 on are zero after the row pass (no coefficients there) */
+  const int shift = lossless ? 0 : (pass ? 4 : row_shift), half = shift > 0 ? 1 << (shift - 1) : 0;
 #pragma unroll
-  for (int i = 0; i < M; ++i) t[i] = i < 32 ? tmp[i * st + x] : 0;
-  if (lossless) {
-    if constexpr (M == 4) itx::iwht(t, 0);
-  } else {
-    const int r = max(bd + 6, 16);
-    itx::tx1d<M>(t, itx::col_kind(tx_type), -(1 << (r - 1)), (1 << (r - 1)) - 1);
+  for (int i = 0; i < N; ++i) t[i] = shift > 0 ? (t[i] + half) >> shift : t[i];
+  if (!pass) {
+    const int cr = 1 << (max(bd + 6, 16) - 1);
+#pragma unroll
+    for (int i = 0; i < N; ++i) p[i] = clampi(t[i], -cr, cr - 1);
+    return;
   }
-  const int ud = itx::flip_ud(tx_type), lr = itx::flip_lr(tx_type);
-  const int xx = lr ? w - 1 - x : x;
-  /* up to 32 rows at a time: their current samples (an inter block's
-   * prediction) are all loaded before any is stored, so the adds do not wait
-   * on one load after another */
-  constexpr int kB = M < 32 ? M : 32;
+  const int ud = itx::flip_ud(tx_type), hop = ud ? -out.stride : out.stride;
+  AV1H_GLOBAL uint16_t* d = out.dst + (itx::flip_lr(tx_type) ? w - 1 - l : l) + (ud ? (N - 1) * out.stride : 0);
+  AV1H_GLOBAL uint16_t* from = d;
+  /* up to 32 rows at a time: their current samples are all loaded before any
+   * is stored, so the adds do not wait on one load after another */
+  constexpr int kB = N < 32 ? N : 32;
 #pragma unroll
-  for (int i0 = 0; i0 < M; i0 += kB) {
+  for (int i0 = 0; i0 < N; i0 += kB) {
     int cur[kB];
 #pragma unroll
-    for (int u = 0; u < kB; ++u) cur[u] = out.load(xx, ud ? M - 1 - (i0 + u) : i0 + u);
+    for (int u = 0; u < kB; ++u) cur[u] = 0;
+    if (out.add) {
+#pragma unroll
+      for (int u = 0; u < kB; ++u) {
+        cur[u] = *from;
+        from += hop;
+        asm volatile("" : "+v"(from));
+      }
+    }
 #pragma unroll
     for (int u = 0; u < kB; ++u) {
-      const int i = i0 + u;
-      out.store(xx, ud ? M - 1 - i : i, cur[u], lossless ? t[i] : rnd2(t[i], 4));
+      *d = (uint16_t)clampi(cur[u] + t[i0 + u], out.lo, out.hi);
+      d += hop;
+      asm volatile("" : "+v"(d));
     }
   }
 }
 
-/* the row / column pass of the size `l2` (log2 points), instantiated only up
- * to the class size G */
+/* the line of the size `l2` (log2 points), instantiated only up to the
+ * launch's largest class G */
 template <int G>
-__device__ __forceinline__ void row_pass_n(int l2, int* tmp, int lane, int w, int h, int tx_type, int lossless, int row_shift,
-                           int bd, int rect) {
+__device__ __forceinline__ void itx_line_n(int l2, int pass, int* tmp, int l, int w, int h, int tx_type, int lossless,
+                                           int row_shift, int bd, int rect, const ItxOut& out) {
   switch (l2) {
-    case 2: row_pass<4>(tmp, lane, w, h, tx_type, lossless, row_shift, bd, rect); break;
-    case 3: if constexpr (G >= 8) row_pass<8>(tmp, lane, w, h, tx_type, lossless, row_shift, bd, rect); break;
-    case 4: if constexpr (G >= 16) row_pass<16>(tmp, lane, w, h, tx_type, lossless, row_shift, bd, rect); break;
-    case 5: if constexpr (G >= 32) row_pass<32>(tmp, lane, w, h, tx_type, lossless, row_shift, bd, rect); break;
-    default: if constexpr (G >= 64) row_pass<64>(tmp, lane, w, h, tx_type, lossless, row_shift, bd, rect); break;
-  }
-}
-template <int G, typename Out>
-__device__ __forceinline__ void col_pass_n(int l2, const int* tmp, int lane, int w, int tx_type, int lossless, int bd, Out&& out) {
-  switch (l2) {
-    case 2: col_pass<4>(tmp, lane, w, tx_type, lossless, bd, out); break;
-    case 3: if constexpr (G >= 8) col_pass<8>(tmp, lane, w, tx_type, lossless, bd, out); break;
-    case 4: if constexpr (G >= 16) col_pass<16>(tmp, lane, w, tx_type, lossless, bd, out); break;
-    case 5: if constexpr (G >= 32) col_pass<32>(tmp, lane, w, tx_type, lossless, bd, out); break;
-    default: if constexpr (G >= 64) col_pass<64>(tmp, lane, w, tx_type, lossless, bd, out); break;
+    case 2: itx_line<4>(pass, tmp, l, w, h, tx_type, lossless, row_shift, bd, rect, out); break;
+    case 3: if constexpr (G >= 8) itx_line<8>(pass, tmp, l, w, h, tx_type, lossless, row_shift, bd, rect, out); break;
+    case 4: if constexpr (G >= 16) itx_line<16>(pass, tmp, l, w, h, tx_type, lossless, row_shift, bd, rect, out); break;
+    case 5: if constexpr (G >= 32) itx_line<32>(pass, tmp, l, w, h, tx_type, lossless, row_shift, bd, rect, out); break;
+    default: if constexpr (G >= 64) itx_line<64>(pass, tmp, l, w, h, tx_type, lossless, row_shift, bd, rect, out); break;
   }
 }
 
-/* The transform blocks of class G (larger side G): G lanes per transform,
- * 64 / G transforms per wave, coefficients staged in LDS between the row and
- * the column pass. The residual of an inter block is added into the frame
- * (its prediction is already there); that of an intra block goes to `res`,
- * where the dependency queue adds it after the prediction. */
+/* The transform blocks of one class (larger side 1 << lg, at most G): 1 << lg
+ * lanes per transform, 64 >> lg transforms per wave, coefficients staged in LDS
+ * between the row and the column pass. The residual of an inter block is added
+ * into the frame (its prediction is already there); that of an intra block goes
+ * to `res`, where the dependency queue adds it after the prediction. The lanes
+ * per transform are a variable so that the classes of a launch share the code
+ * of each size. */
 template <int G>
-__device__ __forceinline__ void itx_group(RArgs a, const int32_t* list, int n, int wg, int* s_tmp) {
-  constexpr int kPer = 64 / G;
-  const int grp = threadIdx.x / G, l = threadIdx.x - grp * G;
-  const int idx = wg * kPer + grp;
+__device__ __forceinline__ void itx_group(RArgs a, const int32_t* list, int n, int wg, int lg, int* s_tmp) {
+  const int lanes = 1 << lg;
+  const int grp = threadIdx.x >> lg, l = threadIdx.x & (lanes - 1);
+  const int idx = wg * (64 >> lg) + grp;
   const bool live = idx < n;
+  const int ti = live ? list[idx] : 0;
   DevTx tx;
   if (live) {
-    tx = a.plan.tx[list[idx]];
+    tx = a.plan.tx[ti];
   } else {
     tx.w = tx.h = 4;
     tx.flags = kTxRaw;
     tx.plane = 0;
     tx.x = tx.y = tx.coef = tx.tx_type = tx.row_shift = tx.eob = 0;
   }
-  int* tmp = s_tmp + grp * G * (G + 1);
-  const int w = tx.w, h = tx.h;
-  const int stride = plane_vals(a.lay.stride)[tx.plane];
-  const int64_t poff = plane_vals(a.lay.plane_off)[tx.plane];
-  const int64_t off = poff + (int64_t)tx.y * stride + tx.x;
+  int* tmp = s_tmp + grp * lanes * (lanes + 1);
+  const int w = tx.w, h = tx.h, lw = ilog2(w), lh = ilog2(h);
   const bool to_res = (tx.flags & kTxToResidual) != 0;
-  const int maxv = a.maxv;
-  struct {
-    RArgs a;
-    int64_t off;
-    int stride, maxv;
-    bool to_res;
-    __device__ __forceinline__ int load(int xx, int yy) const {
-      return to_res ? 0 : (int)a.frame[off + (int64_t)yy * stride + xx];
-    }
-    __device__ __forceinline__ void store(int xx, int yy, int cur, int v) const {
-      const int64_t o = off + (int64_t)yy * stride + xx;
-      if (to_res)
-        a.res[o] = (int16_t)clampi(v, -32768, 32767);
-      else
-        a.frame[o] = (uint16_t)clampi(cur + v, 0, maxv);
-    }
-  } out{a, off, stride, maxv, to_res};
+  ItxOut out;
+  out.stride = plane_vals(a.lay.stride)[tx.plane];
+  out.dst = (to_res ? (AV1H_GLOBAL uint16_t*)a.res : (AV1H_GLOBAL uint16_t*)a.frame) +
+            plane_vals(a.lay.plane_off)[tx.plane] + (int64_t)tx.y * out.stride + tx.x;
+  out.lo = to_res ? -32768 : 0;
+  out.hi = to_res ? 32767 : a.maxv;
+  out.add = !to_res;
   const bool coded = live && !(tx.flags & kTxRaw);
-  const int lw = ilog2(w), lh = ilog2(h);
   if (live && !coded) {
     /* raw residual (av1gpu_kernels.h:933-937), eight samples per lane at a
      * time: residuals and current samples loaded before any store */
     const int n = w * h;
-    for (int i0 = l; i0 < n; i0 += 8 * G) {
+    for (int i0 = l; i0 < n; i0 += 8 * lanes) {
       int r[8], cur[8];
 #pragma unroll
       for (int u = 0; u < 8; ++u) {
-        const int i = i0 + u * G;
+        const int i = i0 + u * lanes;
         r[u] = i < n ? a.plan.residual[tx.coef + i] : 0;
-        cur[u] = i < n ? out.load(i & (w - 1), i >> lw) : 0;
+        cur[u] = i < n && out.add ? (int)out.dst[(i >> lw) * out.stride + (i & (w - 1))] : 0;
       }
 #pragma unroll
       for (int u = 0; u < 8; ++u) {
-        const int i = i0 + u * G;
-        if (i < n) out.store(i & (w - 1), i >> lw, cur[u], r[u]);
+        const int i = i0 + u * lanes;
+        if (i < n) out.dst[(i >> lw) * out.stride + (i & (w - 1))] = (uint16_t)clampi(cur[u] + r[u], out.lo, out.hi);
       }
     }
   }
   if (coded) {
-    /* every coefficient a lane stages is loaded before the first LDS write:
-     * one memory round trip instead of one per coefficient row */
-    constexpr int kC = G < 32 ? G : 32, kIt = kC * kC / G;
-    const int cs = w < 32 ? w : 32, cr = h < 32 ? h : 32;
-    const int lcs = ilog2(cs), st = w + 1, n = cs * cr;
-    int v[kIt];
+    /* the coefficients, eight neighbours (of one row, or of two rows of
+     * four) per lane and step */
+    const int cs = min(w, 32), cr = min(h, 32);
+    const int lcs = ilog2(cs), st = w + 1, n = cs * cr, second = cs == 4 ? st - 4 : 0;
+    auto put = [&](int i0, const int* v) {
+      int* p = tmp + (i0 >> lcs) * st + (i0 & (cs - 1));
+#pragma unroll
+      for (int u = 0; u < 8; ++u) p[u + (u >= 4 ? second : 0)] = v[u];
+    };
     if (a.plan.levels) {
       /* dequantised here from the coded levels: raster position i holds
        * scan index si, coded when below the transform's count */
-      const DevDq q = a.plan.dq[list[idx]];
+      const DevDq q = a.plan.dq[ti];
       const int cls = av1scan::tx_class(tx.tx_type), lcw = lcs - 2, lch = ilog2(cr) - 2;
       const int count = tx.eob < n ? tx.eob : n;
       const int16_t* lv = a.plan.levels + q.level_off;
-      int si[kIt];
+      for (int i0 = 8 * l; i0 < n; i0 += 8 * lanes) {
+        int si[8], v[8];
 #pragma unroll
-      for (int k = 0; k < kIt; ++k) {
-        const int i = l + k * G;
-        si[k] = i < n ? av1scan::scan_index(kScanTab.iscan, cls, lcw, lch, i) : n;
-      }
+        for (int u = 0; u < 8; ++u) si[u] = av1scan::scan_index(kScanTab.iscan, cls, lcw, lch, i0 + u);
 #pragma unroll
-      for (int k = 0; k < kIt; ++k) v[k] = si[k] < count ? (int)lv[si[k]] : 0;
-      if (q.qm_off >= 0) {
-        const uint8_t* qm = a.plan.qm + q.qm_off;
+        for (int u = 0; u < 8; ++u) v[u] = si[u] < count ? (int)lv[si[u]] : 0;
 #pragma unroll
-        for (int k = 0; k < kIt; ++k) {
-          const int i = l + k * G;
-          if (v[k]) v[k] = av1scan::dequant(v[k], i ? q.ac_step : q.dc_step, qm[i], q.denom_shift, a.lay.bit_depth);
+        for (int u = 0; u < 8; ++u) {
+          const int i = i0 + u;
+          if (v[u])
+            v[u] = av1scan::dequant(v[u], i ? q.ac_step : q.dc_step, q.qm_off >= 0 ? (int)a.plan.qm[q.qm_off + i] : -1,
+                                    q.denom_shift, a.lay.bit_depth);
         }
-      } else {
-#pragma unroll
-        for (int k = 0; k < kIt; ++k) {
-          const int i = l + k * G;
-          if (v[k]) v[k] = av1scan::dequant(v[k], i ? q.ac_step : q.dc_step, -1, q.denom_shift, a.lay.bit_depth);
-        }
+        put(i0, v);
       }
     } else if (a.plan.coef16) {
-      const int16_t* src = static_cast<const int16_t*>(a.plan.coef) + tx.coef;
+      /* every coefficient a lane stages is loaded before the first LDS write */
+      constexpr int kSteps = G < 32 ? 2 : 4;
+      const AV1H_GLOBAL uint16_t* src = (const AV1H_GLOBAL uint16_t*)a.plan.coef + tx.coef;
+      uint32_t c[kSteps][4];
 #pragma unroll
-      for (int k = 0; k < kIt; ++k) v[k] = l + k * G < n ? (int)src[l + k * G] : 0;
+      for (int k = 0; k < kSteps; ++k)
+        if (8 * (l + k * lanes) < n) load_words<4>(src + 8 * (l + k * lanes), c[k]);
+#pragma unroll
+      for (int k = 0; k < kSteps; ++k) {
+        if (8 * (l + k * lanes) >= n) break;
+        int v[8];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          v[2 * u] = (int)(int16_t)c[k][u];
+          v[2 * u + 1] = (int)c[k][u] >> 16;
+        }
+        put(8 * (l + k * lanes), v);
+      }
     } else {
       const int32_t* src = static_cast<const int32_t*>(a.plan.coef) + tx.coef;
+      for (int i0 = 8 * l; i0 < n; i0 += 8 * lanes) {
+        int v[8];
 #pragma unroll
-      for (int k = 0; k < kIt; ++k) v[k] = l + k * G < n ? src[l + k * G] : 0;
-    }
-#pragma unroll
-    for (int k = 0; k < kIt; ++k) {
-      const int i = l + k * G;
-      if (i < n) tmp[(i >> lcs) * st + (i & (cs - 1))] = v[k];
+        for (int u = 0; u < 8; ++u) v[u] = src[i0 + u];
+        put(i0, v);
+      }
     }
   }
-  __syncthreads();
-  const int lossless = (tx.flags & kTxLossless) ? 1 : 0;
-  if (coded)
-    row_pass_n<G>(lw, tmp, l, w, h, tx.tx_type, lossless, tx.row_shift, a.lay.bit_depth,
-                  (lw - lh == 1 || lh - lw == 1) ? 1 : 0);
-  __syncthreads();
-  if (coded) col_pass_n<G>(lh, tmp, l, w, tx.tx_type, lossless, a.lay.bit_depth, out);
+  const int lossless = (tx.flags & kTxLossless) ? 1 : 0, rect = (lw - lh == 1 || lh - lw == 1) ? 1 : 0;
+#pragma unroll 1
+  for (int pass = 0; pass < 2; ++pass) {
+    __syncthreads();
+    if (coded)
+      itx_line_n<G>(pass ? lh : lw, pass, tmp, l, w, h, tx.tx_type, lossless, tx.row_shift, a.lay.bit_depth, rect, out);
+  }
 }
 
 /* The classes [C0, C1) of a set in one launch, the larger first: two
@@ -299,20 +324,13 @@ __device__ __forceinline__ void itx_group(RArgs a, const int32_t* list, int n, i
  * with the registers and LDS they need rather than the 64-point ones'. */
 template <int C0, int C1>
 __device__ __forceinline__ void itx_body(RArgs a, const int32_t* offs, int b, int* s_tmp) {
-#pragma unroll
   for (int c = C1 - 1; c >= C0; --c) {
     const int o0 = offs[c], n = offs[c + 1] - o0;
     const int per = 16 >> c;
     const int wgs = (n + per - 1) / per;
     if (b < wgs) {
       const int32_t* list = a.plan.itx_list + o0;
-      switch (c) {
-        case 0: itx_group<4>(a, list, n, b, s_tmp); break;
-        case 1: itx_group<8>(a, list, n, b, s_tmp); break;
-        case 2: itx_group<16>(a, list, n, b, s_tmp); break;
-        case 3: itx_group<32>(a, list, n, b, s_tmp); break;
-        default: itx_group<64>(a, list, n, b, s_tmp); break;
-      }
+      itx_group<(4 << (C1 - 1))>(a, list, n, b, c + 2, s_tmp);
       return;
     }
     b -= wgs;
@@ -320,10 +338,8 @@ __device__ __forceinline__ void itx_body(RArgs a, const int32_t* offs, int b, in
 }
 
 /* Both sets of every frame, the inter blocks' first: the intra blocks'
- * residuals are independent of the prediction, and one launch of both is as
- * long as one of either on all but the largest frames (a wave's transform is
- * latency: 1080p inter frame, 32- and 64-point classes, 24 + 27 us in two
- * launches). */
+ * residuals are independent of the prediction, and one launch of both is
+ * hardly longer than one of either (itx_line). */
 template <int C0, int C1>
 __global__ __launch_bounds__(64) void k_itx(BatchDev B) {
   constexpr int kG = 4 << (C1 - 1);
@@ -416,17 +432,6 @@ __device__ const uint16_t* ref_plane(RArgs a, int slot, int plane) {
 /* ------------------------------------------------------------------------ */
 
 typedef short mc_s2 __attribute__((ext_vector_type(2)));
-/* n words of sample pairs from any sample's address, one wide load */
-template <int N>
-struct __attribute__((packed, aligned(2))) McWords {
-  uint32_t v[N];
-};
-template <int N>
-__device__ __forceinline__ void load_words(const AV1H_GLOBAL uint16_t* p, uint32_t* s) {
-  const AV1H_GLOBAL McWords<N>* q = (const AV1H_GLOBAL McWords<N>*)p;
-#pragma unroll
-  for (int t = 0; t < N; ++t) s[t] = q->v[t];
-}
 __device__ __forceinline__ int dot2(uint32_t s, int taps, int acc) {
   return __builtin_amdgcn_sdot2(__builtin_bit_cast(mc_s2, s), __builtin_bit_cast(mc_s2, taps), acc, false);
 }
@@ -2349,7 +2354,6 @@ __global__ __launch_bounds__(64) void k_inter_special(BatchDev B) {
  * own: inlined, its registers (above 256) halved the kernel's waves and its
  * spills lay in the way of every block (queue of a 1080p key frame 762 -> 992
  * us). */
-#define AV1H_LDS __attribute__((address_space(3)))
 __device__ __noinline__ uint64_t queue_general(const AV1H_CMEM ReconArgs* args, const AV1H_CMEM DevBlock* block,
                                                AV1H_LDS int* lds_work, AV1H_LDS uint16_t* lds_pred,
                                                AV1H_LDS const int* lds_tab, uint32_t* error, bool trace) {
