@@ -2035,7 +2035,7 @@ int kernel_groups(const FrameJob& fj, int k, int cdef_batch) {
     }
     case kKUpscale: return f.upscaled ? upscale_tiles(L, f.uses_lr ? 2 : 1) : 0;
     case kKLr: return f.uses_lr ? p.n_lr_tiles : 0;
-    case kKGrainTemplate: return f.has_grain ? 1 : 0;
+    case kKGrainTemplate: return f.has_grain ? 2 : 0; /* two halves */
     case kKGrainApply: return f.has_grain ? grain_tiles(L) : 0;
     case kKNv12: return f.nv12 ? (L.height + ((L.height + 1) >> 1)) * ((f.nv12_pitch + 1023) / 1024) : 0;
     case kKHash: {
@@ -2265,7 +2265,6 @@ int batch_launch(Ctx* lead, std::vector<JobSpec>& js, double t0) {
   B.queue_counter = lead->counters + kTicketStep;
   B.error = lead->counters + 1;
   B.trace = nullptr;
-  grain_jump_matrices(B.jump82, B.jump44);
   if (lead->trace_on && nq > 0) {
     const size_t need = (size_t)nq * 4;
     if (lead->trace_cap < need) {

@@ -2,13 +2,10 @@
  * Film grain synthesis (specification 7.18.3) on gfx950.
  *
  * The reference synthesises the grain on the host every frame and uploads a
- * full-frame noise image (src/core/grain.cpp:70-139, 6.2 MB at 1080p). Here:
- *   k_grain_template - one workgroup builds the three grain templates
- *     (82x73 luma, 44x38 chroma at 4:2:0): the Gaussian white noise with the
- *     16 bit LFSR jumped ahead per row (so every row starts in parallel), then
- *     the auto-regressive filter as a wavefront over rows (a row lags its
- *     predecessor by four columns, which is all the lag-3 filter reads), and
- *     the per stripe block offsets;
+ * full-frame noise image (src/core/grain.cpp:70-139, 6.2 MB at 1080p). Here the
+ * three grain templates (82x73 luma, 44x38 chroma at 4:2:0) and the per stripe
+ * block offsets are built on a second stream (k_grain_template,
+ * av1hip_grain_template.hpp), and
  *   k_grain_apply - the noise sample of every picture sample is derived on
  *     the fly from the templates (the block and stripe overlap blends of
  *     av1gpu_kernels.h:3218-3291 evaluated per sample) and blended in, chroma
@@ -16,7 +13,7 @@
  * The arithmetic is the reference's (av1gpu_kernels.h:3039-3365).
  */
 #define AV1T_TABLE_QUAL static __constant__ const
-#include "av1hip_internal.hpp"
+#include "av1hip_grain_template.hpp"
 #include "spec_tables.h"
 
 namespace av1hip {
@@ -29,177 +26,14 @@ constexpr int kLW = 82, kLH = 73;
 __device__ __forceinline__ int clampi(int v, int lo, int hi) { return v < lo ? lo : (v > hi ? hi : v); }
 __device__ __forceinline__ int grnd(int v, int n) { return n <= 0 ? v : (v + (1 << (n - 1))) >> n; }
 
-__device__ __forceinline__ unsigned lfsr_step(unsigned r) {
-  const unsigned bit = (r ^ (r >> 1) ^ (r >> 3) ^ (r >> 12)) & 1u;
-  return (r >> 1) | (bit << 15);
-}
-/* apply a 16x16 GF(2) matrix given by its columns */
-__device__ __forceinline__ unsigned mat_apply(const uint16_t* cols, unsigned v) {
-  unsigned r = 0;
-  for (int j = 0; j < 16; ++j)
-    if (v & (1u << j)) r ^= cols[j];
-  return r;
-}
-
-/* white noise row `y` of a w wide template (av1gpu_kernels.h:3070-3079),
- * the Gaussian sequence `gs` staged in LDS */
-__device__ void noise_row(int16_t* t, int w, int y, unsigned seed, const uint16_t* jump, int shift,
-                          const int16_t* gs) {
-  unsigned st = seed;
-  for (int k = 0; k < y; ++k) st = mat_apply(jump, st);
-  for (int x = 0; x < w; ++x) {
-    st = lfsr_step(st);
-    t[y * w + x] = (int16_t)grnd(gs[(st >> 5) & 2047], shift);
-  }
-}
-
-/* LDS accesses of one wave complete in issue order; this keeps the compiler
- * from moving a later read above an earlier write and waits for the writes. */
-__device__ __forceinline__ void wave_lds_sync() { __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
-
-/* The auto-regressive filter of one template (av1gpu_kernels.h:3087-3122) run
- * by ONE wave as a wavefront: lane l filters row 3 + l (and row 67 + l when the
- * template is taller than 67 rows) and lags the lane above by four columns,
- * which is exactly the lag-3 filter's reach into the previous row, so no two
- * waves ever synchronise. The coefficients stay in registers. */
-template <int LAG>
-__device__ __forceinline__ void ar_plane(int16_t* pl, int w, int h, const int* coeffs, const int16_t* luma, int ss_x, int ss_y,
-                         int shift, int lo, int hi) {
-  constexpr int kTaps = (2 * LAG + 1) * LAG + LAG;
-  int c[kTaps + 1];
-#pragma unroll
-  for (int i = 0; i < kTaps; ++i) c[i] = coeffs[i];
-  c[kTaps] = luma ? coeffs[kTaps] : 0; /* chroma only: the luma tap */
-  const int lane = threadIdx.x & 63;
-  const int rows = h - 3, cols = w - 6;
-  const int steps = (cols - 1) + 4 * (rows - 1) + 1;
-  for (int s = 0; s < steps; ++s) {
-#pragma unroll
-    for (int p = 0; p < 2; ++p) {
-      const int r = lane + 64 * p;
-      const int x = s - 4 * r + 3, y = 3 + r;
-      if (r < rows && x >= 3 && x < w - 3) {
-        int sum = 0, pos = 0;
-#pragma unroll
-        for (int dr = -LAG; dr <= 0; ++dr)
-#pragma unroll
-          for (int dc = -LAG; dc <= LAG; ++dc) {
-            if (dr == 0 && dc >= 0) break;
-            sum += __mul24(pl[(y + dr) * w + x + dc], c[pos]); /* 16 x 8 bit */
-            ++pos;
-          }
-        if (luma) {
-          const int lx = ((x - 3) << ss_x) + 3, ly = ((y - 3) << ss_y) + 3;
-          int acc = 0;
-          for (int i = 0; i <= ss_y; ++i)
-            for (int k = 0; k <= ss_x; ++k) acc += luma[(ly + i) * kLW + lx + k];
-          sum += __mul24(grnd(acc, ss_x + ss_y), c[kTaps]);
-        }
-        pl[y * w + x] = (int16_t)clampi(pl[y * w + x] + grnd(sum, shift), lo, hi);
-      }
-    }
-    wave_lds_sync();
-  }
-}
-
-/* inlined into its callers so that the template pointers stay LDS accesses */
-__device__ __forceinline__ void ar_dispatch(int lag, int16_t* pl, int w, int h, const int* coeffs, const int16_t* luma, int ss_x,
-                            int ss_y, int shift, int lo, int hi) {
-  switch (lag) {
-    case 0: ar_plane<0>(pl, w, h, coeffs, luma, ss_x, ss_y, shift, lo, hi); break;
-    case 1: ar_plane<1>(pl, w, h, coeffs, luma, ss_x, ss_y, shift, lo, hi); break;
-    case 2: ar_plane<2>(pl, w, h, coeffs, luma, ss_x, ss_y, shift, lo, hi); break;
-    default: ar_plane<3>(pl, w, h, coeffs, luma, ss_x, ss_y, shift, lo, hi); break;
-  }
-}
-
-constexpr int kTmplThreads = 192; /* three waves: luma, cb, cr */
-
-/* Templates and block offsets. `tmpl` receives luma (82x73) then cb and cr
- * (cw x ch each); `offs` the 8 bit offset draw of every (stripe, block).
- * Phases: white noise (one row per thread); luma filter on wave 0 while
- * waves 1-2 draw the offsets; cb on wave 1 and cr on wave 2 (both read the
- * finished luma template) while wave 0 stores luma. */
-__device__ void grain_template(const DevGrain& g, const uint16_t* jm82, const uint16_t* jm44, int ss_x, int ss_y,
-                               int16_t* tmpl, uint8_t* offs, int16_t* s_l, int16_t (*s_c)[kLW * kLH],
-                               const int16_t* s_gauss) {
-  const int tid = threadIdx.x, wave = tid >> 6;
-  const int bd = g.bit_depth;
-  const int lo = -(128 << (bd - 8)), hi = (256 << (bd - 8)) - 1 - (128 << (bd - 8));
-  const int cw = ss_x ? 44 : kLW, ch = ss_y ? 38 : kLH;
-  const int chroma = g.cfl || g.num_cb > 0 || g.num_cr > 0;
-  const unsigned seed = (unsigned)g.seed;
-  /* white noise (av1gpu_kernels.h:3070-3079), one row per thread */
-  const uint16_t* jc = ss_x ? jm44 : jm82;
-  for (int r = tid; r < kLH + 2 * ch; r += kTmplThreads) {
-    if (r < kLH) {
-      if (g.num_y > 0)
-        noise_row(s_l, kLW, r, seed, jm82, g.scale_shift, s_gauss);
-      else
-        for (int x = 0; x < kLW; ++x) s_l[r * kLW + x] = 0;
-    } else if (chroma) {
-      const int pl = (r - kLH) / ch, y = (r - kLH) - pl * ch;
-      if (pl == 0 ? (g.num_cb > 0 || g.cfl) : (g.num_cr > 0 || g.cfl))
-        noise_row(s_c[pl], cw, y, seed ^ (pl == 0 ? 0xb524u : 0x49d8u), jc, g.scale_shift, s_gauss);
-      else
-        for (int x = 0; x < cw; ++x) s_c[pl][y * cw + x] = 0;
-    }
-  }
-  __syncthreads();
-  if (wave == 0) {
-    if (g.num_y > 0) ar_dispatch(g.lag, s_l, kLW, kLH, g.ar_y, nullptr, 0, 0, g.shift, lo, hi);
-  } else {
-    /* per stripe block offsets (av1gpu_kernels.h:3236-3247) */
-    for (int st = tid - 64; st < g.stripes; st += kTmplThreads - 64) {
-      unsigned r = seed;
-      r ^= (unsigned)(((st * 37 + 178) & 255) << 8);
-      r ^= (unsigned)((st * 173 + 105) & 255);
-      for (int b = 0; b < g.blocks; ++b) {
-        r = lfsr_step(r);
-        offs[st * g.blocks + b] = (uint8_t)((r >> 8) & 255);
-      }
-    }
-  }
-  __syncthreads();
-  if (wave == 0) {
-    for (int i = tid; i < kLW * kLH; i += 64) tmpl[i] = s_l[i];
-  } else if (chroma) {
-    const int pl = wave - 1;
-    ar_dispatch(g.lag, s_c[pl], cw, ch, pl ? g.ar_cr : g.ar_cb, g.num_y > 0 ? s_l : nullptr, ss_x, ss_y, g.shift,
-                lo, hi);
-    for (int i = tid & 63; i < cw * ch; i += 64) tmpl[kLW * kLH + pl * cw * ch + i] = s_c[pl][i];
-  }
-}
-
-/* one workgroup per frame with film grain */
-__global__ __launch_bounds__(kTmplThreads) void k_grain_template(BatchDev B) {
-  __shared__ int16_t s_l[kLW * kLH];
-  __shared__ int16_t s_c[2][kLW * kLH];
-  __shared__ int16_t s_gauss[2048];
-  {
-    /* the Gaussian sequence (12 bit values), every load issued before the
-     * LDS writes */
-    constexpr int kPer = (2048 + kTmplThreads - 1) / kTmplThreads;
-    const int* gs = SPEC(AV1T_OFF_GAUSSIAN);
-    int v[kPer];
-#pragma unroll
-    for (int u = 0; u < kPer; ++u) {
-      const int i = threadIdx.x + kTmplThreads * u;
-      v[u] = i < 2048 ? gs[i] : 0;
-    }
-#pragma unroll
-    for (int u = 0; u < kPer; ++u) {
-      const int i = threadIdx.x + kTmplThreads * u;
-      if (i < 2048) s_gauss[i] = (int16_t)v[u];
-    }
-  }
-  __syncthreads();
+/* two workgroups (of one wave) per frame with film grain, a half each */
+__global__ __launch_bounds__(64) void k_grain_template(BatchDev B) {
+  __shared__ __align__(16) uint8_t s_lds[grain::kTemplateLds];
   const AV1H_CMEM int32_t* pre = kernel_prefix(B, kKGrainTemplate);
   const int total = pre[B.njobs];
   for (int v = blockIdx.x; v < total; v += gridDim.x) {
-    FArgs a = filter_args(B, find_job(pre, B.njobs, v));
-    grain_template(*a.plan.grain, B.jump82, B.jump44, a.lay.ss_x, a.lay.ss_y, a.grain_tmpl, a.grain_offs, s_l, s_c,
-                   s_gauss);
+    const int j = find_job(pre, B.njobs, v);
+    grain::template_half(filter_args(B, j), v - pre[j], s_lds);
     __syncthreads();
   }
 }
@@ -360,29 +194,14 @@ __global__ __launch_bounds__(256) void k_grain_apply(BatchDev B) {
   }
 }
 
-unsigned host_step(unsigned r) {
-  const unsigned bit = (r ^ (r >> 1) ^ (r >> 3) ^ (r >> 12)) & 1u;
-  return (r >> 1) | (bit << 15);
-}
-
 }  // namespace
-
-void grain_jump_matrices(uint16_t m82[16], uint16_t m44[16]) {
-  for (int j = 0; j < 16; ++j) {
-    unsigned a = 1u << j, b = 1u << j;
-    for (int k = 0; k < 82; ++k) a = host_step(a);
-    for (int k = 0; k < 44; ++k) b = host_step(b);
-    m82[j] = (uint16_t)a;
-    m44[j] = (uint16_t)b;
-  }
-}
 
 int grain_tiles(const Layout& lay) { return (lay.out_w[0] + 63) / 64 * ((lay.out_h[0] + 31) / 32); }
 
 hipError_t launch_grain_kernel(const BatchDev& b, int k, int total, int cap, hipStream_t s) {
   const dim3 grid(min(total, cap));
   switch (k) {
-    case kKGrainTemplate: hipLaunchKernelGGL(k_grain_template, grid, dim3(kTmplThreads), 0, s, b); break;
+    case kKGrainTemplate: hipLaunchKernelGGL(k_grain_template, grid, dim3(64), 0, s, b); break;
     case kKGrainApply: hipLaunchKernelGGL(k_grain_apply, grid, dim3(256), 0, s, b); break;
     default: return hipErrorInvalidValue;
   }

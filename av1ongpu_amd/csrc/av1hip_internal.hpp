@@ -402,7 +402,6 @@ struct BatchDev {
   uint32_t* queue_counter;
   uint32_t* error;           /* bit 0: a dependency wait timed out   */
   uint64_t* trace;           /* null, or 4 timestamps per queue entry */
-  uint16_t jump82[16], jump44[16]; /* grain LFSR jump matrices        */
 };
 
 typedef const AV1H_CMEM ReconArgs& RArgs;
@@ -480,9 +479,6 @@ hipError_t launch_rgb(const Layout& lay, const uint16_t* src, uint8_t* out, cons
 /* transform workgroups of classes [c0, c1) of one set of a frame (0 inter,
  * 1 intra) */
 int itx_groups(const FramePlanDev& p, int set, int c0, int c1);
-
-/* film grain: the LFSR jump matrices the template kernel uses */
-void grain_jump_matrices(uint16_t m82[16], uint16_t m44[16]);
 
 }  // namespace av1hip
 
