@@ -598,200 +598,325 @@ __global__ __launch_bounds__(256) void k_upscale(BatchDev B) {
 
 /* ---- loop restoration (av1gpu_kernels.h:2832-2982) ---------------------- */
 
-/* Row / column of element i of a w-wide 2D range walked by 256 threads
- * (i = threadIdx.x, then + 256 each step), without a division per step. */
-struct Walk256 {
-  int r, q, dr, dq, w;
-  __device__ __forceinline__ explicit Walk256(int width) : w(width) {
-    r = (int)threadIdx.x / w;
-    q = (int)threadIdx.x - r * w;
-    dr = 256 / w;
-    dq = 256 - dr * w;
-  }
-  __device__ __forceinline__ void next() {
-    q += dq;
-    r += dr;
-    if (q >= w) {
-      q -= w;
-      ++r;
-    }
-  }
-};
-
 /* a2 of the self-guided filter for z = 0 .. 255 (the specification's
  * x_by_xplus1 mapping, av1gpu_kernels.h:2898): z >= 255 gives 256 */
 __device__ __forceinline__ int sgr_a2(int z) { return z == 0 ? 1 : ((z << 8) + z / 2) / (z + 1); }
 
-struct LrCtx {
-  const uint16_t* cdef;
-  const uint16_t* curr;
-  int stride, pw, ph, s0, s1;
-  __device__ __forceinline__ int src(int x, int y) const {
-    x = clampi(x, 0, pw - 1);
-    y = clampi(y, 0, ph - 1);
-    if (y < s0) return curr[(size_t)max(y, s0 - 2) * stride + x];
-    if (y > s1) return curr[(size_t)min(y, s1 + 2) * stride + x];
-    return cdef[(size_t)y * stride + x];
-  }
+typedef short lr_s2 __attribute__((ext_vector_type(2)));
+/* two 16-bit products added to acc */
+__device__ __forceinline__ int dot2(uint32_t a, uint32_t b, int acc) {
+  return __builtin_amdgcn_sdot2(__builtin_bit_cast(lr_s2, a), __builtin_bit_cast(lr_s2, b), acc, false);
+}
+__device__ __forceinline__ uint32_t pack2(int lo, int hi) { return (uint32_t)(lo & 0xffff) | ((uint32_t)hi << 16); }
+
+/* Loop restoration of one tile (at most kLrTileCols x kLrTileRows samples of
+ * one restoration job, i.e. one unit inside one 64 row stripe) per workgroup,
+ * four neighbouring samples per lane:
+ *   the source window with its halo is staged in LDS as 16-bit samples,
+ *   through the stripe rule (rows above / below the stripe from the deblocked
+ *   picture, at most two away), eight bytes a load inside the picture;
+ *   Wiener - the horizontal 7 tap pass into a 16-bit LDS intermediate (rounded
+ *            and clamped to 15 bits and a sign), then the vertical pass
+ *            (av1gpu_kernels.h:2832-2870), taps two at a time;
+ *   SGR    - a lane walks a column of six positions down with its 5 and 3 wide
+ *            row sums in registers; A and B of both passes, packed in a word
+ *            (A at most 256; B at most 255 * 25 * 4095 * 164 >> 12 < 2^20), at
+ *            every position the 3x3 neighbourhoods of the tile touch, pass 0
+ *            only on the odd rows it weighs; then the weighted neighbourhood
+ *            sums and the projection (av1gpu_kernels.h:2872-2982).
+ * Bound by instructions: one sample per lane with 32-bit LDS samples and
+ * multiplies took 37 us on a 1080p frame, 133 on a 2160p one, 50 on eight
+ * streams (Wiener); now 19, 61 and 38, with a 64 x 16 tile in 13.6 KB. */
+constexpr int kLrW = kLrTileCols, kLrH = kLrTileRows;
+constexpr int kLrSrcLd = kLrW + 12, kLrSrcRows = kLrH + 6; /* from 4 left, 3 above */
+constexpr int kLrMidLd = kLrW + 4, kLrAbLd = kLrW + 4, kLrAbRows = kLrH + 2;
+
+struct LrLds {
+  __align__(16) uint16_t src[kLrSrcRows * kLrSrcLd];
+  union {
+    __align__(16) int16_t mid[kLrSrcRows * kLrMidLd]; /* Wiener */
+    __align__(16) uint32_t ab[2][kLrAbRows * kLrAbLd]; /* SGR, B << 9 | A */
+  };
+  uint16_t a2[256];
 };
 
-/* Loop restoration of one tile (at most kLrTileW x kLrTileH samples of one
- * restoration job, i.e. one unit inside one 64 row stripe) per workgroup:
- * the source window with its 3 sample halo is staged in LDS through the
- * stripe rule (LrCtx::src), then
- *   Wiener - the horizontal 7 tap pass into an LDS intermediate, rounded and
- *            clamped, then the vertical pass (av1gpu_kernels.h:2832-2870);
- *   SGR    - the box sums, A and B of both passes at every position the 3x3
- *            neighbourhoods of the tile touch, into LDS, then the weighted
- *            neighbourhood sums and the projection (av1gpu_kernels.h:2872-2982).
- * Each intermediate is computed once instead of once per output sample. */
-constexpr int kLrTileW = kLrTileCols, kLrTileH = kLrTileRows;
-constexpr int kLrSrcW = kLrTileW + 6, kLrSrcH = kLrTileH + 6;
-constexpr int kLrAbW = kLrTileW + 2, kLrAbH = kLrTileH + 2;
-
-__device__ void lr_tile(FArgs a, int t, int* s_src, int* s_mid, const int* s_a2) {
-  const uint16_t* cdef = a.lr_cdef;
-  const uint16_t* curr = a.upscaled ? a.lr_prev_up : a.lr_curr;
-  const int2 tile = a.plan.lr_tiles[t];
-  const DevLr& j = a.plan.lr[tile.x];
-  const int x0 = j.x + (tile.y & 0xffff), y0 = j.y + (tile.y >> 16);
-  const int tw = min(kLrTileW, j.x + j.w - x0), th = min(kLrTileH, j.y + j.h - y0);
-  LayRef L = a.lay;
-  const int p = j.plane, bd = L.bit_depth;
-  LrCtx c;
-  c.cdef = cdef + L.plane_off[p];
-  c.curr = curr + L.plane_off[p];
-  c.stride = L.stride[p];
-  c.pw = L.out_w[p];
-  c.ph = L.out_h[p];
-  c.s0 = j.stripe0;
-  c.s1 = j.stripe1;
-  {
-    /* all of a thread's loads issued before its LDS writes */
-    constexpr int kStage = (kLrSrcW * kLrSrcH + 255) / 256;
-    int val[kStage], at[kStage];
-    Walk256 it(tw + 6);
+__device__ __forceinline__ void lr_store(uint16_t* dst, const int* v, int n, bool aligned) {
+  if (n >= 4 && aligned) {
+    uint2 w;
+    w.x = pack2(v[0], v[1]);
+    w.y = pack2(v[2], v[3]);
+    *reinterpret_cast<uint2*>(dst) = w;
+  } else {
 #pragma unroll
-    for (int u = 0; u < kStage; ++u) {
-      at[u] = it.r < th + 6 ? it.r * kLrSrcW + it.q : -1;
-      val[u] = at[u] >= 0 ? c.src(x0 - 3 + it.q, y0 - 3 + it.r) : 0;
-      it.next();
-    }
-#pragma unroll
-    for (int u = 0; u < kStage; ++u)
-      if (at[u] >= 0) s_src[at[u]] = val[u];
-  }
-  __syncthreads();
-  uint16_t* dst = a.frame + L.plane_off[p] + (size_t)y0 * c.stride + x0;
-  if (j.type == 1) {
-    const int r0 = bd == 12 ? 5 : 3, r1 = bd == 12 ? 9 : 11;
-    const int off = 1 << (bd + 7 - r0 - 1);
-    const int lim = (1 << (bd + 1 + 7 - r0)) - 1;
-    int ht[7], vt[7];
-#pragma unroll
-    for (int t = 0; t < 3; ++t) {
-      vt[t] = vt[6 - t] = j.vf[t];
-      ht[t] = ht[6 - t] = j.hf[t];
-    }
-    vt[3] = 128 - 2 * (j.vf[0] + j.vf[1] + j.vf[2]);
-    ht[3] = 128 - 2 * (j.hf[0] + j.hf[1] + j.hf[2]);
-    for (Walk256 it(tw); it.r < th + 6; it.next()) {
-      const int r = it.r, q = it.q;
-      const int* row = s_src + r * kLrSrcW + q;
-      int sum = 0;
-#pragma unroll
-      for (int k = 0; k < 7; ++k) sum += ht[k] * row[k];
-      s_mid[r * kLrTileW + q] = clampi(rsr64(sum, r0), -off, lim - off);
-    }
-    __syncthreads();
-    for (Walk256 it(tw); it.r < th; it.next()) {
-      const int r = it.r, q = it.q;
-      int sum = 0;
-#pragma unroll
-      for (int t = 0; t < 7; ++t) sum += vt[t] * s_mid[(r + t) * kLrTileW + q];
-      dst[(size_t)r * c.stride + q] = (uint16_t)clampi(rsr64(sum, r1), 0, a.maxv);
-    }
-    return;
-  }
-  /* self guided: A and B of each pass on the (th + 2) x (tw + 2) positions
-   * around the tile */
-  for (int pass = 0; pass < 2; ++pass) {
-    const int rr = j.r[pass];
-    if (rr == 0) continue;
-    const int d = 2 * rr + 1, n = d * d;
-    const int64_t n2e = (int64_t)n * n * j.eps[pass];
-    const int64_t mt = (((int64_t)1 << 20) + n2e / 2) / n2e;
-    const int inv = ((1 << 12) + n / 2) / n;
-    int* A = s_mid + (2 * pass) * kLrAbH * kLrAbW;
-    int* B = A + kLrAbH * kLrAbW;
-    for (Walk256 it(tw + 2); it.r < th + 2; it.next()) {
-      const int r = it.r, q = it.q;
-      /* position (x0 - 1 + q, y0 - 1 + r); its window starts at src row
-       * r + 2 - rr, column q + 2 - rr of the staged window */
-      /* at most 25 samples of 12 bits: the sums fit 32 bits */
-      int sa32 = 0, sb32 = 0;
-      for (int dy = 0; dy < d; ++dy) {
-        const int* row = s_src + (r + 2 - rr + dy) * kLrSrcW + q + 2 - rr;
-        for (int dx = 0; dx < d; ++dx) {
-          const int v = row[dx];
-          sa32 += v * v;
-          sb32 += v;
-        }
-      }
-      int64_t sa = sa32, sb = sb32;
-      const int64_t braw = sb;
-      if (bd > 8) {
-        sa = rsr64(sa, 2 * (bd - 8));
-        sb = rsr64(sb, bd - 8);
-      }
-      int64_t pp = sa * n - sb * sb;
-      if (pp < 0) pp = 0;
-      const int z = rsr64(pp * mt, 20);
-      const int a2 = z >= 255 ? 256 : s_a2[z];
-      A[r * kLrAbW + q] = a2;
-      B[r * kLrAbW + q] = rsr64((int64_t)(256 - a2) * braw * inv, 12);
-    }
-  }
-  __syncthreads();
-  const int w0 = j.xqd[0], w1 = j.xqd[1], w2 = (1 << 7) - w0 - w1;
-  for (Walk256 it(tw); it.r < th; it.next()) {
-    const int r = it.r, q = it.q;
-    const int y = y0 + r;
-    const int u = s_src[(r + 3) * kLrSrcW + q + 3];
-    int flt[2] = {0, 0};
-#pragma unroll
-    for (int pass = 0; pass < 2; ++pass) {
-      if (j.r[pass] == 0) continue;
-      const int* A = s_mid + (2 * pass) * kLrAbH * kLrAbW;
-      const int* B = A + kLrAbH * kLrAbW;
-      int sa = 0, sb = 0;
-#pragma unroll
-      for (int dy = -1; dy <= 1; ++dy)
-#pragma unroll
-        for (int dx = -1; dx <= 1; ++dx) {
-          const int wgt =
-              pass == 0 ? (((y + dy) & 1) ? (dx == 0 ? 6 : 5) : 0) : ((dx == 0 || dy == 0) ? 4 : 3);
-          if (!wgt) continue;
-          const int o = (r + 1 + dy) * kLrAbW + q + 1 + dx;
-          sa += wgt * A[o];
-          sb += wgt * B[o];
-        }
-      const int sh = (pass == 0 && (y & 1)) ? 4 : 5;
-      flt[pass] = rsr64((int64_t)sa * u + sb, 8 + sh - 4);
-    }
-    const int us = u << 4;
-    int64_t v = (int64_t)w1 * us;
-    v += (int64_t)w0 * (j.r[0] ? flt[0] : us);
-    v += (int64_t)w2 * (j.r[1] ? flt[1] : us);
-    dst[(size_t)r * c.stride + q] = (uint16_t)clampi(rsr64(v, 4 + 7), 0, a.maxv);
+    for (int i = 0; i < 4; ++i)
+      if (i < n) dst[i] = (uint16_t)v[i];
   }
 }
 
+__device__ __forceinline__ void lr_wiener(LrLds& S, const DevLr& j, int bd, int maxv, int tw, int th, uint16_t* dst,
+                                          int stride, bool aligned) {
+  const int r0 = bd == 12 ? 5 : 3, r1 = bd == 12 ? 9 : 11;
+  const int off = 1 << (bd + 7 - r0 - 1);
+  const int top = (1 << (bd + 1 + 7 - r0)) - 1 - off;
+  int ht[7], vt[7];
+  bool narrow = true;
+#pragma unroll
+  for (int t = 0; t < 3; ++t) {
+    vt[t] = vt[6 - t] = j.vf[t];
+    ht[t] = ht[6 - t] = j.hf[t];
+  }
+  vt[3] = 128 - 2 * (j.vf[0] + j.vf[1] + j.vf[2]);
+  ht[3] = 128 - 2 * (j.hf[0] + j.hf[1] + j.hf[2]);
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+    narrow = narrow && abs(ht[t]) < 8192 && abs(vt[t]) < 8192;
+  const int quads = (tw + 3) >> 2, k = threadIdx.x & 15;
+  if (!narrow) {
+    /* taps beyond 13 bits and a sign (no stream codes them), whose sums of
+     * products could leave 32 bits: one product at a time */
+    for (int r = threadIdx.x >> 4; r < th + 6; r += 16)
+      for (int i = 0; k < quads && i < 4; ++i) {
+        int sum = 0;
+        for (int t = 0; t < 7; ++t) sum += ht[t] * (int)S.src[r * kLrSrcLd + 4 * k + i + 1 + t];
+        S.mid[r * kLrMidLd + 4 * k + i] = (int16_t)clampi(rsr64(sum, r0), -off, top);
+      }
+    __syncthreads();
+    for (int r = threadIdx.x >> 4; r < th; r += 16)
+      for (int i = 0; k < quads && i < 4 && 4 * k + i < tw; ++i) {
+        int sum = 0;
+        for (int t = 0; t < 7; ++t) sum += vt[t] * (int)S.mid[(r + t) * kLrMidLd + 4 * k + i];
+        dst[(size_t)r * stride + 4 * k + i] = (uint16_t)clampi(rsr64(sum, r1), 0, maxv);
+      }
+    return;
+  }
+  const uint32_t h01 = pack2(ht[0], ht[1]), h23 = pack2(ht[2], ht[3]), h45 = pack2(ht[4], ht[5]), h6 = pack2(ht[6], 0);
+  for (int r = threadIdx.x >> 4; r < th + 6; r += 16) {
+    if (k >= quads) break;
+    /* samples x - 4 .. x + 7 */
+    const uint2* q = reinterpret_cast<const uint2*>(S.src + r * kLrSrcLd + 4 * k);
+    const uint2 q0 = q[0], q1 = q[1], q2 = q[2];
+    const uint32_t w[6] = {q0.x, q0.y, q1.x, q1.y, q2.x, q2.y};
+    uint32_t m[5];
+#pragma unroll
+    for (int t = 0; t < 5; ++t) m[t] = __builtin_amdgcn_alignbit(w[t + 1], w[t], 16);
+    const int half = 1 << (r0 - 1);
+    int v[4];
+    v[0] = dot2(m[3], h6, dot2(m[2], h45, dot2(m[1], h23, dot2(m[0], h01, half))));
+    v[1] = dot2(w[4], h6, dot2(w[3], h45, dot2(w[2], h23, dot2(w[1], h01, half))));
+    v[2] = dot2(m[4], h6, dot2(m[3], h45, dot2(m[2], h23, dot2(m[1], h01, half))));
+    v[3] = dot2(w[5], h6, dot2(w[4], h45, dot2(w[3], h23, dot2(w[2], h01, half))));
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = clampi(v[i] >> r0, -off, top);
+    uint2 out;
+    out.x = pack2(v[0], v[1]);
+    out.y = pack2(v[2], v[3]);
+    *reinterpret_cast<uint2*>(S.mid + r * kLrMidLd + 4 * k) = out;
+  }
+  __syncthreads();
+  const uint32_t v01 = pack2(vt[0], vt[1]), v23 = pack2(vt[2], vt[3]), v45 = pack2(vt[4], vt[5]), v6 = pack2(vt[6], 0),
+                 v6h = pack2(0, vt[6]);
+  const int r = threadIdx.x >> 4;
+  if (r < th && k < quads) {
+    const int half = 1 << (r1 - 1);
+    int v[4] = {half, half, half, half};
+    const uint32_t vv[3] = {v01, v23, v45};
+#pragma unroll
+    for (int t = 0; t < 3; ++t) {
+      const uint2 u = *reinterpret_cast<const uint2*>(S.mid + (r + 2 * t) * kLrMidLd + 4 * k);
+      const uint2 d = *reinterpret_cast<const uint2*>(S.mid + (r + 2 * t + 1) * kLrMidLd + 4 * k);
+      v[0] = dot2(__builtin_amdgcn_perm(d.x, u.x, 0x05040100u), vv[t], v[0]);
+      v[1] = dot2(__builtin_amdgcn_perm(d.x, u.x, 0x07060302u), vv[t], v[1]);
+      v[2] = dot2(__builtin_amdgcn_perm(d.y, u.y, 0x05040100u), vv[t], v[2]);
+      v[3] = dot2(__builtin_amdgcn_perm(d.y, u.y, 0x07060302u), vv[t], v[3]);
+    }
+    const uint2 e = *reinterpret_cast<const uint2*>(S.mid + (r + 6) * kLrMidLd + 4 * k);
+    v[0] = dot2(e.x, v6, v[0]);
+    v[1] = dot2(e.x, v6h, v[1]);
+    v[2] = dot2(e.y, v6, v[2]);
+    v[3] = dot2(e.y, v6h, v[3]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = clampi(v[i] >> r1, 0, maxv);
+    lr_store(dst + (size_t)r * stride + 4 * k, v, tw - 4 * k, aligned);
+  }
+}
+
+/* A and B of one position of a pass from its box sums (at most 25 samples of
+ * 12 bits), n samples in the box */
+__device__ __forceinline__ uint32_t sgr_ab(int sq, int sum, int n, uint32_t mt, uint32_t inv, int bd, const uint16_t* a2s) {
+  int sa = sq, sb = sum;
+  if (bd > 8) {
+    sa = rnd2(sa, 2 * (bd - 8));
+    sb = rnd2(sb, bd - 8);
+  }
+  const int pp = max(0, sa * n - sb * sb);
+  const uint32_t z = (uint32_t)(((uint64_t)(uint32_t)pp * mt + (1u << 19)) >> 20);
+  const uint32_t a2 = z >= 255 ? 256 : a2s[z];
+  const uint32_t b = ((256 - a2) * (uint32_t)sum * inv + (1u << 11)) >> 12;
+  return b << 9 | a2;
+}
+
+__device__ __forceinline__ void lr_sgr(LrLds& S, const DevLr& j, int bd, int maxv, int tw, int th, int y0, uint16_t* dst,
+                                       int stride, bool aligned) {
+  constexpr int kQ = kLrW + 2, kRun = 6; /* columns of positions, rows a lane walks */
+  static_assert(kQ * (kLrAbRows / kRun) <= 256 && kLrAbRows % kRun == 0, "self-guided positions per lane");
+  const bool p0 = j.r[0] != 0, p1 = j.r[1] != 0;
+  const int q = threadIdx.x % kQ, g = threadIdx.x / kQ;
+  if (g < kLrAbRows / kRun && q < tw + 2) {
+    uint32_t mt[2], inv[2];
+#pragma unroll
+    for (int pass = 0; pass < 2; ++pass) {
+      const int n = pass ? 9 : 25;
+      const uint32_t n2e = (uint32_t)(n * n) * (uint32_t)max(j.eps[pass], 1);
+      mt[pass] = ((1u << 20) + n2e / 2) / n2e;
+      inv[pass] = ((1 << 12) + n / 2) / n;
+    }
+    /* row sums of the walked rows: five wide, three wide, and of squares */
+    int h5[kRun + 4], s5[kRun + 4], h3[kRun + 4], s3[kRun + 4];
+    const int sh = ((q + 1) & 1) * 16;
+    const uint32_t* col = reinterpret_cast<const uint32_t*>(S.src + kRun * g * kLrSrcLd + ((q + 1) & ~1));
+#pragma unroll
+    for (int i = 0; i < kRun + 4; ++i) {
+      const uint32_t w0 = col[i * (kLrSrcLd / 2)], w1 = col[i * (kLrSrcLd / 2) + 1], w2 = col[i * (kLrSrcLd / 2) + 2];
+      const uint32_t a = __builtin_amdgcn_alignbit(w1, w0, sh), b = __builtin_amdgcn_alignbit(w2, w1, sh),
+                     c = (w2 >> sh) & 0xffffu;
+      const int first = (int)(a & 0xffffu), last = (int)c;
+      const int mh = dot2(b, 0x00010001u, (int)(a >> 16));
+      const int ms = dot2(b, b, __mul24((int)(a >> 16), (int)(a >> 16)));
+      h3[i] = mh;
+      s3[i] = ms;
+      h5[i] = mh + first + last;
+      s5[i] = ms + __mul24(first, first) + __mul24(last, last);
+    }
+    uint32_t* ab0 = S.ab[0] + kRun * g * kLrAbLd + q;
+    uint32_t* ab1 = S.ab[1] + kRun * g * kLrAbLd + q;
+    const int odd = (y0 - 1) & 1; /* kRun is even: of the run's first row */
+#pragma unroll
+    for (int i = 0; i < kRun; ++i) {
+      if (p0 && ((i & 1) ^ odd))
+        ab0[i * kLrAbLd] = sgr_ab(s5[i] + s5[i + 1] + s5[i + 2] + s5[i + 3] + s5[i + 4],
+                                  h5[i] + h5[i + 1] + h5[i + 2] + h5[i + 3] + h5[i + 4], 25, mt[0], inv[0], bd, S.a2);
+      if (p1)
+        ab1[i * kLrAbLd] = sgr_ab(s3[i + 1] + s3[i + 2] + s3[i + 3], h3[i + 1] + h3[i + 2] + h3[i + 3], 9, mt[1], inv[1],
+                                  bd, S.a2);
+    }
+  }
+  __syncthreads();
+  const int r = threadIdx.x >> 4, k = threadIdx.x & 15;
+  if (r >= th || 4 * k >= tw) return;
+  const int y = y0 + r;
+  auto row = [&](int pass, int rr, uint32_t* v) {
+    const uint32_t* p = S.ab[pass] + rr * kLrAbLd + 4 * k;
+    const uint4 lo = *reinterpret_cast<const uint4*>(p);
+    const uint2 hi = *reinterpret_cast<const uint2*>(p + 4);
+    v[0] = lo.x, v[1] = lo.y, v[2] = lo.z, v[3] = lo.w, v[4] = hi.x, v[5] = hi.y;
+  };
+  const uint2 us = *reinterpret_cast<const uint2*>(S.src + (r + 3) * kLrSrcLd + 4 * k + 4);
+  const int u[4] = {(int)(us.x & 0xffff), (int)(us.x >> 16), (int)(us.y & 0xffff), (int)(us.y >> 16)};
+  int f0[4], f1[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) f0[i] = f1[i] = u[i] << 4;
+  if (p0) {
+    /* the odd rows among y - 1 .. y + 1, 5 6 5 across */
+    uint32_t a[6], b[6], v[6];
+    if (y & 1) {
+      row(0, r + 1, v);
+#pragma unroll
+      for (int i = 0; i < 6; ++i) a[i] = v[i] & 511, b[i] = v[i] >> 9;
+    } else {
+      uint32_t d[6];
+      row(0, r, v);
+      row(0, r + 2, d);
+#pragma unroll
+      for (int i = 0; i < 6; ++i) a[i] = (v[i] & 511) + (d[i] & 511), b[i] = (v[i] >> 9) + (d[i] >> 9);
+    }
+    const int sh = 4 + ((y & 1) ? 4 : 5);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int sa = 5 * (int)(a[i] + a[i + 1] + a[i + 2]) + (int)a[i + 1];
+      const int sb = 5 * (int)(b[i] + b[i + 1] + b[i + 2]) + (int)b[i + 1];
+      f0[i] = rnd2(__mul24(sa, u[i]) + sb, sh);
+    }
+  }
+  if (p1) {
+    /* 3x3, 4 on the cross, 3 in the corners */
+    uint32_t t[6], m[6], d[6];
+    row(1, r, t);
+    row(1, r + 1, m);
+    row(1, r + 2, d);
+    int ap[6], aq[6], bp[6], bq[6]; /* a column in the middle, at a side */
+#pragma unroll
+    for (int i = 0; i < 6; ++i) {
+      const int ea = (int)((t[i] & 511) + (d[i] & 511)), eb = (int)((t[i] >> 9) + (d[i] >> 9));
+      ap[i] = (ea + (int)(m[i] & 511)) << 2;
+      bp[i] = (eb + (int)(m[i] >> 9)) << 2;
+      aq[i] = ap[i] - ea;
+      bq[i] = bp[i] - eb;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int sa = aq[i] + ap[i + 1] + aq[i + 2], sb = bq[i] + bp[i + 1] + bq[i + 2];
+      f1[i] = rnd2(__mul24(sa, u[i]) + sb, 9);
+    }
+  }
+  const int w0 = j.xqd[0], w1 = j.xqd[1], w2 = (1 << 7) - w0 - w1;
+  int out[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    int64_t v = (int64_t)w1 * (u[i] << 4);
+    v += (int64_t)w0 * f0[i];
+    v += (int64_t)w2 * f1[i];
+    out[i] = clampi(rsr64(v, 4 + 7), 0, maxv);
+  }
+  lr_store(dst + (size_t)r * stride + 4 * k, out, tw - 4 * k, aligned);
+}
+
+__device__ __forceinline__ void lr_tile(FArgs a, int t, LrLds& S) {
+  const int2 tile = a.plan.lr_tiles[t];
+  const DevLr& j = a.plan.lr[tile.x];
+  const int x0 = j.x + (tile.y & 0xffff), y0 = j.y + (tile.y >> 16);
+  const int tw = min(kLrW, j.x + j.w - x0), th = min(kLrH, j.y + j.h - y0);
+  LayRef L = a.lay;
+  const int p = j.plane, bd = L.bit_depth;
+  const int stride = L.stride[p], pw = L.out_w[p], ph = L.out_h[p], s0 = j.stripe0, s1 = j.stripe1;
+  const uint16_t* cdef = a.lr_cdef + L.plane_off[p];
+  const uint16_t* curr = (a.upscaled ? a.lr_prev_up : a.lr_curr) + L.plane_off[p];
+  const bool aligned = (x0 & 3) == 0; /* units are multiples of 4 wide but for the smallest sizes */
+  {
+    /* all of a thread's loads issued before its LDS writes */
+    constexpr int kQuads = kLrSrcLd / 4 - 1, kIt = (kQuads * kLrSrcRows + 255) / 256; /* columns -4 .. kLrW + 3 */
+    uint2 val[kIt];
+#pragma unroll
+    for (int u = 0; u < kIt; ++u) {
+      const int e = (int)threadIdx.x + 256 * u, r = e / kQuads, x = x0 - 4 + 4 * (e - r * kQuads);
+      val[u] = make_uint2(0, 0);
+      if (r >= th + 6 || x >= x0 + tw + 3) continue;
+      const int y = clampi(y0 - 3 + r, 0, ph - 1);
+      const uint16_t* src = y < s0 ? curr + (size_t)max(y, s0 - 2) * stride
+                                   : y > s1 ? curr + (size_t)min(y, s1 + 2) * stride : cdef + (size_t)y * stride;
+      if (aligned && x >= 0 && x + 3 < pw) {
+        val[u] = *reinterpret_cast<const uint2*>(src + x);
+      } else {
+        val[u].x = pack2(src[clampi(x, 0, pw - 1)], src[clampi(x + 1, 0, pw - 1)]);
+        val[u].y = pack2(src[clampi(x + 2, 0, pw - 1)], src[clampi(x + 3, 0, pw - 1)]);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < kIt; ++u) {
+      const int e = (int)threadIdx.x + 256 * u, r = e / kQuads;
+      if (r < kLrSrcRows) *reinterpret_cast<uint2*>(S.src + r * kLrSrcLd + 4 * (e - r * kQuads)) = val[u];
+    }
+  }
+  __syncthreads();
+  uint16_t* dst = a.frame + L.plane_off[p] + (size_t)y0 * stride + x0;
+  if (j.type == 1)
+    lr_wiener(S, j, bd, a.maxv, tw, th, dst, stride, aligned);
+  else
+    lr_sgr(S, j, bd, a.maxv, tw, th, y0, dst, stride, aligned);
+}
+
 __global__ __launch_bounds__(256) void k_lr(BatchDev B) {
-  __shared__ int s_src[kLrSrcH * kLrSrcW];
-  __shared__ int s_mid[4 * kLrAbH * kLrAbW]; /* Wiener rows, or A0 B0 A1 B1 */
-  __shared__ int s_a2[256];
-  s_a2[threadIdx.x] = sgr_a2(threadIdx.x);
+  __shared__ LrLds S;
+  S.a2[threadIdx.x] = (uint16_t)sgr_a2(threadIdx.x);
   __syncthreads();
   const AV1H_CMEM int32_t* pre = kernel_prefix(B, kKLr);
   const int total = pre[B.njobs];
@@ -799,7 +924,7 @@ __global__ __launch_bounds__(256) void k_lr(BatchDev B) {
     const int v = xcd_group(base, total);
     if (v < 0) continue;
     const int j = find_job(pre, B.njobs, v);
-    lr_tile(filter_args(B, j), v - pre[j], s_src, s_mid, s_a2);
+    lr_tile(filter_args(B, j), v - pre[j], S);
     __syncthreads();
   }
 }
