@@ -2027,10 +2027,10 @@ int kernel_groups(const FrameJob& fj, int k, int cdef_batch) {
     case kKDeblockV: return p.n_deblock_v > 0 ? (p.lines_v + 255) / 256 : 0;
     case kKDeblockH: return p.n_deblock_h > 0 ? (p.lines_h + 255) / 256 : 0;
     case kKCdefDir: return p.n_cdef > 0 ? (p.n_cdef_dir + kCdefDirPerGroup - 1) / kCdefDirPerGroup : 0;
-    case kKCdefLuma: return p.n_cdef > 0 ? (p.n_cdef_luma + 4 * cdef_batch - 1) / (4 * cdef_batch) : 0;
+    case kKCdefLuma: return p.n_cdef > 0 ? (p.n_cdef_luma + 16 * cdef_batch - 1) / (16 * cdef_batch) : 0;
     case kKCdefChroma: {
       const int nc = p.n_cdef - p.n_cdef_luma;
-      const int per = cdef_batch * 256 / ((8 >> L.ss_x) * (8 >> L.ss_y));
+      const int per = cdef_batch * 1024 / ((8 >> L.ss_x) * (8 >> L.ss_y));
       return nc > 0 ? (nc + per - 1) / per : 0;
     }
     case kKUpscale: return f.upscaled ? upscale_tiles(L, f.uses_lr ? 2 : 1) : 0;

@@ -14,6 +14,9 @@ namespace {
 
 #define SPEC(off) (av1t_spec_table + (off))
 
+/* global (not generic) pointers: their accesses need no wait for LDS */
+#define AV1H_GLOBAL __attribute__((address_space(1)))
+
 __device__ __forceinline__ int clampi(int v, int lo, int hi) { return v < lo ? lo : (v > hi ? hi : v); }
 __device__ __forceinline__ int rnd2(int v, int n) { return n <= 0 ? v : (v + (1 << (n - 1))) >> n; }
 __device__ __forceinline__ int rsr64(int64_t v, int n) { return (int)((v + ((int64_t)1 << (n - 1))) >> n); }
@@ -163,36 +166,6 @@ __global__ __launch_bounds__(256) void k_deblock(BatchDev B, int pass) {
 
 __device__ __forceinline__ int flog2(int v) { return 31 - __builtin_clz(v); }
 
-__device__ __forceinline__ int constrain(int diff, int thr, int damping) {
-  if (!thr) return 0;
-  const int adj = max(0, damping - flog2(thr));
-  const int mag = abs(diff);
-  const int v = clampi(thr - (mag >> adj), 0, mag);
-  return diff < 0 ? -v : v;
-}
-
-/* A sample at byte offset o of a picture whose base is the same for the
- * whole wave: one scalar base plus a 32-bit vector offset, no per-lane
- * 64-bit address arithmetic (a picture buffer is far below 4 GB) */
-__device__ __forceinline__ int tap16(const char* base, unsigned o) {
-  return *reinterpret_cast<const uint16_t*>(base + o);
-}
-
-/* constrain() of tap v around the centre x, the shift of its threshold
- * precomputed: |v - x| is one sum-of-absolute-differences instruction
- * (samples are at most 16 bit, the upper halves zero) */
-__device__ __forceinline__ int constrain_vx(int v, int x, int thr, int adj) {
-  const int mag = (int)__builtin_amdgcn_sad_u16((unsigned)v, (unsigned)x, 0u);
-  const int c = max(0, min(thr - (mag >> adj), mag));
-  return v < x ? -c : c;
-}
-
-__constant__ const int kCdefDirs[8][2][2] = {{{-1, 1}, {-2, 2}}, {{0, 1}, {-1, 2}}, {{0, 1}, {0, 2}},
-                                             {{0, 1}, {1, 2}},   {{1, 1}, {2, 2}},   {{1, 0}, {2, 1}},
-                                             {{1, 0}, {2, 0}},   {{1, 0}, {2, -1}}};
-__constant__ const int kCdefUvDir[2][2][8] = {{{0, 1, 2, 3, 4, 5, 6, 7}, {1, 2, 2, 2, 3, 4, 6, 0}},
-                                              {{7, 0, 2, 4, 5, 6, 6, 6}, {0, 1, 2, 3, 4, 5, 6, 7}}};
-
 /* Direction search of luma 8x8 blocks (av1gpu_kernels.h:2601-2660), one
  * block per lane: a lane reads its block's eight rows (one 16-byte load
  * each: rows start on 8-sample boundaries of 128-sample aligned strides),
@@ -280,224 +253,235 @@ __global__ __launch_bounds__(256) void k_cdef_dir(BatchDev B) {
   }
 }
 
-/* CDEF of the listed blocks (av1gpu_kernels.h:2662-2775). A wave takes
- * 64 / (W x H) blocks of one plane kind (W x H samples each: 8x8 luma, the
- * chroma size by subsampling) and first stages each block with a 2-sample
- * border from the deblocked snapshot into LDS, one 32-bit load per sample
- * pair (rows start on even samples of 128-sample aligned strides), marking
- * samples outside the plane; then one lane per sample reads its twelve taps
- * from LDS. Samples of unlisted blocks are already final in the frame. */
-constexpr uint16_t kCdefOutside = 0xffff; /* no sample reaches this value */
-constexpr int kCdefTileWave = 256;         /* LDS samples per wave         */
+/* CDEF of the listed blocks (av1gpu_kernels.h:2662-2775), four neighbouring
+ * samples of a block row per lane: a wave holds four luma blocks, four to
+ * sixteen chroma blocks by subsampling. A lane reads its samples and each of
+ * its twelve taps straight from the deblocked snapshot, three whole words that
+ * hold them (loads that start inside a word ran at a fraction of the rate: 57
+ * us on a 2160p frame instead of 48), and filters two samples per instruction
+ * in packed 16-bit words. A tap outside the plane reads as
+ * kCdefOutside, which is no minimum without a sign, no maximum with one, and so
+ * far from every sample that its constrained difference is 0. Samples of
+ * unlisted blocks are already final in the frame.
+ * One sample per lane from LDS tiles, bound by instructions, took 24.5 us on a
+ * 1080p frame, 79 on a 2160p one, 92 on eight streams; now 21, 43 and 53,
+ * bound by the cache lines the loads touch: eight samples per lane halved the
+ * instructions per sample and took 23, 56 and 66. */
+typedef short cdef_s2 __attribute__((ext_vector_type(2)));
+typedef unsigned short cdef_u2 __attribute__((ext_vector_type(2)));
+constexpr uint32_t kCdefOutside = 0x80008000u;
 
-/* the tap of direction table entry e = (dy, dx) as an offset in a tile of
- * row pitch tw */
-__device__ __forceinline__ int cdef_tap(const int* e, int tw) { return e[0] * tw + e[1]; }
+/* (dy, dx) of direction d's near and far tap: signed nibble d */
+constexpr uint32_t kCdefDy0 = 0x1111000fu, kCdefDx0 = 0x00011111u, kCdefDy1 = 0x222210feu, kCdefDx1 = 0xf0122222u;
+__device__ __forceinline__ int cdef_nibble(uint32_t table, int d) { return __builtin_amdgcn_sbfe((int)table, 4 * d, 4); }
 
-/* A block's CDEF record and, when its direction is searched, its entry of
- * the direction map: loaded before its tile is staged, so that the two
- * loads' latencies overlap. A luma wave holds one block: its values are
- * wave-uniform and come through the scalar cache (the map was written by an
- * earlier kernel); chroma waves hold several blocks. */
-struct CdefBlockIn {
-  int plane, x, y, pri, sec, damping, dir, yd, var;
+/* one chroma direction for a luma one where the axes are scaled apart */
+__device__ __forceinline__ int cdef_uv_dir(int ss_x, int ss_y, int d) {
+  if (ss_x == ss_y) return d;
+  return (int)((ss_x ? 0x66654207u : 0x06432221u) >> (4 * d)) & 7;
+}
+
+struct CdefPlane {
+  const AV1H_GLOBAL uint16_t* src; /* the plane in the snapshot */
+  int stride, w, h;
 };
 
-template <bool kLuma>
-__device__ __forceinline__ CdefBlockIn cdef_block_in(FArgs a, int first, int bi) {
-  CdefBlockIn q;
-  if (kLuma) {
-    bi = __builtin_amdgcn_readfirstlane(bi);
-    const AV1H_CMEM DevCdef& cu = cmem(a.plan.cdef)[first + bi];
-    q = CdefBlockIn{cu.plane_damping & 3, cu.x, cu.y, cu.pri, cu.sec, cu.plane_damping >> 2, cu.dir, 0, 0};
-    if (q.dir < 0) {
-      const AV1H_CMEM int* m = cmem(a.cdef_dir) + 2 * ((q.y >> 3) * a.cdef_dir_w + (q.x >> 3));
-      q.yd = m[0];
-      q.var = m[1];
+/* four samples from (x, y) on; with kEdge they may lie outside the plane, at
+ * most two samples away (w is at least 4, a lane's own samples are inside) */
+template <bool kEdge>
+__device__ __forceinline__ uint2 cdef_load(const CdefPlane& P, int x, int y) {
+  const int xa = kEdge ? clampi(x, 0, P.w - 4) : x, ya = kEdge ? clampi(y, 0, P.h - 1) : y;
+  const int at = ya * P.stride + xa;
+  const AV1H_GLOBAL uint32_t* q = (const AV1H_GLOBAL uint32_t*)(P.src + (at & ~1));
+  const uint32_t w0 = q[0], w1 = q[1], w2 = q[2];
+  uint2 v = make_uint2(__builtin_amdgcn_alignbit(w1, w0, (at & 1) * 16), __builtin_amdgcn_alignbit(w2, w1, (at & 1) * 16));
+  if (kEdge) {
+    const int n = x - xa;
+    if (n < 0) {
+      v.y = n == -1 ? __builtin_amdgcn_alignbit(v.y, v.x, 16) : v.x;
+      v.x = n == -1 ? __builtin_amdgcn_alignbit(v.x, kCdefOutside, 16) : kCdefOutside;
+    } else if (n > 0) {
+      v.x = n == 1 ? __builtin_amdgcn_alignbit(v.y, v.x, 16) : v.y;
+      v.y = n == 1 ? __builtin_amdgcn_alignbit(kCdefOutside, v.y, 16) : kCdefOutside;
     }
-  } else {
-    const DevCdef c = a.plan.cdef[first + bi];
-    q = CdefBlockIn{c.plane_damping & 3, c.x, c.y, c.pri, c.sec, c.plane_damping >> 2, c.dir, 0, 0};
-    if (q.dir < 0) {
-      LayRef L = a.lay;
-      const int lx = c.x << L.ss_x, ly = c.y << L.ss_y;
-      q.yd = a.cdef_dir[2 * ((ly >> 3) * a.cdef_dir_w + (lx >> 3))];
-    }
+    if (y != ya) v = make_uint2(kCdefOutside, kCdefOutside);
   }
-  return q;
+  return v;
 }
 
-/* One sample (r, k) of block `c`, its tile at `t` (row pitch TW, the sample
- * at t[(r + 2) * TW + k + 2]). False when it keeps the snapshot's value.
- * Luma reads the direction table from constant memory (its direction is
- * wave-uniform), chroma from LDS. */
-template <int W, int H, bool kLuma>
-__device__ __forceinline__ bool cdef_tile_sample(FArgs a, const CdefBlockIn& c, int r, int k, const uint16_t* t,
-                                                 const int (*sdirs)[2][2], int64_t* off, int* val) {
-  constexpr int TW = W + 4;
-  const int (*dirs)[2][2] = kLuma ? kCdefDirs : sdirs;
-  LayRef L = a.lay;
-  const int p = kLuma ? 0 : c.plane;
-  const int cs = L.bit_depth - 8;
-  const int pw = L.grid_w[p], ph = L.grid_h[p];
-  if (c.x + k >= pw || c.y + r >= ph) return false;
-  int pri = c.pri << cs;
-  const int sec = c.sec << cs;
-  const int damping = c.damping + cs - (kLuma ? 0 : 1);
-  int dir = c.dir;
-  if (dir < 0) {
-    if (!kLuma) {
-      dir = pri == 0 ? 0 : kCdefUvDir[L.ss_x][L.ss_y][c.yd];
-    } else {
-      const int vs = (c.var >> 6) ? min(flog2(c.var >> 6), 12) : 0;
-      dir = pri == 0 ? 0 : c.yd;
-      pri = c.var ? ((pri * (4 + vs) + 8) >> 4) : 0;
-    }
-  }
-  if (pri == 0 && sec == 0) return false; /* the destination already holds the snapshot's value */
-  const int adjp = pri ? max(0, damping - flog2(pri)) : 0, adjs = sec ? max(0, damping - flog2(sec)) : 0;
-  const int ts = (pri >> cs) & 1;
-  const int pt0 = ts ? 3 : 4, pt1 = ts ? 3 : 2;
-  const int d1 = (dir + 2) & 7, d2 = (dir + 6) & 7;
-  const uint16_t* s0 = t + (r + 2) * TW + k + 2;
-  const int x = s0[0];
-  int sum = 0, lo = x, hi = x;
-  /* every tap inside the plane: no marks to test */
-  const bool inner = c.x >= 2 && c.y >= 2 && c.x + W + 2 <= pw && c.y + H + 2 <= ph;
+struct CdefSum {
+  cdef_s2 x[2], sum[2], hi[2];
+  cdef_u2 lo[2];
+};
+
+/* one tap of weight wt: constrain() of its difference is the difference
+ * clamped to +-max(0, thr - (|difference| >> adj)) */
+__device__ __forceinline__ void cdef_add(CdefSum& s, uint2 v, uint32_t thr, uint32_t adj, uint32_t wt) {
 #pragma unroll
-  for (int tt = 0; tt < 2; ++tt) {
-    const int op = cdef_tap(dirs[dir][tt], TW), o1 = cdef_tap(dirs[d1][tt], TW), o2 = cdef_tap(dirs[d2][tt], TW);
-    const int wp = tt ? pt1 : pt0, ws = tt ? 1 : 2;
-#pragma unroll
-    for (int sg = -1; sg <= 1; sg += 2) {
-      const int vp = s0[sg * op], v1 = s0[sg * o1], v2 = s0[sg * o2];
-      if (inner) {
-        if (pri) sum += __mul24(wp, constrain_vx(vp, x, pri, adjp));
-        if (sec) sum += __mul24(ws, constrain_vx(v1, x, sec, adjs) + constrain_vx(v2, x, sec, adjs));
-        lo = min(lo, min(vp, min(v1, v2)));
-        hi = max(hi, max(vp, max(v1, v2)));
-      } else {
-        if (vp != kCdefOutside) {
-          if (pri) sum += __mul24(wp, constrain_vx(vp, x, pri, adjp));
-          lo = min(lo, vp);
-          hi = max(hi, vp);
-        }
-        if (v1 != kCdefOutside) {
-          if (sec) sum += __mul24(ws, constrain_vx(v1, x, sec, adjs));
-          lo = min(lo, v1);
-          hi = max(hi, v1);
-        }
-        if (v2 != kCdefOutside) {
-          if (sec) sum += __mul24(ws, constrain_vx(v2, x, sec, adjs));
-          lo = min(lo, v2);
-          hi = max(hi, v2);
-        }
-      }
-    }
+  for (int i = 0; i < 2; ++i) {
+    const uint32_t w = i ? v.y : v.x;
+    const cdef_s2 d = __builtin_bit_cast(cdef_s2, w) - s.x[i];
+    const cdef_u2 mag = __builtin_bit_cast(cdef_u2, __builtin_elementwise_max(d, -d));
+    const cdef_s2 lim = __builtin_bit_cast(
+        cdef_s2, __builtin_elementwise_sub_sat(__builtin_bit_cast(cdef_u2, thr), mag >> __builtin_bit_cast(cdef_u2, adj)));
+    s.sum[i] += __builtin_bit_cast(cdef_s2, wt) * __builtin_elementwise_max(__builtin_elementwise_min(d, lim), -lim);
   }
-  *off = L.plane_off[p] + (int64_t)(c.y + r) * L.stride[p] + c.x + k;
-  *val = clampi(clampi(x + ((8 + sum - (sum < 0)) >> 4), lo, hi), 0, a.maxv);
-  return true;
 }
 
-/* `batch` (1 to kSets) sets of 256 / (W x H) blocks per workgroup: every
- * lane loads its block record (and direction) of each set, the wave stages
- * all its sets' tiles, and only then filters them, so that a wave has the
- * loads of all its sets in flight at once. kSets bounds the registers the
- * sets take (one set keeps the kernel at 8 waves per SIMD). */
-template <int W, int H, bool kLuma, int kSets>
-__device__ __forceinline__ void cdef_tiles(FArgs a, int first, int count, int grp, int batch, uint16_t* tile,
-                                           const int (*dirs)[2][2]) {
-  constexpr int S = W * H, TW = W + 4, TH = H + 4, kWave = 64 / S, kPer = 256 / S;
-  constexpr int kPairs = TW / 2, kDw = kPairs * TH; /* 32-bit words per block tile */
-  static_assert(kWave * TW * TH <= kCdefTileWave, "tiles of a wave exceed its LDS");
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  uint16_t* wt = tile + wave * kCdefTileWave * kSets;
+__device__ __forceinline__ void cdef_range(CdefSum& s, uint2 v) {
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    s.lo[i] = __builtin_elementwise_min(s.lo[i], __builtin_bit_cast(cdef_u2, i ? v.y : v.x));
+    s.hi[i] = __builtin_elementwise_max(s.hi[i], __builtin_bit_cast(cdef_s2, i ? v.y : v.x));
+  }
+}
+
+struct CdefTaps {
+  int dir, pri, sec, adjp, adjs, pt0, pt1;
+};
+
+/* The result of one strength alone lies between the samples it weighs (12
+ * sixteenths of their differences), so the other's taps, which only the range
+ * needs, are left out then. */
+template <bool kEdge>
+__device__ __forceinline__ uint2 cdef_quad(const CdefPlane& P, int x, int y, const CdefTaps& c, int maxv) {
+  const uint2 own = cdef_load<false>(P, x, y);
+  CdefSum s;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    s.x[i] = s.hi[i] = __builtin_bit_cast(cdef_s2, i ? own.y : own.x);
+    s.lo[i] = __builtin_bit_cast(cdef_u2, i ? own.y : own.x);
+    s.sum[i] = cdef_s2{0, 0};
+  }
+  const bool both = c.pri != 0 && c.sec != 0;
+  /* the primary direction and the two secondary ones; one copy of the code */
+#pragma unroll 1
+  for (int k = 0; k < 3; ++k) {
+    if ((k ? c.sec : c.pri) == 0) continue;
+    const int d = (c.dir + 2 * k + (k == 2 ? 2 : 0)) & 7;
+    const int dx0 = cdef_nibble(kCdefDx0, d), dy0 = cdef_nibble(kCdefDy0, d);
+    const int dx1 = cdef_nibble(kCdefDx1, d), dy1 = cdef_nibble(kCdefDy1, d);
+    const uint32_t thr = (k ? c.sec : c.pri) * 0x10001u, adj = (k ? c.adjs : c.adjp) * 0x10001u;
+    const uint32_t w0 = (k ? 2 : c.pt0) * 0x10001u, w1 = (k ? 1 : c.pt1) * 0x10001u;
+    const uint2 v[4] = {cdef_load<kEdge>(P, x - dx0, y - dy0), cdef_load<kEdge>(P, x + dx0, y + dy0),
+                        cdef_load<kEdge>(P, x - dx1, y - dy1), cdef_load<kEdge>(P, x + dx1, y + dy1)};
+#pragma unroll
+    for (int t = 0; t < 4; ++t) cdef_add(s, v[t], thr, adj, t < 2 ? w0 : w1);
+    if (both) {
+#pragma unroll
+      for (int t = 0; t < 4; ++t) cdef_range(s, v[t]);
+    }
+  }
+  uint32_t out[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    cdef_s2 f = s.x[i] + ((s.sum[i] + (s.sum[i] >> 15) + (short)8) >> 4);
+    if (both) f = __builtin_elementwise_min(__builtin_elementwise_max(f, __builtin_bit_cast(cdef_s2, s.lo[i])), s.hi[i]);
+    out[i] = __builtin_bit_cast(uint32_t, __builtin_elementwise_min(f, cdef_s2{(short)maxv, (short)maxv}));
+  }
+  return make_uint2(out[0], out[1]);
+}
+
+/* the same for strengths and dampings whose sums or shifts leave 16 bits (no
+ * stream codes them): one sample and one tap at a time */
+__device__ __forceinline__ uint2 cdef_quad_wide(const CdefPlane& P, int x, int y, const CdefTaps& c, int maxv) {
+  uint32_t out[4];
+#pragma unroll 1
+  for (int i = 0; i < 4; ++i) {
+    const int own = P.src[y * P.stride + x + i];
+    int sum = 0, lo = own, hi = own;
+#pragma unroll 1
+    for (int t = 0; t < 12; ++t) {
+      const int kind = (t >> 1) % 3, far = t >= 6;
+      const int d = (c.dir + (kind == 0 ? 0 : kind == 1 ? 2 : 6)) & 7;
+      int dy = cdef_nibble(far ? kCdefDy1 : kCdefDy0, d), dx = cdef_nibble(far ? kCdefDx1 : kCdefDx0, d);
+      if (t & 1) dy = -dy, dx = -dx;
+      const int tx = x + i + dx, ty = y + dy;
+      if (tx < 0 || ty < 0 || tx >= P.w || ty >= P.h) continue;
+      const int v = P.src[ty * P.stride + tx], mag = abs(v - own);
+      const int con = max(0, min((kind ? c.sec : c.pri) - (mag >> (kind ? c.adjs : c.adjp)), mag));
+      sum += (kind ? 2 - far : far ? c.pt1 : c.pt0) * (v < own ? -con : con);
+      lo = min(lo, v);
+      hi = max(hi, v);
+    }
+    const uint32_t r = clampi(clampi(own + ((8 + sum - (sum < 0)) >> 4), lo, hi), 0, maxv);
+    out[0] = i == 0 ? r : out[0], out[1] = i == 1 ? r : out[1], out[2] = i == 2 ? r : out[2], out[3] = r;
+  }
+  return make_uint2(out[0] | out[1] << 16, out[2] | out[3] << 16);
+}
+
+/* the lane's four samples of set `grp` of blocks first .. first + count - 1 */
+__device__ __forceinline__ void cdef_lane(FArgs a, int first, int count, int grp, bool luma) {
   LayRef L = a.lay;
-  const int sb = lane / S, sm = lane - sb * S, r = sm / W, k = sm - r * W;
-  CdefBlockIn q[kSets];
-  bool live[kSets];
-#pragma unroll
-  for (int u = 0; u < kSets; ++u) {
-    const int b0 = (grp * batch + u) * kPer + wave * kWave;
-    live[u] = u < batch && b0 + sb < count;
-    q[u] = CdefBlockIn{};
-    if (live[u]) q[u] = cdef_block_in<kLuma>(a, first, b0 + sb);
-  }
-#pragma unroll
-  for (int u = 0; u < kSets; ++u) {
-    if (u >= batch) break;
-    const int b0 = (grp * batch + u) * kPer + wave * kWave;
-    uint16_t* ut = wt + u * kCdefTileWave;
-    for (int e = lane; e < kWave * kDw; e += 64) {
-      const int eb = e / kDw, rem = e - eb * kDw, row = rem / kPairs, cp = rem - row * kPairs;
-      uint32_t v = 0xffffffffu;
-      if (b0 + eb < count) {
-        /* a luma wave stages its own block; a chroma lane may stage another */
-        int p = 0, cx = q[u].x, cy = q[u].y;
-        if (!kLuma) {
-          const DevCdef& c = a.plan.cdef[first + b0 + eb];
-          p = c.plane_damping & 3;
-          cx = c.x;
-          cy = c.y;
-        }
-        const int px = cx - 2 + 2 * cp, py = cy - 2 + row;
-        /* grid widths are even: a pair is inside or outside as a whole */
-        if (px >= 0 && px < L.grid_w[p] && py >= 0 && py < L.grid_h[p])
-          v = *reinterpret_cast<const uint32_t*>(a.cdef_src + L.plane_off[p] + (int64_t)py * L.stride[p] + px);
-      }
-      *reinterpret_cast<uint32_t*>(ut + eb * TW * TH + row * TW + 2 * cp) = v;
+  const int ss_x = luma ? 0 : L.ss_x, ss_y = luma ? 0 : L.ss_y;
+  const int lanes = 4 - ss_x - ss_y; /* log2 of a block's lanes */
+  const int bi = (grp << (8 - lanes)) + ((int)threadIdx.x >> lanes);
+  if (bi >= count) return;
+  const uint2 rec = *reinterpret_cast<const uint2*>(a.plan.cdef + first + bi);
+  const int bx = (int)(rec.x & 0xffffu), by = (int)(rec.x >> 16);
+  const int p = luma ? 0 : (int)(rec.y >> 16) & 3, cs = L.bit_depth - 8;
+  CdefTaps c;
+  c.pri = (int)(rec.y & 0xffu) << cs;
+  c.sec = (int)((rec.y >> 8) & 0xffu) << cs;
+  const int damping = (int)((rec.y >> 18) & 0x3fu) + cs - (luma ? 0 : 1);
+  c.dir = (int)rec.y >> 24;
+  if (c.dir < 0) {
+    const int2 m = *reinterpret_cast<const int2*>(
+        a.cdef_dir + 2 * (((by << ss_y) >> 3) * a.cdef_dir_w + ((bx << ss_x) >> 3)));
+    c.dir = c.pri == 0 ? 0 : cdef_uv_dir(ss_x, ss_y, m.x);
+    if (luma) {
+      const int vs = (m.y >> 6) ? min(flog2(m.y >> 6), 12) : 0;
+      c.pri = m.y ? ((c.pri * (4 + vs) + 8) >> 4) : 0;
     }
   }
-  __syncthreads();
-#pragma unroll
-  for (int u = 0; u < kSets; ++u) {
-    int64_t off = 0;
-    int val = 0;
-    if (live[u] &&
-        cdef_tile_sample<W, H, kLuma>(a, q[u], r, k, wt + u * kCdefTileWave + sb * TW * TH, dirs, &off, &val)) {
-      a.cdef_dst[off] = (uint16_t)val;
-      if (a.cdef_dst2) a.cdef_dst2[off] = (uint16_t)val;
-    }
-  }
-  __syncthreads();
+  if (c.pri == 0 && c.sec == 0) return; /* the destination already holds the snapshot's values */
+  c.adjp = c.pri ? max(0, damping - flog2(c.pri)) : 0;
+  c.adjs = c.sec ? max(0, damping - flog2(c.sec)) : 0;
+  const int ts = (c.pri >> cs) & 1;
+  c.pt0 = ts ? 3 : 4;
+  c.pt1 = ts ? 3 : 2;
+  CdefPlane P;
+  P.src = (const AV1H_GLOBAL uint16_t*)(a.cdef_src + L.plane_off[p]);
+  P.stride = L.stride[p];
+  P.w = L.grid_w[p];
+  P.h = L.grid_h[p];
+  const int l = (int)threadIdx.x & ((1 << lanes) - 1);
+  const int x = bx + 4 * (l & (1 - ss_x)), y = by + (l >> (1 - ss_x));
+  uint2 v;
+  /* the weighted sum stays below 12 (pri + sec), a threshold shifted up by
+   * its adjustment below 1 << (damping + 1): 2^15 and 28672 (the distance of
+   * kCdefOutside from a sample) are out of reach */
+  if (12 * (c.pri + c.sec) >= 32752 || damping > 13)
+    v = cdef_quad_wide(P, x, y, c, a.maxv);
+  else if (x < 2 || y < 2 || x + 6 > P.w || y + 3 > P.h)
+    v = cdef_quad<true>(P, x, y, c, a.maxv);
+  else
+    v = cdef_quad<false>(P, x, y, c, a.maxv);
+  const int64_t at = L.plane_off[p] + y * P.stride + x;
+  *reinterpret_cast<uint2*>(a.cdef_dst + at) = v;
+  if (a.cdef_dst2) *reinterpret_cast<uint2*>(a.cdef_dst2 + at) = v;
 }
 
 /* The luma blocks (plane 0) and then the chroma blocks (planes 1 and 2) of
  * every frame in one launch: the luma groups of every frame come first, then
  * the chroma groups (both read the deblocked snapshot and the direction
- * map, and write different planes, so nothing orders them). `batch` sets
- * per workgroup, at most kSets (a kernel per bound: the registers of more
- * sets would lower the occupancy of one). */
-template <int kSets>
+ * map, and write different planes, so nothing orders them). `batch` sets of
+ * 1024 samples per workgroup. */
 __global__ __launch_bounds__(256) void k_cdef(BatchDev B, int batch) {
-  /* the direction table in LDS: lanes index it by their own direction */
-  __shared__ int s_dirs[8][2][2];
-  __shared__ __align__(16) uint16_t s_tile[4 * kCdefTileWave * kSets];
-  if (threadIdx.x < 32) (&s_dirs[0][0][0])[threadIdx.x] = (&kCdefDirs[0][0][0])[threadIdx.x];
-  __syncthreads();
   const AV1H_CMEM int32_t* pre_l = kernel_prefix(B, kKCdefLuma);
   const AV1H_CMEM int32_t* pre_c = kernel_prefix(B, kKCdefChroma);
   const int tl = pre_l[B.njobs], total = tl + pre_c[B.njobs];
   for (int base = 0; base < total; base += gridDim.x) {
     const int v = xcd_group(base, total);
     if (v < 0) continue;
-    if (v < tl) {
-      const int j = find_job(pre_l, B.njobs, v);
-      FArgs a = filter_args(B, j);
-      cdef_tiles<8, 8, true, kSets>(a, 0, a.plan.n_cdef_luma, v - pre_l[j], batch, s_tile, s_dirs);
-      continue;
-    }
-    const int vc = v - tl;
-    const int j = find_job(pre_c, B.njobs, vc);
+    const bool luma = v < tl;
+    const AV1H_CMEM int32_t* pre = luma ? pre_l : pre_c;
+    const int vk = luma ? v : v - tl;
+    const int j = find_job(pre, B.njobs, vk);
     FArgs a = filter_args(B, j);
-    const int nl = a.plan.n_cdef_luma, nc = a.plan.n_cdef - nl, grp = vc - pre_c[j];
-    switch (a.lay.ss_x * 2 + a.lay.ss_y) {
-      case 3: cdef_tiles<4, 4, false, kSets>(a, nl, nc, grp, batch, s_tile, s_dirs); break;
-      case 2: cdef_tiles<4, 8, false, kSets>(a, nl, nc, grp, batch, s_tile, s_dirs); break;
-      case 1: cdef_tiles<8, 4, false, kSets>(a, nl, nc, grp, batch, s_tile, s_dirs); break;
-      default: cdef_tiles<8, 8, false, kSets>(a, nl, nc, grp, batch, s_tile, s_dirs); break;
-    }
+    const int nl = a.plan.n_cdef_luma;
+    for (int u = 0; u < batch; ++u)
+      cdef_lane(a, luma ? 0 : nl, luma ? nl : a.plan.n_cdef - nl, (vk - pre[j]) * batch + u, luma);
   }
 }
 
@@ -1165,12 +1149,7 @@ hipError_t launch_filter_kernel(const BatchDev& b, int k, int total, int cap, in
     case kKCdefDir: hipLaunchKernelGGL(k_cdef_dir, grid, blk, 0, s, b); break;
     case kKCdefLuma:
       /* luma and chroma in one launch (kKCdefLuma's): `total` counts both */
-      if (cdef_batch <= 1)
-        hipLaunchKernelGGL(k_cdef<1>, grid, blk, 0, s, b, 1);
-      else if (cdef_batch == 2)
-        hipLaunchKernelGGL(k_cdef<2>, grid, blk, 0, s, b, 2);
-      else
-        hipLaunchKernelGGL(k_cdef<kCdefMaxBatch>, grid, blk, 0, s, b, cdef_batch);
+      hipLaunchKernelGGL(k_cdef, grid, blk, 0, s, b, cdef_batch);
       break;
     case kKUpscale: hipLaunchKernelGGL(k_upscale, grid, blk, 0, s, b); break;
     case kKLr: hipLaunchKernelGGL(k_lr, grid, blk, 0, s, b); break;

@@ -371,8 +371,7 @@ constexpr size_t kCounterBytes = (size_t)(kTickets + 1) * kTicketStep * 4;
 /* k_inter_special: workgroups (of one wave) that share a block's samples */
 constexpr int kSpecialStrips = 4;
 
-/* CDEF: groups of 256 / (block samples) blocks a workgroup takes per step
- * (a thread's samples of up to kCdefMaxBatch blocks computed together) */
+/* CDEF: sets of 1024 / (block samples) blocks a workgroup takes, at most */
 constexpr int kCdefMaxBatch = 4;
 /* CDEF direction search: luma 8x8 blocks per workgroup (one per lane) */
 constexpr int kCdefDirPerGroup = 256;
