@@ -1,7 +1,8 @@
 """Film grain templates against the oracle, bit exact, where the wavefront of
 one wave can go wrong: every filter lag, shift and noise scale, luma noise
 off, chroma from luma, chroma planes with and without points, 8 to 12 bits, at
-pictures of one and of many noise stripes."""
+pictures of one and of many noise stripes; and its application four samples
+per lane, with and without overlap and the restricted range."""
 import numpy as np
 import pytest
 
@@ -11,12 +12,12 @@ from oracle_lib import OracleDecoder
 pytestmark = pytest.mark.gpu
 
 GRAIN = 16 + 4 * 43  # byte of av1h_grain in a wire frame
-NUM_Y, CFL, NUM_CB, NUM_CR, LAG, SHIFT, SCALE = 2, 35, 36, 69, 103, 178, 179
+NUM_Y, CFL, NUM_CB, NUM_CR, LAG, SHIFT, SCALE, OVERLAP, RESTRICTED = 2, 35, 36, 69, 103, 178, 179, 186, 187
 
 
 def _patched(wire, values):
     b = bytearray(wire)
-    g = np.frombuffer(b, np.int32, 190, GRAIN)
+    g = np.frombuffer(b, np.int32, 188, GRAIN)
     assert g[0] == 1 and g[LAG] == 3  # apply, ar_coeff_lag as generated
     for k, v in values.items():
         g[k] = v
@@ -41,3 +42,17 @@ def test_templates(values):
             slots[f] = s
             for p in range(3):
                 assert np.array_equal(ph[p], po[p]), (depth, f, p, np.argwhere(ph[p] != po[p])[:3].tolist())
+
+
+@pytest.mark.parametrize("values", [{}, {OVERLAP: 0}, {OVERLAP: 1, RESTRICTED: 1}, {OVERLAP: 1, CFL: 1}, {OVERLAP: 1, NUM_Y: 0},
+                                    {OVERLAP: 1, CFL: 0, NUM_CR: 0}], ids=str)
+def test_ragged_pictures(values):
+    """Four samples per lane at right and bottom edges of every remainder."""
+    for depth in (8, 10, 12):
+        for w, h in ((33, 17), (66, 34), (71, 67), (97, 33), (132, 66)):
+            clip = pkg.Clip("c2_mini", 53, frames=1, bit_depth=depth, width=w, height=h, coded_width=0)
+            wire = _patched(clip.wire(0), values)
+            _, got = pkg.HipDecoder().decode_wire(wire)
+            _, want = OracleDecoder().decode_wire(wire)
+            for p in range(3):
+                assert np.array_equal(got[p], want[p]), (depth, w, h, p, np.argwhere(got[p] != want[p])[:3].tolist())
