@@ -487,21 +487,31 @@ __global__ __launch_bounds__(256) void k_cdef(BatchDev B, int batch) {
 
 /* ---- superres (av1gpu_kernels.h:2387-2402) ------------------------------ */
 
-/* 256 x 4 output samples of one plane of one picture per workgroup: the
- * source span of the 256 columns (at most 264 samples when upscaling) is
- * staged in LDS per row, clamped to the coded width as each tap is
- * (av1gpu_kernels.h:2387-2402). Picture 0 is the frame (from the CDEF
- * output in `scratch`; also stored to lr_cdef when loop restoration reads
- * it), picture 1 the deblocked picture loop restoration reads (lr_curr into
- * lr_prev_up). */
-constexpr int kUpW = 256, kUpRows = 8, kUpSpan = 272;
+typedef short lr_s2 __attribute__((ext_vector_type(2)));
+/* two 16-bit products added to acc */
+__device__ __forceinline__ int dot2(uint32_t a, uint32_t b, int acc) {
+  return __builtin_amdgcn_sdot2(__builtin_bit_cast(lr_s2, a), __builtin_bit_cast(lr_s2, b), acc, false);
+}
+__device__ __forceinline__ uint32_t pack2(int lo, int hi) { return (uint32_t)(lo & 0xffff) | ((uint32_t)hi << 16); }
+
+/* 256 x 16 output samples of one plane of one picture per workgroup, four
+ * neighbouring samples of a row per lane: the source span of the 256 columns
+ * (at most 264 samples when upscaling) is staged in LDS per row, eight bytes a
+ * load, clamped to the coded width as each tap is (av1gpu_kernels.h:2387-2402).
+ * A lane's columns stay the same down the rows, so their packed filters and
+ * the shifts that align their taps are set up once. Picture 0 is the frame
+ * (from the CDEF output in `scratch`; also stored to lr_cdef when loop
+ * restoration reads it), picture 1 the deblocked picture loop restoration
+ * reads (lr_curr into lr_prev_up). One sample per lane and row with 32-bit
+ * products took 18 us on a 1080p frame, 57 on a 2160p one; now 12 and 30. */
+constexpr int kUpW = 256, kUpRows = 16, kUpSpan = 280; /* from 3 to 6 samples left of the first tap's column */
 
 /* output tiles of a plane of ow x oh display samples */
 __host__ __device__ __forceinline__ int up_tiles(int ow, int oh) {
   return (ow + kUpW - 1) / kUpW * ((oh + kUpRows - 1) / kUpRows);
 }
 
-__device__ void upscale_tile(FArgs a, int t, const int* s_k, uint16_t (*s_row)[kUpSpan]) {
+__device__ void upscale_tile(FArgs a, int t, const uint4* s_k, uint16_t (*s_row)[kUpSpan]) {
   LayRef L = a.lay;
   const int t0 = up_tiles(L.out_w[0], L.out_h[0]), t1 = up_tiles(L.out_w[1], L.out_h[1]);
   const int tp = t0 + t1 + up_tiles(L.out_w[2], L.out_h[2]);
@@ -518,58 +528,89 @@ __device__ void upscale_tile(FArgs a, int t, const int* s_k, uint16_t (*s_row)[k
   const int ow = L.out_w[p], oh = L.out_h[p];
   const int tx = (ow + kUpW - 1) / kUpW;
   const int by = rem / tx, bx = rem - by * tx;
-  const uint16_t* src = pic ? a.lr_curr : a.scratch;
-  uint16_t* dst = pic ? a.lr_prev_up : a.frame;
+  const uint16_t* src = (pic ? a.lr_curr : a.scratch) + L.plane_off[p];
+  uint16_t* dst = (pic ? a.lr_prev_up : a.frame) + L.plane_off[p];
+  uint16_t* dst2 = pic || !a.up_dst2 ? nullptr : a.up_dst2 + L.plane_off[p];
   const int x0 = bx * kUpW, y0 = by * kUpRows;
   const int step = a.up_step[p], init = a.up_initial[p];
   const int maxx = L.plane_w[p] - 1;
   const int stride = L.stride[p];
-  const int64_t poff = L.plane_off[p];
   const int xl = min(x0 + kUpW, ow) - 1;
-  const int ws = ((-(1 << 14) + init + x0 * step) >> 14) - 3;
+  /* the first tap's column, down to a multiple of 4 */
+  const int ws = (((-(1 << 14) + init + x0 * step) >> 14) - 3) & ~3;
   const int wn = ((-(1 << 14) + init + xl * step) >> 14) + 4 - ws + 1;
   const int rows = min(kUpRows, oh - y0);
   {
     /* all of a thread's loads issued before its LDS writes */
-    constexpr int kPer = (kUpSpan + 255) / 256;
-    uint16_t val[kUpRows][kPer];
+    constexpr int kQuads = kUpSpan / 4, kIt = (kQuads * kUpRows + 255) / 256;
+    uint2 val[kIt];
 #pragma unroll
-    for (int r = 0; r < kUpRows; ++r)
-#pragma unroll
-      for (int u = 0; u < kPer; ++u) {
-        const int c = threadIdx.x + 256 * u;
-        val[r][u] = r < rows && c < wn ? src[poff + (size_t)(y0 + r) * stride + clampi(ws + c, 0, maxx)] : 0;
+    for (int u = 0; u < kIt; ++u) {
+      const int e = (int)threadIdx.x + 256 * u, r = e / kQuads, c = 4 * (e - r * kQuads), x = ws + c;
+      val[u] = make_uint2(0, 0);
+      if (r >= rows || c >= wn) continue;
+      const uint16_t* q = src + (size_t)(y0 + r) * stride;
+      if (x >= 0 && x + 3 <= maxx) {
+        val[u] = *reinterpret_cast<const uint2*>(q + x);
+      } else {
+        val[u].x = pack2(q[clampi(x, 0, maxx)], q[clampi(x + 1, 0, maxx)]);
+        val[u].y = pack2(q[clampi(x + 2, 0, maxx)], q[clampi(x + 3, 0, maxx)]);
       }
+    }
 #pragma unroll
-    for (int r = 0; r < kUpRows; ++r)
-#pragma unroll
-      for (int u = 0; u < kPer; ++u) {
-        const int c = threadIdx.x + 256 * u;
-        if (r < rows && c < wn) s_row[r][c] = val[r][u];
-      }
+    for (int u = 0; u < kIt; ++u) {
+      const int e = (int)threadIdx.x + 256 * u, r = e / kQuads;
+      if (r < kUpRows) *reinterpret_cast<uint2*>(&s_row[r][4 * (e - r * kQuads)]) = val[u];
+    }
   }
   __syncthreads();
-  const int x = x0 + threadIdx.x;
-  if (x > xl) return;
-  const int sx = -(1 << 14) + init + x * step;
-  const int o = (sx >> 14) - 3 - ws;
-  const int* k = s_k + ((sx & ((1 << 14) - 1)) >> 8) * 8;
-  uint16_t* dst2 = pic ? nullptr : a.up_dst2;
-  for (int r = 0; r < rows; ++r) {
-    int sum = 0;
+  const int x = x0 + 4 * ((int)threadIdx.x & 63), n = xl - x + 1;
+  if (n <= 0) return;
+  uint4 k[4];
+  int word[4], sh[4];
 #pragma unroll
-    for (int q = 0; q < 8; ++q) sum += s_row[r][o + q] * k[q];
-    const uint16_t v = (uint16_t)clampi((sum + 64) >> 7, 0, a.maxv);
-    const size_t at = poff + (size_t)(y0 + r) * stride + x;
-    dst[at] = v;
-    if (dst2) dst2[at] = v;
+  for (int i = 0; i < 4; ++i) {
+    const int sx = -(1 << 14) + init + min(x + i, xl) * step;
+    const int o = (sx >> 14) - 3 - ws;
+    k[i] = s_k[(sx & ((1 << 14) - 1)) >> 8];
+    word[i] = o >> 1;
+    sh[i] = (o & 1) * 16;
+  }
+  for (int r = (int)threadIdx.x >> 6; r < rows; r += 4) {
+    int v[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t* w = reinterpret_cast<const uint32_t*>(s_row[r]) + word[i];
+      uint32_t m[5];
+#pragma unroll
+      for (int q = 0; q < 5; ++q) m[q] = w[q];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) m[q] = __builtin_amdgcn_alignbit(m[q + 1], m[q], sh[i]);
+      v[i] = clampi(dot2(m[3], k[i].w, dot2(m[2], k[i].z, dot2(m[1], k[i].y, dot2(m[0], k[i].x, 64)))) >> 7, 0, a.maxv);
+    }
+    const size_t at = (size_t)(y0 + r) * stride + x;
+    if (n >= 4) {
+      const uint2 w = make_uint2(pack2(v[0], v[1]), pack2(v[2], v[3]));
+      *reinterpret_cast<uint2*>(dst + at) = w;
+      if (dst2) *reinterpret_cast<uint2*>(dst2 + at) = w;
+    } else {
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+        if (i < n) {
+          dst[at + i] = (uint16_t)v[i];
+          if (dst2) dst2[at + i] = (uint16_t)v[i];
+        }
+    }
   }
 }
 
 __global__ __launch_bounds__(256) void k_upscale(BatchDev B) {
-  __shared__ int s_k[512];
-  __shared__ uint16_t s_row[kUpRows][kUpSpan];
-  for (int i = threadIdx.x; i < 512; i += 256) s_k[i] = av1t_spec_table[AV1T_OFF_UPSCALE + i];
+  __shared__ uint4 s_k[64]; /* a phase's eight taps, two a word */
+  __shared__ __align__(16) uint16_t s_row[kUpRows][kUpSpan];
+  {
+    const int* q = &av1t_spec_table[AV1T_OFF_UPSCALE + 2 * threadIdx.x];
+    reinterpret_cast<uint32_t*>(s_k)[threadIdx.x] = pack2(q[0], q[1]);
+  }
   __syncthreads();
   const AV1H_CMEM int32_t* pre = kernel_prefix(B, kKUpscale);
   const int total = pre[B.njobs];
@@ -585,13 +626,6 @@ __global__ __launch_bounds__(256) void k_upscale(BatchDev B) {
 /* a2 of the self-guided filter for z = 0 .. 255 (the specification's
  * x_by_xplus1 mapping, av1gpu_kernels.h:2898): z >= 255 gives 256 */
 __device__ __forceinline__ int sgr_a2(int z) { return z == 0 ? 1 : ((z << 8) + z / 2) / (z + 1); }
-
-typedef short lr_s2 __attribute__((ext_vector_type(2)));
-/* two 16-bit products added to acc */
-__device__ __forceinline__ int dot2(uint32_t a, uint32_t b, int acc) {
-  return __builtin_amdgcn_sdot2(__builtin_bit_cast(lr_s2, a), __builtin_bit_cast(lr_s2, b), acc, false);
-}
-__device__ __forceinline__ uint32_t pack2(int lo, int hi) { return (uint32_t)(lo & 0xffff) | ((uint32_t)hi << 16); }
 
 /* Loop restoration of one tile (at most kLrTileCols x kLrTileRows samples of
  * one restoration job, i.e. one unit inside one 64 row stripe) per workgroup,
