@@ -2,15 +2,16 @@
  * Reconstruction kernels for gfx950: prediction + inverse transform + residual.
  *
  * Per frame, in stream order:
- *   k_mc     - motion compensation of every inter block, one thread per
- *              output sample, straight into the frame;
- *   k_itx<G> - every transform block, grouped by its larger side G: G lanes
+ *   k_mc     - motion compensation of every inter block, four neighbouring
+ *              samples per lane, straight into the frame;
+ *   k_itx    - every transform block, grouped by its larger side G: G lanes
  *              per transform. Inter residuals are added into the frame, intra
  *              residuals are kept in a residual plane;
  *   k_queue  - a persistent work queue over the intra blocks: waves take
- *              blocks in coding order, spin on per cell epoch flags until the
- *              cells the block reads are final, predict the block, add its
- *              residual and publish its own cells. This replaces the
+ *              blocks in dependency-level order, poll the packed edge words
+ *              (or per cell epoch flags) of the neighbours a block reads until
+ *              they are final, predict the block, add its residual and publish
+ *              its own edges and cells. This replaces the
  *              reference's host wavefront schedule (src/core/engine.cpp:
  *              695-926): the dependencies are the same cells that scheduler
  *              waits for, but they resolve on the device as soon as each

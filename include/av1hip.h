@@ -436,10 +436,11 @@ void av1h_nv12_pack_release(av1h_ctx* ctx, int handle);
 int av1h_set_decode_nv12(av1h_ctx* ctx, size_t pitch);
 
 /* Captured launches. Mode 1 (the default): the first batch of each frame
- * count and set of kernels with work this context leads records its launch
- * sequence into a HIP graph, each of those kernels at its full persistent
- * grid reading its work counts from the batch's device tables; later
- * batches of that shape replay it with one launch. Mode 2: one graph per
+ * count, set of kernels with work and size class this context leads records
+ * its launch sequence into a HIP graph, each of those kernels at a persistent
+ * grid for its class (small batches take smaller grids) reading its work
+ * counts from the batch's device tables; later batches of that shape replay
+ * it with one launch. Mode 2: one graph per
  * frame count with every kernel launched (kernels without work exit at
  * once), for callers whose batches change shape often (the serving loop's
  * launchers): fewer captures, each replay dispatching every kernel. Mode 0:
@@ -451,7 +452,7 @@ int av1h_set_graphs(av1h_ctx* ctx, int mode);
 /* Launch shapes of the batches this context leads, the parameters an
  * autotuner searches (av1ongpu_amd/autotune.py does): for every kernel the
  * persistent workgroups per compute unit of its grid, the queue's, and the
- * sets of CDEF blocks a workgroup stages together (1..4); CDEF's chroma
+ * sets of CDEF blocks a workgroup takes one after the other (1..4); CDEF's chroma
  * blocks run in the luma launch, so "cdef_chroma" has no effect.
  * av1h_tune_params gives
  * their count and av1h_tune_name their names; setting them drops the
