@@ -90,23 +90,17 @@ struct StepLds {
   float w3[kH], b2[kH], y[kBatch], b3, loss[16];
 };
 
-/* Steps over the samples in `perm` order, kBatch at a time, by workgroups of
- * 16 waves that each own one 16x16 tile of every 64x64 product. What bounds a
- * step is one compute unit's matrix rate (992 tiles of 16x16x4, 3.3 us) and
- * its five barriers: training is a chain of Adam steps, so it has one
- * workgroup. Weights, Adam's moments (kTrain) or the gradient sums stay in
- * registers across steps, activations in LDS, both ways round where a product
- * contracts them; the next step's samples load during this one. With 256
- * threads and scalar FMAs from LDS a step took 107 us; two epochs over 8192
- * samples, host work included, 27.4 -> 2.6 ms, the gradient over them 13.3 ->
- * 0.36 ms.
- *   kTrain: an Adam step per batch (gradient of the batch mean), one workgroup.
- *   else: batch i to workgroup i % gridDim.x, whose sums of the gradient of the
- *   mean squared error over all n samples go to part[workgroup]. */
-template <bool kTrain>
-__global__ __launch_bounds__(kSteps) void k_mlp_step(float* params, float* part, float* am, float* av, const float* X,
-                                                    const float* Y, const int32_t* perm, int n, Adam adam,
-                                                    float* loss) {
+/* The gradient of the mean squared error over all n samples: batch i of
+ * kBatch samples (in `perm` order) to workgroup i % gridDim.x of 16 waves that
+ * each own one 16x16 tile of every 64x64 product; a workgroup's sums go to
+ * part[workgroup]. What bounds a batch is one compute unit's matrix rate (992
+ * tiles of 16x16x4, 3.3 us) and its five barriers. Weights and sums stay in
+ * registers or LDS, activations in LDS both ways round where a product
+ * contracts them; the next batch's samples load during this one. With one
+ * workgroup of 256 threads and scalar FMAs the gradient over 8192 samples took
+ * 13.3 ms; now 0.36. */
+__global__ __launch_bounds__(kSteps) void k_mlp_grad(const float* params, float* part, const float* X,
+                                                    const float* Y, const int32_t* perm, int n, float* loss) {
   __shared__ __align__(16) StepLds L;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, col = lane & 15, g = lane >> 4;
   const int ts = wave >> 2, to = wave & 3;
@@ -132,27 +126,6 @@ __global__ __launch_bounds__(kSteps) void k_mlp_step(float* params, float* part,
     L.b2[tid] = params[kB2 + tid];
   }
   if (tid == 0) L.b3 = params[kB3];
-  f4 w2 = {}, m2 = {}, v2 = {}, w1 = {}, m1 = {}, v1 = {};
-  float w3 = 0.f, m3 = 0.f, v3 = 0.f;
-  if (kTrain) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int p = kW2 + (ow + r) * kH + iw;
-      w2[r] = params[p];
-      m2[r] = am[p];
-      v2[r] = av[p];
-      if (has1) {
-        w1[r] = params[p1 + r * s1];
-        m1[r] = am[p1 + r * s1];
-        v1[r] = av[p1 + r * s1];
-      }
-    }
-    if (has3) {
-      w3 = params[p3];
-      m3 = am[p3];
-      v3 = av[p3];
-    }
-  }
   /* a batch's samples: 16 threads each, features c and c + 16 */
   const int xs = tid >> 4, xc = tid & 15;
   const int nbatch = (n + kBatch - 1) / kBatch, hop = (int)gridDim.x;
@@ -179,7 +152,6 @@ __global__ __launch_bounds__(kSteps) void k_mlp_step(float* params, float* part,
   const float* arow_x = L.x + (ts * 16 + col) * kLx + 4 * g;
   const float* brow_w1 = L.w1 + (to * 16 + col) * kLx + 4 * g;
   const int arow = (ts * 16 + col) * kLd + 4 * g, brow = (to * 16 + col) * kLd + 4 * g;
-  int step = adam.t0;
   __syncthreads();
   for (; bi < nbatch; bi += hop) {
     const int nb = min(kBatch, n - bi * kBatch);
@@ -208,7 +180,7 @@ __global__ __launch_bounds__(kSteps) void k_mlp_step(float* params, float* part,
     /* the error and its gradients at the outputs of both layers */
     f4 d3 = ld4(&L.out[ow]) + ld4(&L.out[kBatch + ow]) + ld4(&L.out[2 * kBatch + ow]) + ld4(&L.out[3 * kBatch + ow]);
     const f4 y = ld4(&L.y[ow]);
-    const float scale = kTrain ? 2.f / (float)nb : 2.f / (float)n, b3 = L.b3;
+    const float scale = 2.f / (float)n, b3 = L.b3;
     f4 d2;
     float s3 = 0.f, s2 = 0.f, s0 = 0.f;
 #pragma unroll
@@ -237,82 +209,27 @@ __global__ __launch_bounds__(kSteps) void k_mlp_step(float* params, float* part,
 #pragma unroll
     for (int r = 0; r < 4; ++r) d1[r] = h1[r] > 0.f ? d1[r] : 0.f;
     st4(&L.h1[iw * kLd + ow], d1); /* d1 transposed: h1 was last read two barriers ago */
-    g2 = tile<4>(L.d2t + arow, L.h1t + brow, kTrain ? f4{} : g2);
+    g2 = tile<4>(L.d2t + arow, L.h1t + brow, g2);
     __syncthreads();
     /* the gradient of W1 and b1 */
     if (wave < 8)
-      g1 = tile<4>(L.h1 + ((wave >> 1) * 16 + col) * kLd + 4 * g, L.xt[buf] + c1 * kLd + 4 * g, kTrain ? f4{} : g1);
+      g1 = tile<4>(L.h1 + ((wave >> 1) * 16 + col) * kLd + 4 * g, L.xt[buf] + c1 * kLd + 4 * g, g1);
     if (has3) {
       const float* q = wave == 8 ? L.gw3 + lane : wave == 9 ? L.gb2 + lane : L.gb3;
       const int hopq = wave == 10 ? 1 : kH;
-      const float s = q[0] + q[hopq] + q[2 * hopq] + q[3 * hopq];
-      g3 = kTrain ? s : g3 + s;
-    }
-    if (kTrain) {
-      ++step;
-      const float c1m = 1.f - powf(adam.b1, (float)step), c2m = 1.f - powf(adam.b2, (float)step);
-      auto update = [&](float& w, float& m, float& v, float gr) {
-        m = adam.b1 * m + (1.f - adam.b1) * gr;
-        v = adam.b2 * v + (1.f - adam.b2) * gr * gr;
-        w -= adam.lr * (m / c1m) / (sqrtf(v / c2m) + adam.eps);
-      };
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        float w = w2[r], m = m2[r], v = v2[r];
-        update(w, m, v, g2[r]);
-        w2[r] = w;
-        m2[r] = m;
-        v2[r] = v;
-        L.w2[(ow + r) * kLd + iw] = w;
-      }
-      st4(&L.w2t[iw * kLd + ow], w2);
-      if (has1) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          float w = w1[r], m = m1[r], v = v1[r];
-          update(w, m, v, g1[r]);
-          w1[r] = w;
-          m1[r] = m;
-          v1[r] = v;
-          L.w1[(o1 + r) * kLx + c1] = w;
-        }
-      }
-      if (has3) {
-        update(w3, m3, v3, g3);
-        (wave == 8 ? L.w3[lane] : wave == 9 ? L.b2[lane] : L.b3) = w3;
-      }
+      g3 += q[0] + q[hopq] + q[2 * hopq] + q[3 * hopq];
     }
     buf ^= 1;
     stage(buf);
     __syncthreads();
   }
-  if (kTrain) {
+  float* to_part = part + (size_t)blockIdx.x * kParams;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int p = kW2 + (ow + r) * kH + iw;
-      params[p] = w2[r];
-      am[p] = m2[r];
-      av[p] = v2[r];
-      if (has1) {
-        params[p1 + r * s1] = w1[r];
-        am[p1 + r * s1] = m1[r];
-        av[p1 + r * s1] = v1[r];
-      }
-    }
-    if (has3) {
-      params[p3] = w3;
-      am[p3] = m3;
-      av[p3] = v3;
-    }
-  } else {
-    float* to_part = part + (size_t)blockIdx.x * kParams;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      to_part[kW2 + (ow + r) * kH + iw] = g2[r];
-      if (has1) to_part[p1 + r * s1] = g1[r];
-    }
-    if (has3) to_part[p3] = g3;
+  for (int r = 0; r < 4; ++r) {
+    to_part[kW2 + (ow + r) * kH + iw] = g2[r];
+    if (has1) to_part[p1 + r * s1] = g1[r];
   }
+  if (has3) to_part[p3] = g3;
   if (to == 0 && col == 0) L.loss[ts * 4 + g] = sq;
   __syncthreads();
   if (tid == 0) {
@@ -320,6 +237,182 @@ __global__ __launch_bounds__(kSteps) void k_mlp_step(float* params, float* part,
     for (int i = 0; i < 16; ++i) s += L.loss[i];
     loss[blockIdx.x] = s / (float)n;
   }
+}
+
+struct TrainLds {
+  float w1[kH * 28], w2[kH * kLd];
+  float h1[kBatch * kLd], h2[kBatch * kLd], d1[kBatch * kLd], d2[kBatch * kLd];
+  float x[kBatch * 28], d3[kBatch], y[kBatch];
+  float b1[kH], b2[kH], w3[kH], b3, loss;
+};
+
+/* An epoch: an Adam step per batch of kBatch samples in `perm` order (gradient
+ * of the batch mean), one workgroup, as the steps are a chain. Adam divides by
+ * the gradients' own size, so one rounded otherwise where it is close to zero
+ * moves its weight by up to the learning rate: every sum here is one chain of
+ * FMAs in the order of its index, and the matrix cores, whose sums are grouped
+ * by four, are left to the gradient and the predictions. Sixteen threads per
+ * sample, four neurons each; a thread's parameters (four of one column of W2
+ * and one or two others) and their moments stay in registers, operands come
+ * from LDS four floats a read. What bounds a step is LDS reads and its six
+ * barriers. With 256 threads and a read per product a step took 107 us; two
+ * epochs over 8192 samples, host work included, 27.4 ms -> 6.1. */
+__global__ __launch_bounds__(kSteps) void k_mlp_train(float* params, float* am, float* av, const float* X, const float* Y,
+                                                     const int32_t* perm, int n, Adam adam, float* loss) {
+  __shared__ __align__(16) TrainLds L;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, s = tid >> 4, q = tid & 15;
+  for (int i = tid; i < kH * kIn; i += kSteps) L.w1[i / kIn * 28 + i % kIn] = params[kW1 + i];
+  for (int i = tid; i < kH * kH; i += kSteps) L.w2[(i >> 6) * kLd + (i & 63)] = params[kW2 + i];
+  if (tid < kH) {
+    L.b1[tid] = params[kB1 + tid];
+    L.b2[tid] = params[kB2 + tid];
+    L.w3[tid] = params[kW3 + tid];
+  }
+  if (tid == 0) {
+    L.b3 = params[kB3];
+    L.loss = 0.f;
+  }
+  /* this thread's parameters: W2[4 wave + r][lane], W1[lane][wave], and by
+   * wave W1[lane][wave + 16] (0-7), b1 (8), b2 (9), W3 (10), b3 (11, one lane) */
+  int pi[6];
+  float* pw[6];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    pi[r] = kW2 + (4 * wave + r) * kH + lane;
+    pw[r] = L.w2 + (4 * wave + r) * kLd + lane;
+  }
+  pi[4] = kW1 + lane * kIn + wave;
+  pw[4] = L.w1 + lane * 28 + wave;
+  const bool has5 = wave < 11 || (wave == 11 && lane == 0);
+  pi[5] = wave < 8 ? pi[4] + 16 : wave == 8 ? kB1 + lane : wave == 9 ? kB2 + lane : wave == 10 ? kW3 + lane : kB3;
+  pw[5] = wave < 8 ? pw[4] + 16 : wave == 8 ? L.b1 + lane : wave == 9 ? L.b2 + lane : wave == 10 ? L.w3 + lane : &L.b3;
+  float m[6], v[6];
+#pragma unroll
+  for (int k = 0; k < 6; ++k) {
+    m[k] = am[pi[k]];
+    v[k] = av[pi[k]];
+  }
+  /* the next step's samples load during this one */
+  float fx0 = 0.f, fx1 = 0.f, fy = 0.f;
+  auto fetch = [&](int base) {
+    const int row = base < n && base + s < n ? perm[base + s] : -1;
+    fx0 = row >= 0 ? X[(size_t)row * kIn + q] : 0.f;
+    fx1 = row >= 0 && q < kIn - 16 ? X[(size_t)row * kIn + 16 + q] : 0.f;
+    fy = row >= 0 && q == 0 ? Y[row] : 0.f;
+  };
+  fetch(0);
+  int step = adam.t0;
+  for (int base = 0; base < n; base += kBatch) {
+    const int nb = min(kBatch, n - base);
+    L.x[s * 28 + q] = fx0;
+    if (q < kIn - 16) L.x[s * 28 + 16 + q] = fx1;
+    if (q == 0) L.y[s] = fy;
+    __syncthreads();
+    fetch(base + kBatch);
+    float z[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) z[j] = L.b1[q + 16 * j];
+#pragma unroll
+    for (int i = 0; i < kIn; i += 4) {
+      const f4 x = ld4(L.x + s * 28 + i);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const f4 w = ld4(L.w1 + (q + 16 * j) * 28 + i);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) z[j] += w[t] * x[t];
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) L.h1[s * kLd + q + 16 * j] = z[j] > 0.f ? z[j] : 0.f;
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 4; ++j) z[j] = L.b2[q + 16 * j];
+#pragma unroll 4
+    for (int i = 0; i < kH; i += 4) {
+      const f4 h = ld4(L.h1 + s * kLd + i);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const f4 w = ld4(L.w2 + (q + 16 * j) * kLd + i);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) z[j] += w[t] * h[t];
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      z[j] = z[j] > 0.f ? z[j] : 0.f;
+      L.h2[s * kLd + q + 16 * j] = z[j];
+    }
+    __syncthreads();
+    if (q == 0) {
+      float out = L.b3;
+#pragma unroll
+      for (int i = 0; i < kH; i += 4) {
+        const f4 h = ld4(L.h2 + s * kLd + i), w = ld4(L.w3 + i);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) out += w[t] * h[t];
+      }
+      const float e = s < nb ? out - L.y[s] : 0.f;
+      L.d3[s] = e * (2.f / (float)nb);
+      if (s < nb) atomicAdd(&L.loss, e * e);
+    }
+    __syncthreads();
+    const float e3 = L.d3[s];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) L.d2[s * kLd + q + 16 * j] = z[j] > 0.f ? L.w3[q + 16 * j] * e3 : 0.f;
+    __syncthreads();
+    {
+      f4 g = {};
+#pragma unroll 4
+      for (int o = 0; o < kH; o += 4) {
+        const f4 d = ld4(L.d2 + s * kLd + o);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          const f4 w = ld4(L.w2 + (o + t) * kLd + 4 * q);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) g[r] += w[r] * d[t];
+        }
+      }
+      const f4 h = ld4(L.h1 + s * kLd + 4 * q);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) g[r] = h[r] > 0.f ? g[r] : 0.f;
+      st4(L.d1 + s * kLd + 4 * q, g);
+    }
+    __syncthreads();
+    float g[6] = {};
+#pragma unroll 4
+    for (int b = 0; b < nb; ++b) {
+      const f4 d2 = ld4(L.d2 + b * kLd + 4 * wave);
+      const float h = L.h1[b * kLd + lane], d1 = L.d1[b * kLd + lane];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) g[r] += d2[r] * h;
+      g[4] += d1 * L.x[b * 28 + wave];
+      if (wave < 8) g[5] += d1 * L.x[b * 28 + 16 + wave];
+      if (wave == 8) g[5] += d1;
+      if (wave == 9) g[5] += L.d2[b * kLd + lane];
+      if (wave == 10) g[5] += L.d3[b] * L.h2[b * kLd + lane];
+      if (wave == 11) g[5] += L.d3[b];
+    }
+    ++step;
+    const float c1 = 1.f - powf(adam.b1, (float)step), c2 = 1.f - powf(adam.b2, (float)step);
+#pragma unroll
+    for (int k = 0; k < 6; ++k) {
+      if (k == 5 && !has5) break;
+      m[k] = adam.b1 * m[k] + (1.f - adam.b1) * g[k];
+      v[k] = adam.b2 * v[k] + (1.f - adam.b2) * g[k] * g[k];
+      const float mh = m[k] / c1;
+      const float vh = v[k] / c2;
+      *pw[k] -= adam.lr * mh / (sqrtf(vh) + adam.eps);
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int k = 0; k < 6; ++k) {
+    if (k == 5 && !has5) break;
+    params[pi[k]] = *pw[k];
+    am[pi[k]] = m[k];
+    av[pi[k]] = v[k];
+  }
+  if (tid == 0) *loss = L.loss / (float)n;
 }
 
 /* The gradient and the loss from the workgroups' sums. */
@@ -339,7 +432,7 @@ __global__ __launch_bounds__(kThreads) void k_mlp_sum(const float* part, const f
 }
 
 /* Inference, a wave per 16 samples: standardise, forward on the matrix cores
- * (k_mlp_step's tiles, weights read from the L2 by the lanes that use them,
+ * (k_mlp_grad's tiles, weights read from the L2 by the lanes that use them,
  * hidden activations turned through LDS), back to microseconds. One thread
  * per sample left 2040 samples on 8 compute units with 64 x 64 scalar FMAs
  * one after another: a call of 2040 samples, with the pinned staging, 76 ->
@@ -647,8 +740,8 @@ int av1h_cm_gradients(av1h_costmodel* m, const float* features, const float* y_u
   const int rc = d.make(xs, ys, groups, groups + 1);
   if (rc != AV1H_OK) return rc;
   CM_OK(hipMemcpy(d.perm[0], perm.data(), perm.size() * 4, hipMemcpyHostToDevice));
-  hipLaunchKernelGGL(k_mlp_step<false>, dim3(groups), dim3(kSteps), 0, m->stream, m->params, d.part, m->adam,
-                     m->adam + kParams, d.x, d.y, d.perm[0], (int)n, Adam{0.f, 0.f, 0.f, 0.f, 0}, d.loss);
+  hipLaunchKernelGGL(k_mlp_grad, dim3(groups), dim3(kSteps), 0, m->stream, m->params, d.part, d.x, d.y, d.perm[0],
+                     (int)n, d.loss);
   CM_OK(hipGetLastError());
   hipLaunchKernelGGL(k_mlp_sum, dim3((kParams + kThreads - 1) / kThreads), dim3(kThreads), 0, m->stream, d.part, d.loss,
                      groups, d.grad, d.loss + groups);
@@ -704,8 +797,8 @@ int av1h_cm_train(av1h_costmodel* m, const float* features, const float* y_us, i
         hipStreamSynchronize(m->stream) != hipSuccess)
       break;
     const Adam a{lr, 0.9f, 0.999f, 1e-8f, m->steps};
-    hipLaunchKernelGGL(k_mlp_step<true>, dim3(1), dim3(kSteps), 0, m->stream, m->params, d.part, m->adam,
-                       m->adam + kParams, d.x, d.y, dp, (int)n, a, d.loss + done);
+    hipLaunchKernelGGL(k_mlp_train, dim3(1), dim3(kSteps), 0, m->stream, m->params, m->adam, m->adam + kParams, d.x,
+                       d.y, dp, (int)n, a, d.loss + done);
     if (hipGetLastError() != hipSuccess) break;
     m->steps += (int)((n + kBatch - 1) / kBatch);
   }
