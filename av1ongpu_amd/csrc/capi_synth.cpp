@@ -34,6 +34,8 @@ int av1s_config_set(void* h, const char* key, double v) {
   if (k == "width") c->width = i;
   else if (k == "height") c->height = i;
   else if (k == "bit_depth") c->bit_depth = i;
+  else if (k == "ss_x") c->ss_x = i;
+  else if (k == "ss_y") c->ss_y = i;
   else if (k == "coded_width") c->coded_width = i;
   else if (k == "frames") c->frames = i;
   else if (k == "num_refs") c->num_refs = i;

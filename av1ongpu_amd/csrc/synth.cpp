@@ -125,8 +125,8 @@ class FrameBuilder {
     fs_.height = c.height;
     fs_.coded_width = c.coded_width > 0 && c.coded_width < c.width ? c.coded_width : 0;
     fs_.bit_depth = c.bit_depth;
-    fs_.ss_x = 1;
-    fs_.ss_y = 1;
+    fs_.ss_x = c.ss_x;
+    fs_.ss_y = c.ss_y;
     fs_.base_q_idx = rng_.range(20, 200);
     fs_.sharpness = rng_.range(0, 7);
     fs_.enable_intra_edge_filter = c.contract_tools ? rng_.chance(0.8) : true;
@@ -137,8 +137,8 @@ class FrameBuilder {
     grid_w_ = (coded_w_ + 7) & ~7;
     grid_h_ = (c.height + 7) & ~7;
     planes_[0].init(grid_w_, grid_h_);
-    planes_[1].init(grid_w_ >> 1, grid_h_ >> 1);
-    planes_[2].init(grid_w_ >> 1, grid_h_ >> 1);
+    planes_[1].init(grid_w_ >> c.ss_x, grid_h_ >> c.ss_y);
+    planes_[2].init(grid_w_ >> c.ss_x, grid_h_ >> c.ss_y);
   }
 
   FrameSyntax build() {
@@ -179,6 +179,10 @@ class FrameBuilder {
   bool steps_ready_ = false; /* levels: the frame's steps and matrices are drawn */
   int dc_step_ = 0, ac_step_ = 0;
   PlaneState planes_[3];
+
+  /* log2 of a plane's subsampling */
+  int ssx(int plane) const { return plane ? cfg_.ss_x : 0; }
+  int ssy(int plane) const { return plane ? cfg_.ss_y : 0; }
 
   void partition(int x, int y, int size) {
     if (x >= grid_w_ || y >= grid_h_) return;
@@ -343,7 +347,7 @@ class FrameBuilder {
   void tx_size_for(int plane, int w, int h, bool intra, int* tw, int* th) {
     const int cap = std::min(cfg_.max_tx, plane ? 32 : 64);
     if (plane) {
-      /* the chroma transform is the largest that fits (4:2:0, capped at 32) */
+      /* the chroma transform is the largest that fits (capped at 32) */
       if (cfg_.rect_tx && (w == 2 * h || h == 2 * w) && w <= cap && h <= cap) {
         *tw = w;
         *th = h;
@@ -382,16 +386,14 @@ class FrameBuilder {
       const int uvangle = (uvmode >= 1 && uvmode <= 8) ? rng_.range(-3, 3) : 0;
       const int cfl_alpha = rng_.range(-16, 16);
       for (int p = 1; p < 3; ++p)
-        intra_block(p, x >> 1, y >> 1, w >> 1, h >> 1, uvmode, uvangle, level, lossless,
+        intra_block(p, x >> ssx(p), y >> ssy(p), w >> ssx(p), h >> ssy(p), uvmode, uvangle, level, lossless,
                     cfl_alpha, raw);
     } else {
       InterParams ip = draw_inter();
       if (cfg_.inter_tools > 0 && w >= 8 && h >= 8 && w <= 32 && h <= 32 && rng_.chance(cfg_.inter_tools))
         draw_tool(&ip, w, h);
-      for (int p = 0; p < 3; ++p) {
-        const int s = p ? 1 : 0;
-        inter_block(p, x >> s, y >> s, w >> s, h >> s, ip, level, raw);
-      }
+      for (int p = 0; p < 3; ++p)
+        inter_block(p, x >> ssx(p), y >> ssy(p), w >> ssx(p), h >> ssy(p), ip, level, raw);
     }
   }
 
@@ -471,10 +473,8 @@ class FrameBuilder {
     ip.mv[0][0] = (sx - x) * 8;
     ip.mv[0][1] = -64 * 8;
     ip.intrabc = true;
-    for (int p = 0; p < 3; ++p) {
-      const int s = p ? 1 : 0;
-      inter_block(p, x >> s, y >> s, w >> s, h >> s, ip, level, raw);
-    }
+    for (int p = 0; p < 3; ++p)
+      inter_block(p, x >> ssx(p), y >> ssy(p), w >> ssx(p), h >> ssy(p), ip, level, raw);
   }
 
   void intra_block(int plane, int x, int y, int w, int h, int mode, int angle, int level,
@@ -626,13 +626,12 @@ class FrameBuilder {
       b.warp[0] = true;
       for (int k = 0; k < 6; ++k) b.warp_params[0][k] = ip.warp_params[k];
     }
-    const int sh = plane ? 1 : 0;
     for (const ObmcCandidate& c : ip.obmc) {
       ObmcCandidate o = c;
-      o.x >>= sh;
-      o.y >>= sh;
-      o.w >>= sh;
-      o.h >>= sh;
+      o.x >>= ssx(plane);
+      o.y >>= ssy(plane);
+      o.w >>= ssx(plane);
+      o.h >>= ssy(plane);
       b.obmc.push_back(o);
     }
     for (int ty = 0; ty < h; ty += th)
@@ -731,8 +730,8 @@ class FrameBuilder {
         for (int p = 1; p < 3; ++p) {
           CdefBlock u = c;
           u.plane = p;
-          u.x = x >> 1;
-          u.y = y >> 1;
+          u.x = x >> ssx(p);
+          u.y = y >> ssy(p);
           u.pri_strength = s.uvpri;
           u.sec_strength = s.uvsec;
           fs_.cdef.push_back(u);
@@ -744,12 +743,11 @@ class FrameBuilder {
 
   void build_lr() {
     for (int plane = 0; plane < 3; ++plane) {
-      const int s = plane ? 1 : 0;
       const int l0 = cfg_.lr_log2 > 0 ? cfg_.lr_log2 : 6;
       const int log2 = plane ? std::max(5, l0 - 1) : l0;
       const int unit = 1 << log2;
-      const int pw = (cfg_.width + s) >> s;
-      const int ph = (cfg_.height + s) >> s;
+      const int pw = (cfg_.width + ssx(plane)) >> ssx(plane);
+      const int ph = (cfg_.height + ssy(plane)) >> ssy(plane);
       const int cols = count_units(unit, pw), rows = count_units(unit, ph);
       fs_.restoration_type[plane] = cfg_.lr == 1 ? kRestoreWiener : kRestoreSwitchable;
       fs_.restoration_unit_log2[plane] = log2;

@@ -32,6 +32,7 @@ struct Config {
   int width = 1280;
   int height = 720;
   int bit_depth = 8;
+  int ss_x = 1, ss_y = 1;    /* chroma subsampling: 1,1 4:2:0  1,0 4:2:2  0,0 4:4:4 */
   int coded_width = 0;       /* superres: the width the tiles code (0 = none)     */
   int frames = 30;
   int num_refs = 1;          /* 1: the previous frame; 3: hierarchical mini-GOPs  */
