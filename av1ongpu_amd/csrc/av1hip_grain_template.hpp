@@ -150,7 +150,10 @@ __device__ __forceinline__ void plane(const AV1H_CMEM DevGrain& g, const AV1H_CM
         st = next_in ? drawn : st;
         next = gauss[(st >> 5) & 2047];
         if (from_luma) {
-          const int lx = max(0, min(((x - 3) << ss_x) + 3, kLumaW - 2)), ly = max(0, min(((row - 3) << ss_y) + 3, kLumaH - 2));
+          /* clamped for the lanes outside the filter's reach only: the last
+           * luma row or column is read where a plane isn't subsampled */
+          const int lx = max(0, min(((x - 3) << ss_x) + 3, kLumaW - 1 - ss_x)),
+                    ly = max(0, min(((row - 3) << ss_y) + 3, kLumaH - 1 - ss_y));
           const int16_t* q = s_luma + ly * kLumaW + lx;
           l0 = q[0];
           if (ss_x) l1 = q[1];

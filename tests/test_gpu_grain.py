@@ -56,3 +56,22 @@ def test_ragged_pictures(values):
             _, want = OracleDecoder().decode_wire(wire)
             for p in range(3):
                 assert np.array_equal(got[p], want[p]), (depth, w, h, p, np.argwhere(got[p] != want[p])[:3].tolist())
+
+
+def _equal(wire, *where):
+    _, got = pkg.HipDecoder().decode_wire(wire)
+    _, want = OracleDecoder().decode_wire(wire)
+    for p in range(3):
+        assert np.array_equal(got[p], want[p]), (*where, p, np.argwhere(got[p] != want[p])[:3].tolist())
+
+
+@pytest.mark.parametrize("ss", [(1, 0), (0, 0)], ids=["422", "444"])
+@pytest.mark.parametrize("values", [{}, {LAG: 1}, {CFL: 1}, {CFL: 0, NUM_CB: 0}, {NUM_Y: 0}, {OVERLAP: 0}], ids=str)
+def test_other_formats(values, ss):
+    """Chroma templates of 73 rows, whose last row lies under the last luma
+    row; the overlap of two stripes reads it where a block's vertical offset
+    is the largest, one block in sixteen."""
+    for depth, w, h in ((8, 200, 330), (10, 331, 203), (12, 90, 330)):
+        for seed in (67, 68):
+            clip = pkg.Clip("c2_mini", seed, frames=1, bit_depth=depth, width=w, height=h, coded_width=0, ss_x=ss[0], ss_y=ss[1])
+            _equal(_patched(clip.wire(0), {OVERLAP: 1, **values}), depth, seed)
