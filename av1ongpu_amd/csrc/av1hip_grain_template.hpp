@@ -69,7 +69,6 @@ __device__ __forceinline__ unsigned row_state(const Jump& m, unsigned seed, int 
 }
 
 __device__ __forceinline__ int clip(int v, int lo, int hi) { return v < lo ? lo : (v > hi ? hi : v); }
-__device__ __forceinline__ int round_shift(int v, int n) { return n <= 0 ? v : (v + (1 << (n - 1))) >> n; }
 /* the value of the lane above (lane 0: lane 63, whose row 63 it follows) */
 __device__ __forceinline__ int from_above(int v) { return __builtin_amdgcn_mov_dpp(v, 0x13c, 0xf, 0xf, false); }
 
@@ -92,8 +91,9 @@ __device__ __forceinline__ void plane(const AV1H_CMEM DevGrain& g, const AV1H_CM
   const int lane = threadIdx.x & 63;
   const int bd = g.bit_depth;
   const int lo = -(128 << (bd - 8)), hi = (256 << (bd - 8)) - 1 - (128 << (bd - 8));
-  const int shift = g.shift, half = 1 << (shift - 1); /* 6 .. 9 */
-  const int nshift = g.scale_shift, nhalf = nshift > 0 ? 1 << (nshift - 1) : 0;
+  /* 6 .. 9 and 0 .. 7 in a stream; below 1 nothing is shifted or rounded */
+  const int shift = max(g.shift, 0), half = (1 << shift) >> 1;
+  const int nshift = max(g.scale_shift, 0), nhalf = (1 << nshift) >> 1;
   /* pairs of coefficients: per row above (2 kLag + 1 columns) kLag pairs from
    * the right and the leftmost alone; of the own row's kLag likewise */
   constexpr int kCols = 2 * kLag + 1, kTaps = kCols * kLag + kLag;
@@ -238,7 +238,7 @@ __device__ __forceinline__ void template_half(FArgs a, int half, void* lds) {
     }
   }
   /* luma noise, a row per lane (av1gpu_kernels.h:3070-3079) */
-  const int nshift = g.scale_shift, nhalf = nshift > 0 ? 1 << (nshift - 1) : 0;
+  const int nshift = max(g.scale_shift, 0), nhalf = (1 << nshift) >> 1;
   for (int row = lane; row < kLumaH; row += 64) {
     unsigned st = row_state(kJump82, seed, row);
     int16_t* to = s_luma + row * kLumaW;

@@ -75,3 +75,11 @@ def test_other_formats(values, ss):
         for seed in (67, 68):
             clip = pkg.Clip("c2_mini", seed, frames=1, bit_depth=depth, width=w, height=h, coded_width=0, ss_x=ss[0], ss_y=ss[1])
             _equal(_patched(clip.wire(0), {OVERLAP: 1, **values}), depth, seed)
+
+
+@pytest.mark.parametrize("values", [{SHIFT: -6}, {SHIFT: -9, LAG: 1}, {SCALE: -4}, {SCALE: -9, SHIFT: -7, LAG: 2}], ids=str)
+def test_shifts_of_nothing(values):
+    """Shifts of zero and below leave a value as it is."""
+    for depth in (8, 10, 12):
+        clip = pkg.Clip("c2_mini", 71, frames=1, bit_depth=depth, width=120, height=72, coded_width=0)
+        _equal(_patched(clip.wire(0), {OVERLAP: 1, **values}), depth)
