@@ -2,8 +2,8 @@
 
 Every kernel of a batch runs as a persistent grid of (workgroups per compute
 unit x compute units) workgroups that walk the batch's virtual workgroups;
-the dependency queue has its own grid; CDEF can stage 1 to 4 sets of blocks per
-workgroup. The best values depend on the batch (frame sizes, tools) and the
+the dependency queue has its own grid; a CDEF workgroup takes 1 to 4 sets of
+blocks one after the other. The best values depend on the batch (frame sizes, tools) and the
 device, so they are measured: coordinate descent over the parameters, each
 candidate timed on the caller's own batches (replayed, captured launches
 included), keeping a change only when it is faster by more than `tol`.
@@ -14,6 +14,9 @@ from . import decode_planned_batch
 
 CANDIDATES = {"cdef_blocks_per_thread": (1, 2, 4), "queue": (2, 4, 6, 8, 12), "grain_template": (1, 2)}
 DEFAULT_CANDIDATES = (2, 4, 8, 16, 32)
+# kernels whose work rides in another's launch, whose grid counts: CDEF's chroma
+# blocks in the luma launch, the intra transforms in the inter ones'
+INERT = ("cdef_chroma", "itx_intra", "itx_intra_large")
 
 
 def _time_batches(decoders, batches, reps):
@@ -39,8 +42,7 @@ def tune(decoders, batches, params=None, reps=2, tol=0.01, log=None):
     seconds)."""
     lead = decoders[0]
     cur = lead.tuning()
-    # CDEF's chroma blocks run in the luma launch: its own shape does nothing
-    names = params or [n for n in cur if n != "cdef_chroma"]
+    names = [n for n in params or cur if n not in INERT]
     base = _time_batches(decoders, batches, reps)
     best_t = base
     for name in names:

@@ -452,12 +452,13 @@ int av1h_set_graphs(av1h_ctx* ctx, int mode);
 /* Launch shapes of the batches this context leads, the parameters an
  * autotuner searches (av1ongpu_amd/autotune.py does): for every kernel the
  * persistent workgroups per compute unit of its grid, the queue's, and the
- * sets of CDEF blocks a workgroup takes one after the other (1..4); CDEF's chroma
- * blocks run in the luma launch, so "cdef_chroma" has no effect.
- * av1h_tune_params gives
- * their count and av1h_tune_name their names; setting them drops the
- * captured launch sequences. No counterpart in the reference (fixed launch
- * shapes, av1_cuda.cu). */
+ * sets of CDEF blocks a workgroup takes one after the other (1..4). CDEF's
+ * chroma blocks run in the luma launch and the transforms of intra blocks in
+ * those of the inter blocks, so "cdef_chroma", "itx_intra" and
+ * "itx_intra_large" are kept and read back but have no effect.
+ * av1h_tune_params gives their count and av1h_tune_name their names; setting
+ * them drops the captured launch sequences. No counterpart in the reference
+ * (fixed launch shapes, av1_cuda.cu). */
 int av1h_tune_params(void);
 const char* av1h_tune_name(int index);
 int av1h_tune_get(const av1h_ctx* ctx, int32_t* params, int n);
