@@ -243,7 +243,7 @@ struct TrainLds {
   float w1[kH * 28], w2[kH * kLd];
   float h1[kBatch * kLd], h2[kBatch * kLd], d1[kBatch * kLd], d2[kBatch * kLd];
   float x[kBatch * 28], d3[kBatch], y[kBatch];
-  float b1[kH], b2[kH], w3[kH], b3, loss;
+  float b1[kH], b2[kH], w3[kH], b3;
 };
 
 /* An epoch: an Adam step per batch of kBatch samples in `perm` order (gradient
@@ -268,10 +268,7 @@ __global__ __launch_bounds__(kSteps) void k_mlp_train(float* params, float* am, 
     L.b2[tid] = params[kB2 + tid];
     L.w3[tid] = params[kW3 + tid];
   }
-  if (tid == 0) {
-    L.b3 = params[kB3];
-    L.loss = 0.f;
-  }
+  if (tid == 0) L.b3 = params[kB3];
   /* this thread's parameters: W2[4 wave + r][lane], W1[lane][wave], and by
    * wave W1[lane][wave + 16] (0-7), b1 (8), b2 (9), W3 (10), b3 (11, one lane) */
   int pi[6];
@@ -302,6 +299,7 @@ __global__ __launch_bounds__(kSteps) void k_mlp_train(float* params, float* am, 
   };
   fetch(0);
   int step = adam.t0;
+  float sq = 0.f; /* thread 16 s: the squared errors of the batches' sample s */
   for (int base = 0; base < n; base += kBatch) {
     const int nb = min(kBatch, n - base);
     L.x[s * 28 + q] = fx0;
@@ -353,7 +351,7 @@ __global__ __launch_bounds__(kSteps) void k_mlp_train(float* params, float* am, 
       }
       const float e = s < nb ? out - L.y[s] : 0.f;
       L.d3[s] = e * (2.f / (float)nb);
-      if (s < nb) atomicAdd(&L.loss, e * e);
+      sq += e * e;
     }
     __syncthreads();
     const float e3 = L.d3[s];
@@ -412,7 +410,14 @@ __global__ __launch_bounds__(kSteps) void k_mlp_train(float* params, float* am, 
     am[pi[k]] = m[k];
     av[pi[k]] = v[k];
   }
-  if (tid == 0) *loss = L.loss / (float)n;
+  /* the loss, its 64 sums in order too: equal runs report equal losses */
+  if (q == 0) L.d3[s] = sq;
+  __syncthreads();
+  if (tid == 0) {
+    float all = 0.f;
+    for (int b = 0; b < kBatch; ++b) all += L.d3[b];
+    *loss = all / (float)n;
+  }
 }
 
 /* The gradient and the loss from the workgroups' sums. */

@@ -65,3 +65,14 @@ def test_train_one_batch(n, epochs):
     # a learning rate off; all but a few weights agree to rounding
     d = np.abs(cm.params() - w)
     assert np.median(d) < 1e-6 and (d > 1e-5).mean() < 0.02 and d.max() <= 2.1e-3 * epochs
+
+
+def test_train_repeats():
+    """The same samples, weights and seed train to the same bits: every sum,
+    the loss's too, has one order."""
+    runs = []
+    for _ in range(3):
+        cm, _p, X, y, _mean, _dev = _model(5, 4000)
+        losses = cm.train(X, y, epochs=2, lr=1e-3, seed=3, set_norm=False)
+        runs.append((list(losses), cm.params().tobytes()))
+    assert runs[0] == runs[1] == runs[2]
