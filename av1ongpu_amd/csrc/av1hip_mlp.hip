@@ -704,11 +704,11 @@ static void standardise(const av1h_costmodel* m, const float* X, const float* y_
   }
 }
 
-/* The standardised samples on the device, with room for two epochs' orders,
+/* The standardised samples on the device, with room for an epoch's order,
  * `groups` workgroups' gradient sums and `losses` losses: one allocation. */
 struct Samples {
   float *x = nullptr, *y = nullptr, *part = nullptr, *grad = nullptr, *loss = nullptr;
-  int32_t* perm[2] = {nullptr, nullptr};
+  int32_t* perm = nullptr;
   void* buf = nullptr;
   ~Samples() {
     if (buf) (void)hipFree(buf);
@@ -716,13 +716,12 @@ struct Samples {
   int make(const std::vector<float>& xs, const std::vector<float>& ys, int groups, int losses) {
     const size_t n = ys.size(), pad = 64;
     auto up = [&](size_t v) { return (v + pad - 1) / pad * pad; };
-    const size_t total = up(n * kIn) + 3 * up(n) + up((size_t)groups * kParams) + up(kParams) + up((size_t)losses);
+    const size_t total = up(n * kIn) + 2 * up(n) + up((size_t)groups * kParams) + up(kParams) + up((size_t)losses);
     CM_OK(hipMalloc(&buf, total * sizeof(float)));
     x = static_cast<float*>(buf);
     y = x + up(n * kIn);
-    perm[0] = reinterpret_cast<int32_t*>(y + up(n));
-    perm[1] = perm[0] + up(n);
-    part = reinterpret_cast<float*>(perm[1] + up(n));
+    perm = reinterpret_cast<int32_t*>(y + up(n));
+    part = reinterpret_cast<float*>(perm + up(n));
     grad = part + up((size_t)groups * kParams);
     loss = grad + up(kParams);
     CM_OK(hipMemcpy(x, xs.data(), n * kIn * sizeof(float), hipMemcpyHostToDevice));
@@ -744,8 +743,8 @@ int av1h_cm_gradients(av1h_costmodel* m, const float* features, const float* y_u
   Samples d;
   const int rc = d.make(xs, ys, groups, groups + 1);
   if (rc != AV1H_OK) return rc;
-  CM_OK(hipMemcpy(d.perm[0], perm.data(), perm.size() * 4, hipMemcpyHostToDevice));
-  hipLaunchKernelGGL(k_mlp_grad, dim3(groups), dim3(kSteps), 0, m->stream, m->params, d.part, d.x, d.y, d.perm[0],
+  CM_OK(hipMemcpy(d.perm, perm.data(), perm.size() * 4, hipMemcpyHostToDevice));
+  hipLaunchKernelGGL(k_mlp_grad, dim3(groups), dim3(kSteps), 0, m->stream, m->params, d.part, d.x, d.y, d.perm,
                      (int)n, d.loss);
   CM_OK(hipGetLastError());
   hipLaunchKernelGGL(k_mlp_sum, dim3((kParams + kThreads - 1) / kThreads), dim3(kThreads), 0, m->stream, d.part, d.loss,
@@ -790,20 +789,20 @@ int av1h_cm_train(av1h_costmodel* m, const float* features, const float* y_us, i
   Samples d;
   int rc = d.make(xs, ys, 0, epochs);
   if (rc != AV1H_OK) return rc;
-  /* an epoch's order is shuffled while the one before it runs */
+  /* an epoch's order is shuffled while the one before it runs, and copied
+   * behind it on the stream */
   std::vector<int32_t> perm((size_t)n);
   std::mt19937_64 rng(seed);
   int done = 0; /* epochs whose launches were queued */
   for (; done < epochs; ++done) {
     for (int64_t i = 0; i < n; ++i) perm[(size_t)i] = (int32_t)i;
     std::shuffle(perm.begin(), perm.end(), rng);
-    int32_t* dp = d.perm[done & 1];
-    if (hipMemcpyAsync(dp, perm.data(), perm.size() * 4, hipMemcpyHostToDevice, m->stream) != hipSuccess ||
+    if (hipMemcpyAsync(d.perm, perm.data(), perm.size() * 4, hipMemcpyHostToDevice, m->stream) != hipSuccess ||
         hipStreamSynchronize(m->stream) != hipSuccess)
       break;
     const Adam a{lr, 0.9f, 0.999f, 1e-8f, m->steps};
     hipLaunchKernelGGL(k_mlp_train, dim3(1), dim3(kSteps), 0, m->stream, m->params, m->adam, m->adam + kParams, d.x,
-                       d.y, dp, (int)n, a, d.loss + done);
+                       d.y, d.perm, (int)n, a, d.loss + done);
     if (hipGetLastError() != hipSuccess) break;
     m->steps += (int)((n + kBatch - 1) / kBatch);
   }
