@@ -27,6 +27,7 @@
 
 #define AV1T_TABLE_QUAL static const
 #include "av1hip_internal.hpp"
+#include "graph_cache.hpp"
 #include "scan_order.hpp"
 #include "spec_tables.h"
 
@@ -241,7 +242,7 @@ struct Ctx {
   bool graphs = true;
   bool graph_sets = true; /* graphs keyed by the set of kernels with work too */
   Tuning tune;                   /* launch shapes of the batches it leads */
-  std::vector<std::pair<uint64_t, hipGraphExec_t>> graph_exec; /* (buffer set, size classes, kernel set, frames; graph) */
+  GraphCache<hipGraphExec_t> graph_exec; /* by buffer set, size classes, kernel set, frames */
   bool stage_hit[AV1H_STAGES] = {};
   double stage_ms[AV1H_STAGES] = {};
   int64_t stage_n[AV1H_STAGES] = {};
@@ -1953,8 +1954,7 @@ int prepare(Ctx* c, const Layout& L) {
 }
 
 void drop_graphs(Ctx* c) {
-  for (auto& g : c->graph_exec) (void)hipGraphExecDestroy(g.second);
-  c->graph_exec.clear();
+  c->graph_exec.clear([](hipGraphExec_t e) { (void)hipGraphExecDestroy(e); });
 }
 
 int alloc_slot(Ctx* c) {
@@ -2400,12 +2400,10 @@ int batch_launch(Ctx* lead, std::vector<JobSpec>& js, double t0) {
   };
   for (bool& h : lead->stage_hit) h = false;
   if (use_graph) {
-    hipGraphExec_t exec = nullptr;
     static_assert(8 + kKernels + 1 <= 48, "graph key");
     const uint64_t key = (uint64_t)b << 62 | (uint64_t)queue_class << 50 | (uint64_t)grid_class << 48 | live << 8 |
                          (uint64_t)n; /* n <= 128 */
-    for (auto& g : lead->graph_exec)
-      if (g.first == key) exec = g.second;
+    hipGraphExec_t exec = lead->graph_exec.find(key);
     if (!exec) {
       HIP_OK(lead, hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
       const hipError_t e = sequence();
@@ -2420,11 +2418,7 @@ int batch_launch(Ctx* lead, std::vector<JobSpec>& js, double t0) {
       (void)hipGraphDestroy(graph);
       if (e3 != hipSuccess)
         return set_err(lead, AV1H_ERR_DEVICE, "instantiating the batch graph: %s", hipGetErrorString(e3));
-      if (lead->graph_exec.size() >= 64) {
-        (void)hipGraphExecDestroy(lead->graph_exec.front().second);
-        lead->graph_exec.erase(lead->graph_exec.begin());
-      }
-      lead->graph_exec.emplace_back(key, exec);
+      lead->graph_exec.insert(key, exec, [](hipGraphExec_t e) { (void)hipGraphExecDestroy(e); });
     }
     HIP_OK(lead, hipEventRecord(lead->bev[b][0], s));
     HIP_OK(lead, hipGraphLaunch(exec, s));

@@ -235,3 +235,21 @@ def test_async_batch_holds_its_contexts():
     for p in range(3):
         assert np.array_equal(planes[p], want[p])
     dec.discard_plan(plan)
+
+
+def test_graph_size_classes_match_eager():
+    """One decoder whose frames cross the sizes at which a captured sequence
+    takes other grids (256 and 1024 workgroups, 256 queue entries), up and
+    down and again from the captured graphs."""
+    eager, dec = pkg.HipDecoder(), pkg.HipDecoder()
+    eager.set_graphs(False)
+    clips = [pkg.Clip("c1_mini", 87, width=w, height=h, frames=2, intra_frac=0.3)
+             for w, h in ((854, 480), (64, 64), (426, 240), (160, 96))]
+    plans = [eager.plan_wire(c.wire(0)) for c in clips]
+    queued = [eager.queue_counts(p)["blocks"] for p in plans]
+    assert min(queued) < 256 < max(queued)
+    for p in plans:
+        eager.discard_plan(p)
+    for c in clips + clips[::-1] + clips:
+        for (f, _, want), (_, _, got) in zip(pkg.decode_clip(eager, c), pkg.decode_clip(dec, c)):
+            _check(f"c1_mini of {len(c.wire(0))} bytes", f, got, want)
