@@ -1953,7 +1953,9 @@ int prepare(Ctx* c, const Layout& L) {
   return AV1H_OK;
 }
 
+/* (a batch in flight may be replaying one: it ends first) */
 void drop_graphs(Ctx* c) {
+  if (!c->pending.empty()) (void)hipStreamSynchronize(c->stream);
   c->graph_exec.clear([](hipGraphExec_t e) { (void)hipGraphExecDestroy(e); });
 }
 

@@ -217,6 +217,25 @@ def test_async_batches_match_alone(own_launcher):
             assert a == b, f"{c.workload} seed {c.seed} frame {f}: asynchronous batch differs from the plain decode"
 
 
+def test_launch_shapes_change_under_a_batch():
+    """New launch shapes drop the captured graphs, the running batch's too."""
+    clip = pkg.Clip("c2_mini", 12)
+    keep, rel, refs = pkg.slot_schedule(clip)
+    dec = pkg.HipDecoder()
+    dec.set_output_hash(True)
+    plans = [dec.plan_wire(pkg.wire_set_slots(clip.wire(f), refs[f])) for f in range(clip.frames)]
+    got = []
+    for f, plan in enumerate(plans):
+        pkg.decode_planned_batch_async([dec], [plan], [keep[f] >= 0], [keep[f]])
+        dec.set_tuning({"mc": 4 + f})
+        pkg.batch_finish(dec)
+        got.append(dec.last_hash())
+        for s in rel[f]:
+            dec.release(s)
+        dec.discard_plan(plan)
+    assert got == [pkg.picture_hash(p) for p in _alone(clip)]
+
+
 def test_async_batch_holds_its_contexts():
     """While a launched batch holds a context's frame, its pictures cannot be
     read and another launcher cannot batch it; after the finish they can."""
