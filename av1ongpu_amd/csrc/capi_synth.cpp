@@ -43,6 +43,7 @@ int av1s_config_set(void* h, const char* key, double v) {
   else if (k == "key_interval") c->key_interval = i;
   else if (k == "max_tx") c->max_tx = i;
   else if (k == "rect_tx") c->rect_tx = i != 0;
+  else if (k == "rect4") c->rect4 = i != 0;
   else if (k == "tx_ext") c->tx_ext = i != 0;
   else if (k == "mv_gaussian") c->mv_gaussian = i != 0;
   else if (k == "mv_range") c->mv_range = i;

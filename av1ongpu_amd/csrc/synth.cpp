@@ -346,6 +346,18 @@ class FrameBuilder {
   /* tiling of a w x h region with transforms of tw x th, raster order */
   void tx_size_for(int plane, int w, int h, bool intra, int* tw, int* th) {
     const int cap = std::min(cfg_.max_tx, plane ? 32 : 64);
+    if (cfg_.rect4 && rng_.chance(0.5)) {
+      const bool wide = rng_.chance(0.5);
+      const int along = std::min(wide ? w : h, cap), across = wide ? h : w;
+      int sizes[3], n = 0;
+      for (int s = 16; s <= along && s / 4 <= across; s *= 2) sizes[n++] = s;
+      if (n > 0) {
+        const int s = sizes[rng_.range(0, n - 1)];
+        *tw = wide ? s : s / 4;
+        *th = wide ? s / 4 : s;
+        return;
+      }
+    }
     if (plane) {
       /* the chroma transform is the largest that fits (capped at 32) */
       if (cfg_.rect_tx && (w == 2 * h || h == 2 * w) && w <= cap && h <= cap) {

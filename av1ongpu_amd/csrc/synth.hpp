@@ -40,6 +40,7 @@ struct Config {
   int key_interval = 0;      /* 0: only the first frame is a key frame            */
   int max_tx = 32;           /* largest transform side (32 or 64)                 */
   bool rect_tx = false;      /* 2:1 transforms on 2:1 blocks                      */
+  bool rect4 = false;        /* 4:1 transforms too, so 4:1 intra blocks           */
   bool tx_ext = false;       /* identity, flip-ADST and the 1D transform types    */
   bool mv_gaussian = false;  /* vectors ~ N(0, mv_sigma) instead of U[-r, r]      */
   int mv_range = 128;        /* 1/8 luma samples                                  */

@@ -88,3 +88,22 @@ def test_a_wait_that_gives_up_fails_the_decode_and_the_next_is_clean():
     want = [pkg.picture_hash(planes) for _, _, planes in pkg.decode_clip(OracleDecoder(), clip)]
     assert got == want
     dec.close()
+
+
+def test_ticket_counters():
+    """Queues on both sides of the length that is dealt to eight counters
+    (128 entries), of every remainder modulo eight, and a long one taken by
+    as few and as many waves as the launch shapes allow."""
+    from oracle_lib import OracleDecoder
+    dec, lengths = pkg.HipDecoder(), set()
+    small = [pkg.Clip("c2_mini", seed, frames=1, width=w, height=40, coded_width=0, max_tx=8, cdef=0, lr=0, grain=0)
+             for w in (48, 56, 64, 72) for seed in range(20, 32)]
+    for clip, per_cu in [(c, 6) for c in small] + [(pkg.Clip("c1_mini", 27, frames=1, width=426, height=240), q) for q in (1, 64)]:
+        dec.set_tuning({"queue": per_cu})
+        plan = dec.plan_wire(clip.wire(0))
+        lengths.add(dec.queue_counts(plan)["blocks"])
+        dec.discard_plan(plan)
+        for (_, _, got), (_, _, want) in zip(pkg.decode_clip(dec, clip), pkg.decode_clip(OracleDecoder(), clip)):
+            assert pkg.picture_hash(got) == pkg.picture_hash(want), (clip.seed, per_cu)
+    dec.close()
+    assert min(lengths) < 128 < max(lengths) and len({n % 8 for n in lengths if n >= 128}) == 8, sorted(lengths)

@@ -39,3 +39,16 @@ def test_small_blocks(workload, over, seed):
     for (f, _, ph), (_, _, po) in zip(pkg.decode_clip(pkg.HipDecoder(), clip), ora):
         for p in range(3):
             assert np.array_equal(ph[p], po[p]), (f, p, np.argwhere(ph[p] != po[p])[:3].tolist())
+
+
+@pytest.mark.parametrize("workload,over", [
+    ("c2_mini", dict(frames=2, width=328, height=200, coded_width=0)),
+    ("c2_mini", dict(frames=2, width=200, height=136, coded_width=0, bit_depth=12, intra_frac=0.5, ss_x=0, ss_y=0)),
+    ("c1_mini", dict(frames=2, width=173, height=99, intra_frac=0.4, tx_skip=0.6)),
+    ("tools_mini", dict(frames=3, intra_frac=0.4, levels=1)),
+    ("contract_mini", dict(frames=2, intra_frac=0.5, ss_y=0)),
+])
+@pytest.mark.parametrize("seed", [13, 14, 15])
+def test_four_to_one_blocks(workload, over, seed):
+    """Intra blocks and transforms of 4x16, 16x4, 8x32, 32x8, 16x64 and 64x16."""
+    test_small_blocks(workload, dict(over, rect4=1), seed)
