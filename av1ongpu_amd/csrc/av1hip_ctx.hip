@@ -1535,11 +1535,14 @@ int flatten(const av1h_frame_desc& f, Plan* plan, Host* H, std::string* err) {
   for (int64_t& v : plan->alg_bytes) v = 0;
   {
     /* part 0: inter samples written once and read from each reference, the
-     * coefficients of every transform (int16 each); the queue: per queued
-     * sample its residual read and the picture sample written */
-    plan->alg_bytes[AV1H_STAGE_INTER] = inter_bytes;
-    for (const DevTx& t : H->tx)
-      if (!(t.flags & kTxToResidual)) plan->alg_bytes[AV1H_STAGE_INTER] += 2 * (int64_t)t.w * t.h;
+     * coefficients of every transform (int16 each), the residuals the queue
+     * reads; the queue: per queued sample its residual read and the picture
+     * sample written */
+    int64_t& inter = plan->alg_bytes[AV1H_STAGE_INTER];
+    inter = inter_bytes;
+    for (const int32_t bi : H->special_list)
+      inter += (int64_t)H->blocks[bi].w * H->blocks[bi].h * (H->blocks[bi].compound ? 6 : 4);
+    for (const DevTx& t : H->tx) inter += (int64_t)t.w * t.h * ((t.flags & kTxToResidual) ? 4 : 2);
     for (const int32_t a : plan->q_area) plan->alg_bytes[AV1H_STAGE_QUEUE] += 4 * (int64_t)a;
     bool has_edges[3] = {false, false, false};
     for (const DevDeblock& d : H->deblock) {

@@ -511,8 +511,10 @@ void av1h_set_stage_timing(av1h_ctx* ctx, int enable);
  * since timing was enabled (a stage a frame skips is not counted for it).
  * Compulsory bytes, at 16 bit samples: motion compensation and transforms 2 B
  * written per inter sample, 2 B per reference read, 2 B of coefficients per
- * transform sample; intra prediction 2 B written per sample; deblocking, CDEF, grain and the reference store 4 B (one read, one
- * write) per sample they cover; restoration 4 B per sample plus the two
+ * transform sample and 2 B of residual written where the queue adds it; intra
+ * prediction 4 B per queued sample (its residual read, itself written);
+ * deblocking, CDEF, grain and the reference store 4 B (one read, one write)
+ * per sample they cover; restoration 4 B per sample plus the two
  * boundary rows above and below each stripe; upscaling 2 B per coded and 2 B
  * per upscaled sample, for each picture it upscales. Any argument may be
  * null. */
