@@ -1411,7 +1411,7 @@ __device__ __forceinline__ void queue_small(RArgs a, BlkRef b, const QBlk& q, bo
                                             uint32_t* error, uint64_t* ready, bool trace) {
   LayRef L = a.lay;
   const int lane = threadIdx.x;
-  const int w = q.w, h = q.h, n = w + h, lw = ilog2(w), lh = ilog2(h);
+  const int w = q.w, h = q.h, n = w + h, lw = ilog2(w);
   const int x = lane & (w - 1), y = lane >> lw; /* this lane's sample */
   const bool sample = lane < w * h;
   int res = 0;
@@ -2398,7 +2398,12 @@ __global__ __launch_bounds__(64) void k_queue(BatchDev B) {
    * XCD's workgroups start in order of their number, the first kTickets of
    * them on any XCD cover every counter, and a counter's waves take its
    * entries in order, so the smallest unfinished entry is held by a wave or
-   * next on a counter with a wave that holds none. Queue of a 1080p inter
+   * next on a counter with a wave that holds none. That takes kTickets resident
+   * workgroups on one XCD (with one counter, one in all): a compute unit holds
+   * eight of this kernel (227 registers, 28 bytes of scratch a lane: two waves a
+   * SIMD; 18 KB of LDS), an XCD 256, so of up to 32 such launches at a time (a
+   * process has four hardware queues) one has them even where waiting waves
+   * fill the card, and when it ends its places go to the next. Queue of a 1080p inter
    * frame (2518 entries) 67 -> 42 us, of a batch of eight (12,400) 169 -> 61. */
   const int deal = takers >= 16 * kTickets ? kTickets : 1;
   const int own = ((int)blockIdx.x >> 3) & (deal - 1);
