@@ -243,13 +243,14 @@ struct TrainLds {
   float w1[kH * 28], w2[kH * kLd];
   float h1[kBatch * kLd], h2[kBatch * kLd], d1[kBatch * kLd], d2[kBatch * kLd];
   float x[kBatch * 28], d3[kBatch], y[kBatch];
+  float e[kBatch], sq[kBatch]; /* a batch's errors; their squares summed over the batches */
   float b1[kH], b2[kH], w3[kH], b3;
 };
 
 /* An epoch: an Adam step per batch of kBatch samples in `perm` order (gradient
  * of the batch mean), one workgroup, as the steps are a chain. Adam divides by
  * the gradients' own size, so one rounded otherwise where it is close to zero
- * moves its weight by up to the learning rate: every sum here is one chain of
+ * moves its weight by up to the learning rate: every sum of a step is one chain of
  * FMAs in the order of its index, and the matrix cores, whose sums are grouped
  * by four, are left to the gradient and the predictions. Sixteen threads per
  * sample, four neurons each; a thread's parameters (four of one column of W2
@@ -268,6 +269,7 @@ __global__ __launch_bounds__(kSteps) void k_mlp_train(float* params, float* am, 
     L.b2[tid] = params[kB2 + tid];
     L.w3[tid] = params[kW3 + tid];
   }
+  if (tid < kBatch) L.sq[tid] = 0.f;
   if (tid == 0) L.b3 = params[kB3];
   /* this thread's parameters: W2[4 wave + r][lane], W1[lane][wave], and by
    * wave W1[lane][wave + 16] (0-7), b1 (8), b2 (9), W3 (10), b3 (11, one lane) */
@@ -299,7 +301,6 @@ __global__ __launch_bounds__(kSteps) void k_mlp_train(float* params, float* am, 
   };
   fetch(0);
   int step = adam.t0;
-  float sq = 0.f; /* thread 16 s: the squared errors of the batches' sample s */
   for (int base = 0; base < n; base += kBatch) {
     const int nb = min(kBatch, n - base);
     L.x[s * 28 + q] = fx0;
@@ -351,7 +352,7 @@ __global__ __launch_bounds__(kSteps) void k_mlp_train(float* params, float* am, 
       }
       const float e = s < nb ? out - L.y[s] : 0.f;
       L.d3[s] = e * (2.f / (float)nb);
-      sq += e * e;
+      L.e[s] = e;
     }
     __syncthreads();
     const float e3 = L.d3[s];
@@ -390,6 +391,7 @@ __global__ __launch_bounds__(kSteps) void k_mlp_train(float* params, float* am, 
       if (wave == 10) g[5] += L.d3[b] * L.h2[b * kLd + lane];
       if (wave == 11) g[5] += L.d3[b];
     }
+    if (wave == 12) L.sq[lane] += L.e[lane] * L.e[lane]; /* beside the other waves' last loop */
     ++step;
     const float c1 = 1.f - powf(adam.b1, (float)step), c2 = 1.f - powf(adam.b2, (float)step);
 #pragma unroll
@@ -411,12 +413,10 @@ __global__ __launch_bounds__(kSteps) void k_mlp_train(float* params, float* am, 
     av[pi[k]] = v[k];
   }
   /* the loss, its 64 sums in order too: equal runs report equal losses */
-  if (q == 0) L.d3[s] = sq;
-  __syncthreads();
   if (tid == 0) {
-    float all = 0.f;
-    for (int b = 0; b < kBatch; ++b) all += L.d3[b];
-    *loss = all / (float)n;
+    f4 all = {};
+    for (int b = 0; b < kBatch; b += 4) all += ld4(L.sq + b);
+    *loss = (all[0] + all[1] + all[2] + all[3]) / (float)n;
   }
 }
 
