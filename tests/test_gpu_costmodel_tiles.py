@@ -76,3 +76,17 @@ def test_train_repeats():
         losses = cm.train(X, y, epochs=2, lr=1e-3, seed=3, set_norm=False)
         runs.append((list(losses), cm.params().tobytes()))
     assert runs[0] == runs[1] == runs[2]
+
+
+def test_predict_again_and_from_threads():
+    """Calls of one model share its staging: one after the other and from
+    several threads, each gets its own samples' predictions."""
+    from concurrent.futures import ThreadPoolExecutor
+    cm, p, X, _y, mean, dev = _model(9, 4096)
+    parts = [X[i * 300:i * 300 + n] for i, n in enumerate((300, 17, 1000, 64, 300, 2040))]
+    want = [predict_us(p, x, mean, dev, 20.0, 11.0) for x in parts]
+    for x, w in zip(parts + parts[::-1], want + want[::-1]):
+        assert _off(cm.predict(x), w) < 1e-5
+    with ThreadPoolExecutor(4) as pool:
+        for got, w in zip(pool.map(cm.predict, parts * 20), want * 20):
+            assert _off(got, w) < 1e-5
