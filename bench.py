@@ -21,7 +21,7 @@ reported as p50/p99.
 Also reported: `device_only`, the same clip from plans already resident in
 HBM (one decode call per frame, its call latency p50/p99); `ingest_serial`,
 each frame flattened, uploaded and decoded before the next on one thread; the
-dominant kernel's roofline from HIP events around each stage, on the decode
+dominant stage's roofline from HIP events around each stage, on the decode
 stream, in one more pass over the clip after the timed steps (the timed steps
 replay captured launch sequences; the event pass launches eagerly); the CPU
 oracle on a bounded sample of the same clip, timed on this host, and the
@@ -43,9 +43,11 @@ sys.path.insert(0, REPO)
 METRIC = "decoded Mpixel/s on 1 MI355X, batched vs plain, bit-exact; p99 frame latency"
 HBM_PEAK_GBS = 8000.0
 NV12_PITCH = 2048
-# the kernel that dominates each timed stage (the stage's events bracket it)
-STAGE_KERNEL = {"inter": "k_mc", "queue": "k_queue", "deblock": "k_deblock", "cdef": "k_cdef",
-                "superres": "k_upscale", "lr": "k_lr", "store": "k_copy", "grain": "k_grain_apply"}
+# the kernels each timed stage's events bracket and their launches per frame
+# of the headline's clips (whose blocks use none of k_inter_special's tools)
+STAGE_KERNELS = {"inter": {"k_mc": 1, "k_itx<3, 5>": 1, "k_itx<0, 3>": 1}, "queue": {"k_queue": 1},
+                 "deblock": {"k_deblock": 2}, "cdef": {"k_cdef_dir": 1, "k_cdef": 1}, "superres": {"k_upscale": 1},
+                 "lr": {"k_lr": 1}, "store": {"k_copy": 1}, "grain": {"k_grain_apply": 1}}
 WORKLOADS = {
     "c2": "1920x1080 10-bit 4:2:0, 60 frames, hierarchical GOP 16 with 3 references, compound "
           "(distance weighted + average), transforms 4x4-64x64 incl. identity and flip-ADST, "
@@ -115,11 +117,11 @@ def pct(values, q):
     return v[k]
 
 
-def load_traffic(workload, kernel):
-    """HBM bytes per launch of a kernel from the committed rocprofv3 counter
-    summary (FETCH_SIZE and WRITE_SIZE, scaled by a copy kernel of known size),
-    or None when the summary does not cover the kernel on this workload (said
-    on stderr)."""
+def load_traffic(workload, kernels):
+    """HBM bytes a stage's kernels ({name: launches}) move per frame, from the
+    committed rocprofv3 counter summary (FETCH_SIZE and WRITE_SIZE, scaled by a
+    copy kernel of known size), or None when the summary does not cover a kernel
+    on this workload (said on stderr)."""
     path = os.path.join(REPO, "profiles", "hbm_traffic.json")
     try:
         with open(path) as fh:
@@ -130,11 +132,14 @@ def load_traffic(workload, kernel):
     if t.get("workload") != workload:
         log(f"WARNING: the HBM traffic summary is of workload {t.get('workload')}, not {workload}")
         return None
-    k = t.get("kernels", {}).get(kernel)
-    if k is None:
-        log(f"WARNING: the HBM traffic summary has no kernel {kernel}: roofline traffic left null")
-        return None
-    return int(k["bytes_per_launch"])
+    total = 0
+    for kernel, launches in kernels.items():
+        k = t.get("kernels", {}).get(kernel)
+        if k is None:
+            log(f"WARNING: the HBM traffic summary has no kernel {kernel}: roofline traffic left null")
+            return None
+        total += launches * int(k["bytes_per_launch"])
+    return total
 
 
 def cpu_baseline(clip, seconds, gpu_hashes):
@@ -829,13 +834,13 @@ def main():
 
     value = args.steps * n * px / elapsed / 1e6
     ms_step = elapsed * 1e3 / max(args.steps, 1)
-    # dominant kernel: the stage with the most device time
+    # the stage with the most device time, its kernels together
     dom = max((s for s in stages if stages[s][1] > 0), key=lambda s: stages[s][0])
     ms, cnt, byts = stages[dom]
     avg_ms = ms / cnt
     achieved = byts / cnt / (avg_ms * 1e-3) / 1e9
-    traffic = load_traffic(args.workload, STAGE_KERNEL[dom])
-    roofline = {"bound": "hbm", "kernel": STAGE_KERNEL[dom], "achieved": round(achieved, 1),
+    traffic = load_traffic(args.workload, STAGE_KERNELS[dom])
+    roofline = {"bound": "hbm", "kernel": " + ".join(STAGE_KERNELS[dom]), "achieved": round(achieved, 1),
                 "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
                 "traffic": traffic, "algorithmic_bytes_per_launch": byts // cnt,
                 "avg_launch_ms": round(avg_ms, 4)}

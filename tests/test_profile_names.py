@@ -24,7 +24,12 @@ def test_named_kernels_exist():
         traffic = json.load(fh)
     kernels = _kernels()
     assert {"k_queue", "k_itx", "k_cdef"} <= set(kernels) and kernels["k_itx"]
-    for name in [*bench.STAGE_KERNEL.values(), *traffic["kernels"]]:
+    named = [k for stage in bench.STAGE_KERNELS.values() for k in stage]
+    for name in [*named, *traffic["kernels"]]:
         base = name.split("<")[0]
         assert kernels.get(base) is ("<" in name), name
-    assert traffic["workload"] in bench.WORKLOADS and set(bench.STAGE_KERNEL.values()) <= set(traffic["kernels"])
+    assert traffic["workload"] in bench.WORKLOADS and set(named) <= set(traffic["kernels"])
+    per = {k: v["bytes_per_launch"] for k, v in traffic["kernels"].items()}
+    assert bench.load_traffic("c2", bench.STAGE_KERNELS["deblock"]) == 2 * per["k_deblock"]
+    assert bench.load_traffic("c2", bench.STAGE_KERNELS["cdef"]) == per["k_cdef"] + per["k_cdef_dir"]
+    assert bench.load_traffic("c2", {"k_cdef<1>": 1}) is None and bench.load_traffic("c1", {"k_queue": 1}) is None
