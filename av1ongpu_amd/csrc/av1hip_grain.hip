@@ -117,7 +117,8 @@ __device__ __forceinline__ void store4(uint16_t* dst, const int* v, int n) {
  * samples per lane and step: the loads, the template rows and the stores of a
  * step are one wide access each, and a noise block's offsets are looked up
  * once for the four. One sample per lane and step took 16.6 us on a 1080p
- * frame and 67 on a 2160p one; now 12 and 35. */
+ * frame and 67 on a 2160p one; now 12 and 35 (over the 60 frames of the 1080p
+ * clip 18.9 -> 13.5). */
 __device__ void grain_tile(FArgs a, int t, int2* s_lut) {
   LayRef L = a.lay;
   const DevGrain& g = *a.plan.grain;

@@ -2106,8 +2106,8 @@ __device__ void reconstruct_queued(RArgs a, BlkRef b, const QBlk& q, int* work, 
  * row's eleven samples come in two loads and a scaled sample's eight in one,
  * and taps are multiplied two at a time (v_dot2_i32_i16: samples and taps are
  * 16 bit, sums below 2^31); 64 registers keep 8 workgroups on a compute unit.
- * A launch against one thread per sample: 720p frame 22.5 -> 12.3 us, 1080p
- * (scaled, compound) 45 -> 30, 2160p 169 -> 104, eight streams 122 -> 58. */
+ * A launch against one thread per sample: 720p frame 22.5 -> 12 us, 1080p
+ * (scaled, compound) 45 -> 32, 2160p 169 -> 106, eight streams 122 -> 56. */
 constexpr int kMcPairs = 2 * kMcItems;
 constexpr int kMcChunkS = 16, kMcChunkM = 64; /* lookup: samples, intermediates */
 
