@@ -1,8 +1,8 @@
 """Inverse transforms against the oracle, bit exact, on both sides of the
 rule that picks the 24-bit form: coefficients far below its bound, around it
 (waves whose lanes disagree) and far above it (clamps act), every size and
-type, each bit depth (the clamps' widths), 16- and 32-bit coefficients, coded
-levels and lossless blocks."""
+type, each bit depth (the clamps' widths), 16-bit coefficients (wider ones are in
+test_gpu_odd_syntax.py), coded levels and lossless blocks."""
 import numpy as np
 import pytest
 
