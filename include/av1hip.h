@@ -440,10 +440,11 @@ int av1h_set_decode_nv12(av1h_ctx* ctx, size_t pitch);
  * its launch sequence into a HIP graph, each of those kernels at a persistent
  * grid for its class (small batches take smaller grids) reading its work
  * counts from the batch's device tables; later batches of that shape replay
- * it with one launch. A capture takes milliseconds: a caller whose batches
- * cross 256 or 1024 workgroups in their largest kernel, or 256 queued blocks,
- * pays one for each of up to six size classes (and each of the two batches in
- * flight); a context keeps the 384 graphs used last. Mode 2: one graph per
+ * it with one launch. A capture takes 0.1 ms and a graph 0.6 MB of device
+ * memory: a caller whose batches cross 256 or 1024 workgroups in their largest
+ * kernel, or 256 queued blocks, pays them for each of up to six size classes
+ * (and each of the two batches in flight); a context keeps the 384 graphs used
+ * last. Mode 2: one graph per
  * frame count with every kernel launched (kernels without work exit at
  * once), for callers whose batches change shape often (the serving loop's
  * launchers): fewer captures, each replay dispatching every kernel. Mode 0:
